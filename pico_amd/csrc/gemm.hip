@@ -5,10 +5,13 @@
 // src/autograd.h:96-130), plus a two-level batch and the causal tile/k-range
 // restrictions attention uses.
 //
-// Design (one 256-thread workgroup = 4 waves per C tile):
-//  * Five tile shapes built from v_mfma_f32_32x32x2f32 blocks (4096 FLOP per
-//    instruction, 16 fp32 accumulators per lane per block), chosen per call by
-//    how evenly they spread over the 256 CUs:
+// fp32 products run on the bf16 matrix cores with operands split in three
+// parts (gemm_split.h); this file holds the choice of tile and K split, the
+// small-product kernels, and the opt-in bf16, split-bf16 and fp8 kernels.
+//
+// Design of those (one 256-thread workgroup = 4 waves per C tile):
+//  * Five tile shapes of 32x32 matrix blocks (16 fp32 accumulators per lane per
+//    block), chosen per call by how evenly they spread over the 256 CUs:
 //      256x256  2x2 waves of 128x128 (4x4 blocks, 256 accumulators held in
 //               AGPRs), one workgroup per CU -- large products;
 //      256x96   4x1 waves of 64x96, one per CU -- N a multiple of 96 (an
@@ -19,48 +22,31 @@
 //  * Tiles on the edge of C are handled in the same kernel: with M, N, K and
 //    the strides multiples of 4 each 128-bit load is predicated as a whole;
 //    otherwise loads fall back to 32-bit elements.
-//  * K advances 32 at a time through a double-buffered LDS ring.  A 32-wide
-//    slice is consumed as four k-groups of 4; the fragments of group q+1 are
-//    read from LDS while the MFMAs of group q run (two register sets).  The
-//    next slice is staged into the other LDS buffer, and the slice after it
-//    fetched into registers with 128-bit global loads, spread over groups 0-2.
-//    Unsplit products of the tiles up to 128x128 and of 256x96, which have at
-//    most two workgroups per CU to hide a load, hold two slices in registers
-//    and fetch three ahead.  Every memory instruction is interleaved with the MFMAs through
-//    sched_group_barrier, so the wave never issues a long run of loads or
-//    stores while the matrix pipe drains (measured: a block of 16 back-to-back
-//    stores + 16 loads per slice cost 13 % of the MFMA rate).  One barrier per
-//    slice sits before group 3, so group 0 of the next slice is read under
-//    group 3's MFMAs.
-//  * LDS holds every operand k-contiguous, [rows][32 + 4 pad]: an operand that
-//    is row-contiguous in memory is fetched one row and four consecutive k per
-//    thread (four 32-bit loads, each a contiguous run of 64 rows per wave), so
-//    its values arrive k-contiguous in registers and go to LDS as one 128-bit
-//    store, with no transposing moves (VALU work, which on gfx950 does not
-//    overlap the matrix products).  Within a 32-wide k slice, lanes 0-31 take
-//    k 0..15 and lanes 32-63 take k 16..31, so every fragment read is a 128-bit
-//    LDS load, for all four layouts (measured: paired 32-bit reads of a
-//    row-contiguous tile held NN and TN 5 % below NT).
+//  * K advances 32 at a time through a double-buffered LDS ring, the next slice
+//    staged into the other buffer and the slice after it fetched into registers
+//    under the current slice's matrix instructions, interleaved with them
+//    through sched_group_barrier.
+//  * LDS holds every operand k-contiguous: an operand that is row-contiguous in
+//    memory is fetched one row and four consecutive k per thread (four 32-bit
+//    loads, each a contiguous run of 64 rows per wave), so its values arrive
+//    k-contiguous in registers with no transposing moves.
 //  * Tile order is XCD-aware: the hardware deals consecutive workgroups to
 //    the 8 XCDs round-robin, so the launch index is remapped to give each XCD
 //    a contiguous run of tiles, walked in groups of 8 tile-rows so concurrently
 //    running tiles share A rows and B columns in that XCD's L2.
-//  * Each output element accumulates k in the same order (k, then k+16 within
-//    each pair of a slice) for every tile shape, so the shape choice never
-//    changes a result bit.
 #include <stdarg.h>
 #include <stdio.h>
 
 #include <mutex>
 #include <type_traits>
 
-#include "pk_common.h"
+#include "gemm_common.h"
 
 namespace {
 
-constexpr int BK = 32, NT = 256;
+using namespace pkg;
+
 constexpr int KF = BK + 4;  // row stride of a k-contiguous LDS tile [rows][36]
-constexpr int GROUP_M = 8;
 constexpr int64_t kCUs = 256;  // MI355X
 
 // One operand's R x BK slice, staged into a k-contiguous LDS tile [R][KF].
@@ -87,6 +73,7 @@ template <int BM_, int BN_, int WGM_, int TM_, int TN_, int OCC_>
 struct Tile {
     static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = 4 / WGM_, TM = TM_, TN = TN_;
     static constexpr int OCC = OCC_;  // resident workgroups per CU
+    static constexpr int THREADS = NT, G = 1;
     static_assert(WGM * TM * 32 == BM && WGN * TN * 32 == BN, "tile does not tile");
 };
 using Tile256 = Tile<256, 256, 2, 4, 4, 1>;
@@ -94,48 +81,6 @@ using Tile128 = Tile<128, 128, 2, 2, 2, 2>;
 using Tile96 = Tile<128, 96, 4, 1, 3, 2>;
 using Tile64 = Tile<64, 64, 2, 1, 1, 4>;
 using Tile256x96 = Tile<256, 96, 4, 2, 3, 1>;
-
-struct GemmParams {
-    const float* A;
-    const float* B;
-    float* C;
-    int64_t M, N, K, lda, ldb, ldc;
-    int64_t sAo, sAi, sBo, sBi, sCo, sCi, inner;
-    float alpha, beta;
-    int causal;
-    int tiles_m, tiles_n;
-    int splits;      // > 1: blockIdx.y is a K slice of kchunk, partials go to ws
-    int64_t kchunk;
-    float* ws;
-    // the beta term's source: C itself, or another matrix (batch 1 only)
-    const float* Cin;
-    int64_t ldcin;
-    // SwiGLU-backward epilogue (sg_a non-null, batch 1, no K split): the
-    // product is the upstream gradient dh of h = silu(a) * u and is not
-    // stored; the tile writes da (+)= dh*u*s*(1 + a*(1-s)) and du (+)= dh*a*s
-    // (s = sigmoid(a)), accumulating per sg_flags bit 0 (da) and bit 1 (du)
-    const float *sg_a, *sg_u;
-    float *sg_da, *sg_du;
-    int64_t sg_lda, sg_ldu, sg_ldd;
-    int sg_flags;
-    // the staged epilogue may use float4 accesses: every matrix it touches is
-    // 16-byte aligned with a row stride that is a multiple of 4
-    int epi_vec;
-    // fp8 products: the device address of the two operand scales (NULL: 1, 1)
-    const float* fp8_scale;
-    // SwiGLU-forward epilogue (pair_F > 0, 'N','N', batch 1, no K split): C is
-    // [gate | up], N = 2 pair_F columns.  A tile takes BN/2 gate columns and
-    // the BN/2 up columns pair_F to their right, so it holds matching pairs;
-    // it writes both to C and h = silu(gate) * up to sf_h
-    int64_t pair_F;
-    float* sf_h;
-    int64_t sf_ldh;
-};
-
-// Bounds handling of a tile's loads and stores: none (whole tiles), per float4
-// (M, N, K, the leading dimensions and batch strides multiples of 4, 16-byte
-// aligned operands: a float4 is wholly inside or wholly outside), or per element.
-constexpr int kEdgeNone = 0, kEdgeVec = 1, kEdgeScalar = 2;
 
 // The float4 at logical (row r, k) of an operand: 4 consecutive k when
 // KFAST (element (r,k) at base[r*ld + k]), else 4 consecutive rows (element
@@ -300,10 +245,6 @@ __device__ __forceinline__ int fp8_pack2(float a, float b, int old) {
     return __builtin_amdgcn_cvt_pk_fp8_f32(fp8_clamp(a), fp8_clamp(b), old, HI);
 }
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
 // An element of a split-bf16 tile: x is stored as hi = bf16(x) and
 // lo = bf16(x - hi), in two tiles LO elements apart (x - hi is exact in fp32,
 // so hi + lo is x to 2^-17 relative).
@@ -361,35 +302,6 @@ __device__ __forceinline__ void store_item(E* lds, int item, const f32x4* v) {
     int rr, kk;
     item_origin<KFAST, R>(item, rr, kk);
     put4(lds, rr * LS + kk, v[0]);
-}
-
-// k-group q (k = 4q..4q+3 for lanes 0-31, 16+4q.. for lanes 32-63) of the
-// fragments of NB blocks starting at LDS row r0 (one row per lane)
-template <int NB>
-__device__ __forceinline__ void read_group(const float* lds, int r0, int lr, int lh, int q,
-                                           float (&f)[NB][4]) {
-#pragma unroll
-    for(int b = 0; b < NB; ++b) {
-        const f32x4 x =
-            *reinterpret_cast<const f32x4*>(lds + (r0 + b * 32 + lr) * KF + lh * 16 + 4 * q);
-        f[b][0] = x[0];
-        f[b][1] = x[1];
-        f[b][2] = x[2];
-        f[b][3] = x[3];
-    }
-}
-
-template <int TM, int TN>
-__device__ __forceinline__ void mfma_group(f32x16 (&acc)[TM][TN], const float (&fa)[TM][4],
-                                           const float (&fb)[TN][4]) {
-#pragma unroll
-    for(int t = 0; t < 4; ++t)
-#pragma unroll
-        for(int i = 0; i < TM; ++i)
-#pragma unroll
-            for(int j = 0; j < TN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][t], fb[j][t], acc[i][j], 0,
-                                                                 0, 0);
 }
 
 // Scheduling hints for one k-group: NMEM memory instructions (LDS or global)
@@ -457,237 +369,6 @@ __device__ __forceinline__ void stage(f32x4 (&ra)[NA], f32x4 (&rb)[NB], EA* sa, 
     }
 }
 
-// One workgroup's job: its tile, operand bases, output, K range.
-struct TileJob {
-    const float* A;
-    const float* B;
-    float* C;
-    const float* Cin;
-    int64_t ldc, ldcin, row0, col0, kbeg, kend;
-    float alpha, beta;
-    int nslices;
-    bool skip;
-};
-
-template <class T>
-__device__ __forceinline__ TileJob tile_job(const GemmParams& p) {
-    TileJob j;
-    // tile selection: XCD-contiguous runs, grouped by GROUP_M tile-rows
-    const int ntiles = p.tiles_m * p.tiles_n;
-    int bid = blockIdx.x;
-    if((ntiles & 7) == 0) bid = (bid & 7) * (ntiles >> 3) + (bid >> 3);
-    const int group_span = GROUP_M * p.tiles_n;
-    const int first_m = (bid / group_span) * GROUP_M;
-    const int gm = min(p.tiles_m - first_m, GROUP_M);
-    const int local = bid % group_span;
-    const int tm = first_m + local % gm;
-    const int tn = local / gm;
-
-    // blockIdx.y is the batch index, or the K slice of a split product
-    const int64_t z = p.splits > 1 ? 0 : blockIdx.y;
-    const int64_t zo = z / p.inner, zi = z % p.inner;
-    j.A = p.A + zo * p.sAo + zi * p.sAi;
-    j.B = p.B + zo * p.sBo + zi * p.sBi;
-    j.C = p.C + zo * p.sCo + zi * p.sCi;
-    j.ldc = p.ldc;
-    j.Cin = p.Cin ? p.Cin : j.C;
-    j.ldcin = p.Cin ? p.ldcin : p.ldc;
-    j.alpha = p.alpha;
-    j.beta = p.beta;
-
-    j.row0 = (int64_t)tm * T::BM;
-    j.col0 = (int64_t)tn * (p.pair_F ? T::BN / 2 : T::BN);
-    j.kbeg = 0;
-    j.kend = p.K;
-    j.skip = p.causal == 1 && j.col0 > j.row0 + T::BM - 1;  // wholly above the diagonal
-    if(p.causal == 2) j.kend = min(p.K, j.row0 + T::BM);
-    if(p.causal == 3) j.kbeg = min(p.K, (j.row0 / BK) * BK);
-    if(p.splits > 1) {
-        // slice s of K; its partial product goes to workspace plane s
-        j.kbeg = (int64_t)blockIdx.y * p.kchunk;
-        j.kend = min(p.K, j.kbeg + p.kchunk);
-        j.C = p.ws + (int64_t)blockIdx.y * p.M * p.N;
-        j.ldc = p.N;
-        j.Cin = j.C;
-        j.ldcin = p.N;
-        j.alpha = 1.0f;
-        j.beta = 0.0f;
-    }
-    j.nslices = (int)((j.kend - j.kbeg + BK - 1) / BK);
-    return j;
-}
-
-// C tile = alpha * acc (+ beta * C).  32x32 block accumulator r of lane l is
-// row 8*(r/4) + 4*(l/32) + r%4, column l%32: each half-wave writes 128
-// contiguous bytes per register.
-template <int EDGE, int TM, int TN>
-__device__ __forceinline__ void store_tile(const GemmParams& p, const TileJob& j,
-                                           const f32x16 (&acc)[TM][TN], int ar0, int br0, int lr,
-                                           int lh) {
-#pragma unroll
-    for(int i = 0; i < TM; ++i)
-#pragma unroll
-        for(int jj = 0; jj < TN; ++jj) {
-            const int64_t col = j.col0 + br0 + jj * 32 + lr;
-#pragma unroll
-            for(int r = 0; r < 16; ++r) {
-                const int64_t row = j.row0 + ar0 + i * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
-                if(EDGE != kEdgeNone && (row >= p.M || col >= p.N)) continue;
-                float v = j.alpha * acc[i][jj][r];
-                float* c = j.C + row * j.ldc + col;
-                if(j.beta != 0.0f) v += j.beta * *c;
-                // 64x64 tiles (products of about 1024^2 outputs, where the
-                // launch's end is a large share of its time) store C
-                // non-temporally: 1024^3 1.1-1.6 % and 768^3 0.6-1.1 % faster,
-                // config-4 and config-5 steps unchanged (same box, alternating);
-                // for every tile they cost a config-5 step 0.05 ms
-                if constexpr(TM * TN == 1) __builtin_nontemporal_store(v, c);
-                else *c = v;
-            }
-        }
-}
-
-// Epilogues that read other matrices: the tile goes through LDS (free once
-// the main loop is done) in passes of RP rows, and all 256 threads then walk
-// the staged rows in float4 runs, so every global access is a coalesced
-// 128-bit one and no per-element loads wait inside the accumulator loops
-// (which, in the 256x256 tile, also pushed the accumulators out of
-// registers).
-//   kEpiAdd:    C = alpha * acc + beta * Cin
-//   kEpiSwiglu: dh = alpha * acc; da (+)= dh*u*s*(1 + a*(1-s)), du (+)= dh*a*s
-//   kEpiSwigluFwd: the tile's two column halves are matching gate and up
-//               columns: C gets g = alpha * acc and u alike (as the plain
-//               store writes them), sf_h gets silu(g) * u
-constexpr int kEpiPlain = 0, kEpiAdd = 1, kEpiSwiglu = 2, kEpiSwigluFwd = 3;
-
-template <int EPI>
-__device__ __forceinline__ void epi_one(const GemmParams& p, const TileJob& j, int64_t row,
-                                        int64_t col, float x) {
-    if constexpr(EPI == kEpiAdd) {
-        float v = j.alpha * x;
-        if(j.beta != 0.0f) v += j.beta * j.Cin[row * j.ldcin + col];
-        j.C[row * j.ldc + col] = v;
-    } else {
-        float ga, gu;
-        pk::swiglu_bwd1(p.sg_a[row * p.sg_lda + col], p.sg_u[row * p.sg_ldu + col], j.alpha * x,
-                        ga, gu);
-        float* da = p.sg_da + row * p.sg_ldd + col;
-        float* du = p.sg_du + row * p.sg_ldd + col;
-        if(p.sg_flags & PK_ACCUM) ga = pk::add_nc(*da, ga);
-        if(p.sg_flags & PK_ACCUM2) gu = pk::add_nc(*du, gu);
-        *da = ga;
-        *du = gu;
-    }
-}
-
-template <int EPI>
-__device__ __forceinline__ void epi_four(const GemmParams& p, const TileJob& j, int64_t row,
-                                         int64_t col, f32x4 x) {
-    if constexpr(EPI == kEpiAdd) {
-        f32x4 v;
-#pragma unroll
-        for(int e = 0; e < 4; ++e) v[e] = j.alpha * x[e];
-        if(j.beta != 0.0f) {
-            const f32x4 c = *reinterpret_cast<const f32x4*>(j.Cin + row * j.ldcin + col);
-#pragma unroll
-            for(int e = 0; e < 4; ++e) v[e] += j.beta * c[e];
-        }
-        *reinterpret_cast<f32x4*>(j.C + row * j.ldc + col) = v;
-    } else {
-        const f32x4 a = *reinterpret_cast<const f32x4*>(p.sg_a + row * p.sg_lda + col);
-        const f32x4 u = *reinterpret_cast<const f32x4*>(p.sg_u + row * p.sg_ldu + col);
-        f32x4* dap = reinterpret_cast<f32x4*>(p.sg_da + row * p.sg_ldd + col);
-        f32x4* dup = reinterpret_cast<f32x4*>(p.sg_du + row * p.sg_ldd + col);
-        f32x4 pa = {0.f, 0.f, 0.f, 0.f}, pu = {0.f, 0.f, 0.f, 0.f};
-        if(p.sg_flags & PK_ACCUM) pa = *dap;
-        if(p.sg_flags & PK_ACCUM2) pu = *dup;
-        f32x4 ga, gu;
-#pragma unroll
-        for(int e = 0; e < 4; ++e) {
-            float y, z;
-            pk::swiglu_bwd1(a[e], u[e], j.alpha * x[e], y, z);
-            ga[e] = (p.sg_flags & PK_ACCUM) ? pk::add_nc(pa[e], y) : y;
-            gu[e] = (p.sg_flags & PK_ACCUM2) ? pk::add_nc(pu[e], z) : z;
-        }
-        *dap = ga;
-        *dup = gu;
-    }
-}
-
-template <int EPI, class T, int LDS_FLOATS>
-__device__ __forceinline__ void staged_epilogue(const GemmParams& p, const TileJob& j,
-                                                const f32x16 (&acc)[T::TM][T::TN], float* lds,
-                                                int ar0, int br0, int lr, int lh) {
-    constexpr int BN = T::BN, LDE = BN + 4, TM = T::TM, TN = T::TN;
-    // rows per pass: whole 32-row blocks that fit in the operand buffers
-    constexpr int rp = (LDS_FLOATS / LDE) / 32 * 32 < T::BM ? (LDS_FLOATS / LDE) / 32 * 32 : T::BM;
-    static_assert(rp >= 32, "the staging buffer must hold at least one 32-row block");
-    __syncthreads();  // every wave is done reading the operand tiles
-    for(int lo = 0; lo < T::BM; lo += rp) {
-#pragma unroll
-        for(int i = 0; i < TM; ++i) {
-            const int rb = ar0 + i * 32;
-            if(rb < lo || rb >= lo + rp) continue;
-#pragma unroll
-            for(int jj = 0; jj < TN; ++jj)
-#pragma unroll
-                for(int r = 0; r < 16; ++r)
-                    lds[(rb - lo + (r >> 2) * 8 + lh * 4 + (r & 3)) * LDE + br0 + jj * 32 + lr] =
-                        acc[i][jj][r];
-        }
-        __syncthreads();
-        const int rows = rp < T::BM - lo ? rp : T::BM - lo;
-        if constexpr(EPI == kEpiSwigluFwd) {
-            // column c of the gate half pairs with column BN/2 + c; the host
-            // guarantees whole column halves (pair_F a multiple of BN/2)
-            constexpr int HB = BN / 2;
-            for(int idx = threadIdx.x; idx < rows * (HB / 4); idx += NT) {
-                const int rr = idx / (HB / 4), c = (idx % (HB / 4)) * 4;
-                const int64_t row = j.row0 + lo + rr, col = j.col0 + c;
-                if(row >= p.M) continue;
-                const f32x4 g = *reinterpret_cast<const f32x4*>(lds + rr * LDE + c);
-                const f32x4 u = *reinterpret_cast<const f32x4*>(lds + rr * LDE + HB + c);
-                f32x4 gv, uv, hv;
-#pragma unroll
-                for(int e = 0; e < 4; ++e) {
-                    gv[e] = j.alpha * g[e];
-                    uv[e] = j.alpha * u[e];
-                    hv[e] = pk::swiglu_fwd1(gv[e], uv[e]);
-                }
-                float* cg = j.C + row * j.ldc + col;
-                float* hp = p.sf_h + row * p.sf_ldh + col;
-                if(p.epi_vec) {
-                    *reinterpret_cast<f32x4*>(cg) = gv;
-                    *reinterpret_cast<f32x4*>(cg + p.pair_F) = uv;
-                    *reinterpret_cast<f32x4*>(hp) = hv;
-                } else {
-#pragma unroll
-                    for(int e = 0; e < 4; ++e) {
-                        cg[e] = gv[e];
-                        cg[p.pair_F + e] = uv[e];
-                        hp[e] = hv[e];
-                    }
-                }
-            }
-        } else {
-            for(int idx = threadIdx.x; idx < rows * (BN / 4); idx += NT) {
-                const int rr = idx / (BN / 4), c = (idx % (BN / 4)) * 4;
-                const int64_t row = j.row0 + lo + rr, col = j.col0 + c;
-                const f32x4 x = *reinterpret_cast<const f32x4*>(lds + rr * LDE + c);
-                if(row >= p.M) continue;
-                if(p.epi_vec && col + 3 < p.N) {
-                    epi_four<EPI>(p, j, row, col, x);
-                } else {
-#pragma unroll
-                    for(int e = 0; e < 4; ++e)
-                        if(col + e < p.N) epi_one<EPI>(p, j, row, col + e, x[e]);
-                }
-            }
-        }
-        __syncthreads();
-    }
-}
-
 // prologue shared by both kernels: slice 0 into LDS buffer 0, slice 1 into
 // the staging registers
 template <bool AK, bool BKF, int EDGE, class T, bool PAIR = false, int NA, int NB, class EA,
@@ -717,142 +398,10 @@ __device__ __forceinline__ void prologue(const GemmParams& p, const TileJob& j, 
                                           &rb[e], p.pair_F - T::BN / 2);
 }
 
-// the tiles that can hold a second slice in their staging registers
-template <class T>
-constexpr bool deep_staging() {
-    return T::BM * T::BN <= 128 * 128 || (T::BM == 256 && T::BN == 96);
-}
-
-template <bool TA, bool TB, int EDGE, class T, int EPI, bool DEEP = false>
-__global__ __launch_bounds__(NT, T::OCC) void gemm_f32_kernel(GemmParams p) {
-    constexpr int BM = T::BM, BN = T::BN, TM = T::TM, TN = T::TN, WGN = T::WGN;
-    // op(A) rows are k-contiguous when A is not transposed; op(B)^T rows
-    // (indexed by n) are k-contiguous when B is transposed.
-    constexpr bool AK = !TA, BKF = TB;
-    using OA = Operand<AK, BM>;
-    using OB = Operand<BKF, BN>;
-    using S = Staging<AK, BKF, T>;
-    __shared__ __attribute__((aligned(16))) float ldsA[2][OA::FLOATS];
-    __shared__ __attribute__((aligned(16))) float ldsB[2][OB::FLOATS];
-
-    const TileJob job = tile_job<T>(p);
-    if(job.skip) return;
-    const float* __restrict__ A = job.A;
-    const float* __restrict__ B = job.B;
-    const int64_t row0 = job.row0, col0 = job.col0, kbeg = job.kbeg, kend = job.kend;
-    const int nslices = job.nslices;
-
-    const int w = threadIdx.x / 64, l = threadIdx.x % 64;
-    const int wm = w / WGN, wn = w % WGN;
-    const int lr = l & 31, lh = l >> 5;
-    const int ar0 = wm * TM * 32, br0 = wn * TN * 32;
-
-    f32x16 acc[TM][TN];
-#pragma unroll
-    for(int i = 0; i < TM; ++i)
-#pragma unroll
-        for(int j = 0; j < TN; ++j)
-#pragma unroll
-            for(int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    constexpr int RD = TM + TN;  // 128-bit LDS reads per k-group
-    constexpr int NMFMA = TM * TN * 4;
-
-    if(nslices > 0) {
-        constexpr bool PAIR = EPI == kEpiSwigluFwd;
-        // DEEP (tiles of at most 128x128, whose slices are short: 0.4-1.7 us,
-        // and 256x96, one workgroup per CU): two slices in the staging
-        // registers, fetched three slices ahead, so a load has two slices'
-        // time to arrive rather than one.  It costs 15-60 VGPRs, which the
-        // launcher spends only on unsplit products; 256x256 has none to spare
-        constexpr bool PF2 = DEEP && deep_staging<T>();
-        constexpr int AHEAD = PF2 ? 3 : 2;
-        f32x4 ra[OA::F4], rb[OB::F4];
-        prologue<AK, BKF, EDGE, T, PAIR>(p, job, ra, rb, ldsA[0], ldsB[0]);
-        f32x4 ra2[PF2 ? OA::F4 : 1], rb2[PF2 ? OB::F4 : 1];
-        if constexpr(PF2) {
-            const int64_t k2 = kbeg + (int64_t)min(2, nslices - 1) * BK;
-#pragma unroll
-            for(int e = 0; e < OA::ITEMS; ++e)
-                load_item<AK, EDGE, BM>(A, p.lda, row0, k2, p.M, kend, e, &ra2[e]);
-#pragma unroll
-            for(int e = 0; e < OB::ITEMS; ++e)
-                load_item<BKF, EDGE, BN, PAIR>(B, p.ldb, col0, k2, p.N, kend, e, &rb2[e],
-                                               p.pair_F - BN / 2);
-        }
-        __syncthreads();
-        float fa0[TM][4], fb0[TN][4], fa1[TM][4], fb1[TN][4];
-        read_group<TM>(ldsA[0], ar0, lr, lh, 0, fa0);
-        read_group<TN>(ldsB[0], br0, lr, lh, 0, fb0);
-        // slice s: stage (xa, xb) -- slice s+1 -- into the other LDS buffer and
-        // refill them with slice s+AHEAD; past the end the refill re-fetches the
-        // last slice, which keeps the loop free of branches
-        auto slice = [&](int s, f32x4 (&xa)[OA::F4], f32x4 (&xb)[OB::F4]) {
-            const int cur = s & 1;
-            const float* la = ldsA[cur];
-            const float* lb = ldsB[cur];
-            float* sa = ldsA[cur ^ 1];
-            float* sb = ldsB[cur ^ 1];
-            const int64_t kn = kbeg + (int64_t)min(s + AHEAD, nslices - 1) * BK;
-
-            // group 0: read group 1, stage part 0
-            read_group<TM>(la, ar0, lr, lh, 1, fa1);
-            read_group<TN>(lb, br0, lr, lh, 1, fb1);
-            stage<AK, BKF, EDGE, T, 0, PAIR>(xa, xb, sa, sb, A, B, p, row0, col0, kn, kend);
-            mfma_group<TM, TN>(acc, fa0, fb0);
-            interleave<NMFMA, RD + S::group_ops(0)>();
-            __builtin_amdgcn_sched_barrier(0);
-            // group 1: read group 2, stage part 1
-            read_group<TM>(la, ar0, lr, lh, 2, fa0);
-            read_group<TN>(lb, br0, lr, lh, 2, fb0);
-            stage<AK, BKF, EDGE, T, 1, PAIR>(xa, xb, sa, sb, A, B, p, row0, col0, kn, kend);
-            mfma_group<TM, TN>(acc, fa1, fb1);
-            interleave<NMFMA, RD + S::group_ops(1)>();
-            __builtin_amdgcn_sched_barrier(0);
-            // group 2: read group 3, stage part 2
-            read_group<TM>(la, ar0, lr, lh, 3, fa1);
-            read_group<TN>(lb, br0, lr, lh, 3, fb1);
-            stage<AK, BKF, EDGE, T, 2, PAIR>(xa, xb, sa, sb, A, B, p, row0, col0, kn, kend);
-            mfma_group<TM, TN>(acc, fa0, fb0);
-            interleave<NMFMA, RD + S::group_ops(2)>();
-            __builtin_amdgcn_sched_barrier(0);
-            // every wave has staged slice s+1 and finished reading slice s
-            __syncthreads();
-            // group 3, with group 0 of slice s+1 read underneath (on the last
-            // slice this reads the re-staged data and is discarded)
-            read_group<TM>(sa, ar0, lr, lh, 0, fa0);
-            read_group<TN>(sb, br0, lr, lh, 0, fb0);
-            mfma_group<TM, TN>(acc, fa1, fb1);
-            interleave<NMFMA, RD>();
-            __builtin_amdgcn_sched_barrier(0);
-        };
-        if constexpr(PF2) {
-            // even slices stage ra/rb, odd ones ra2/rb2
-            int s = 0;
-            for(; s + 1 < nslices; s += 2) {
-                slice(s, ra, rb);
-                slice(s + 1, ra2, rb2);
-            }
-            if(s < nslices) slice(s, ra, rb);
-        } else {
-            for(int s = 0; s < nslices; ++s) slice(s, ra, rb);
-        }
-    }
-    if constexpr(EPI == kEpiPlain)
-        store_tile<EDGE, TM, TN>(p, job, acc, ar0, br0, lr, lh);
-    else if constexpr(sizeof(ldsA) >= sizeof(ldsB))
-        staged_epilogue<EPI, T, sizeof(ldsA) / sizeof(float)>(p, job, acc, &ldsA[0][0], ar0, br0,
-                                                             lr, lh);
-    else
-        staged_epilogue<EPI, T, sizeof(ldsB) / sizeof(float)>(p, job, acc, &ldsB[0][0], ar0, br0,
-                                                             lr, lh);
-}
-
 // The same product with bf16 multiplies: op(A) and op(B) are rounded to bf16
 // (nearest even) on their way to LDS and multiplied by
 // v_mfma_f32_32x32x16_bf16 (32768 FLOP per instruction, eight times the fp32
-// rate), accumulating in fp32.  Global traffic, staging, tiles and split-K
-// are the fp32 kernel's; a 32-wide k slice is two MFMA steps of k 16, the
+// rate), accumulating in fp32.  A 32-wide k slice is two MFMA steps of k 16, the
 // second step's fragments read under the first step's MFMAs and the next
 // slice's first fragments under the second.  A lane's 8 k of a step are k
 // 16t + 8*(lane/32) .. +7, the same for both operands.
@@ -1396,8 +945,6 @@ __global__ void splitk_reduce(int64_t M, int64_t N, int S, const float* __restri
 // Examples: 4096^2 -> 256 tiles of 256x256; an [8192, 768] output (every
 // projection of a d_model-768 transformer) -> 256 of 256x96; 2048^2 -> 256
 // of 128x128; 1024^2 -> 256 of 64x64 rather than 64 of 128x128.
-enum TileKind { kTile128, kTile96, kTile256, kTile64, kTile256x96 };
-
 struct TileChoice {
     TileKind kind;
     int bm, bn;
@@ -1523,18 +1070,6 @@ void launch_epi(const GemmParams& gp, dim3 grid, int prec, hipStream_t st) {
         gemm_bf16_kernel<TA, TB, EDGE, T, false, EPI><<<grid, NT, 0, st>>>(gp);
     else if(prec == kBf16x3)
         gemm_bf16_kernel<TA, TB, EDGE, T, true, EPI><<<grid, NT, 0, st>>>(gp);
-    else if constexpr(deep_staging<T>()) {
-        // unsplit products of the small tiles stage two slices ahead; a split
-        // product (weight gradients, concurrent with other work) keeps the
-        // smaller register footprint, which lets more of that work share its
-        // CUs (a config-5 step measured 0.5 ms slower with both deep)
-        if(gp.splits == 1)
-            gemm_f32_kernel<TA, TB, EDGE, T, EPI, true><<<grid, NT, 0, st>>>(gp);
-        else
-            gemm_f32_kernel<TA, TB, EDGE, T, EPI><<<grid, NT, 0, st>>>(gp);
-    } else {
-        gemm_f32_kernel<TA, TB, EDGE, T, EPI><<<grid, NT, 0, st>>>(gp);
-    }
 }
 
 // The staged epilogues are instantiated only where they are used: the
@@ -1661,6 +1196,7 @@ int gemm_impl(char ta, char tb, int64_t M, int64_t N, int64_t K, float alpha, co
     gp.pair_F = 0;
     gp.sf_h = nullptr;
     gp.sf_ldh = 0;
+    gp.exact_only = 0;
     if(sfwd) {
         if(TA || TB || batch != 1 || causal != 0 || beta != 0.0f || !own_c)
             return pk::fail("pk_gemm_swiglu_fwd_f32: only the plain ('N','N') product is built");
@@ -1756,61 +1292,56 @@ int gemm_impl(char ta, char tb, int64_t M, int64_t N, int64_t K, float alpha, co
     // is exercised at that size)
     TileChoice tc = gp.splits > 1 ? TileChoice{kTile128, 128, 128}
                                   : pick_tile(M, N, batch, causal == 0, gp.pair_F);
-    // a short K over two or more rounds of 256x256 tiles (fp32, unsplit):
-    // 128x128 tiles with the two-slice staging, two per CU, where one tile's
-    // C stores and first loads overlap the other's products.  Measured in the
-    // config-5 forward (the SwiGLU-forward [8192, 4096] and LM-head [8192,
-    // 32000] products, K 768) and config 4's LM head ([4096, 8192], K 512):
-    // config-5 step 46.36-46.44 -> 46.16-46.23 ms on one box, 47.48-47.56 ->
-    // 47.40-47.46 on another.  One round (4096^2) and long K (8192^3) keep
-    // 256x256.
-    if(prec == kFp32 && gp.splits == 1 && tc.kind == kTile256 && K <= 1024 &&
-       ((M + 255) / 256) * ((N + 255) / 256) * batch > kCUs &&
-       (gp.pair_F == 0 || gp.pair_F % 64 == 0))
-        tc = TileChoice{kTile128, 128, 128};
-    // A.B products on 256x96 tiles (one per CU) take 128x96 (two per CU,
-    // two-slice staging), so one tile's start and C writes overlap the other's
-    // products.  In a training step the A.B products are the forward's, which
-    // run alone: config 5's Q/K/V projection 213 -> 207 us, the residual-add
-    // products 81 -> 76 us (K 768) and 184 -> 180 us (K 2048), step 46.63-46.67
-    // -> 46.36-46.39 ms.  A.B^T and A^T.B keep 256x96: the backward runs them
-    // beside the weight-gradient stream, where 128x96 cost the step 0.75 ms.
-    if(prec == kFp32 && gp.splits == 1 && tc.kind == kTile256x96 && !TA && !TB)
-        tc = TileChoice{kTile96, 128, 96};
     if(tc.bm == 0)
         return pk::fail("pk_gemm_swiglu_fwd_f32: F=%lld is not a multiple of 32 (no tile holds "
                         "whole gate/up column pairs)", (long long)gp.pair_F);
-    const int64_t tiles_m = (M + tc.bm - 1) / tc.bm, tiles_n = (N + tc.bn - 1) / tc.bn;
+    // fp32: the SwiGLU-forward product takes the plain product's shape (its
+    // tiles may hold partial columns), so both add K in the same order
+    if(prec == kFp32 && gp.pair_F) tc = pick_tile(M, N, batch, causal == 0);
+    const int64_t tiles_m = (M + tc.bm - 1) / tc.bm,
+                  tiles_n = gp.pair_F ? (gp.pair_F + tc.bn / 2 - 1) / (tc.bn / 2)
+                                      : (N + tc.bn - 1) / tc.bn;
     if(tiles_m * tiles_n > (int64_t)1 << 30)
         return pk::fail("pk_gemm_f32: problem too large for one launch");
     gp.tiles_m = (int)tiles_m;
     gp.tiles_n = (int)tiles_n;
-    // float4 loads need 16-byte aligned operands and leading dimensions and
-    // batch strides that are multiples of 4; the unchecked path also needs
-    // whole tiles
-    const bool vec = (lda % 4) == 0 && (ldb % 4) == 0 && (sA_outer % 4) == 0 &&
-                     (sA_inner % 4) == 0 && (sB_outer % 4) == 0 && (sB_inner % 4) == 0 &&
-                     pk::aligned16(A) && pk::aligned16(B);
-    const bool whole = (M % tc.bm) == 0 && (N % tc.bn) == 0 && (K % BK) == 0;
-    // whole tiles load through buffer resources with 32-bit offsets from each
-    // operand's start: op(A) and op(B) must each span less than 2^31 bytes
-    auto extent = [K](bool kfast, int64_t rows, int64_t ld) {
-        return 4 * (kfast ? (rows - 1) * ld + K : (K - 1) * ld + rows);
-    };
-    const bool small = extent(!TA, M, lda) < INT32_MAX && extent(TB, N, ldb) < INT32_MAX;
-    const int edge = vec && whole && small ? kEdgeNone
-                     : vec && (M % 4) == 0 && (N % 4) == 0 && (K % 4) == 0 ? kEdgeVec
-                                                                           : kEdgeScalar;
     const TileKind kind = tc.kind;
     int rc;
-    if(!TA && !TB)
-        rc = launch<false, false>(gp, batch, edge, kind, prec, st);
-    else if(!TA && TB)
-        rc = launch<false, true>(gp, batch, edge, kind, prec, st);
-    else if(TA && !TB)
-        rc = launch<true, false>(gp, batch, edge, kind, prec, st);
-    else
-        rc = launch<true, true>(gp, batch, edge, kind, prec, st);
+    if(prec == kFp32) {
+        const int64_t kstep = 32 * split_groups(kind);
+        const bool whole = M % tc.bm == 0 && K % kstep == 0 && gp.kchunk % kstep == 0 &&
+                           (gp.pair_F ? gp.pair_F % (tc.bn / 2) == 0 : N % tc.bn == 0);
+        // a tile's loads reach 32-bit byte offsets: 256 rows of a k-contiguous
+        // operand, 16 k rows of the other kind
+        const int64_t near_k = (int64_t)1 << 21, near_r = (int64_t)1 << 25;
+        gp.exact_only = lda > (TA ? near_r : near_k) || ldb > (TB ? near_k : near_r);
+        rc = launch_split(TA, TB, gp, batch, !whole, kind, st);
+    } else {
+        // float4 loads need 16-byte aligned operands and leading dimensions and
+        // batch strides that are multiples of 4; the unchecked path also needs
+        // whole tiles
+        const bool vec = (lda % 4) == 0 && (ldb % 4) == 0 && (sA_outer % 4) == 0 &&
+                         (sA_inner % 4) == 0 && (sB_outer % 4) == 0 && (sB_inner % 4) == 0 &&
+                         pk::aligned16(A) && pk::aligned16(B);
+        const bool whole = (M % tc.bm) == 0 && (N % tc.bn) == 0 && (K % BK) == 0;
+        // whole tiles load through buffer resources with 32-bit offsets from each
+        // operand's start: op(A) and op(B) must each span less than 2^31 bytes
+        auto extent = [K](bool kfast, int64_t rows, int64_t ld) {
+            return 4 * (kfast ? (rows - 1) * ld + K : (K - 1) * ld + rows);
+        };
+        const bool small = extent(!TA, M, lda) < INT32_MAX && extent(TB, N, ldb) < INT32_MAX;
+        const int edge = vec && whole && small ? kEdgeNone
+                         : vec && (M % 4) == 0 && (N % 4) == 0 && (K % 4) == 0 ? kEdgeVec
+                                                                               : kEdgeScalar;
+        if(!TA && !TB)
+            rc = launch<false, false>(gp, batch, edge, kind, prec, st);
+        else if(!TA && TB)
+            rc = launch<false, true>(gp, batch, edge, kind, prec, st);
+        else if(TA && !TB)
+            rc = launch<true, false>(gp, batch, edge, kind, prec, st);
+        else
+            rc = launch<true, true>(gp, batch, edge, kind, prec, st);
+    }
     if(rc || gp.splits == 1) return rc;
     splitk_reduce<<<pk::grid_for(M * N / 4 + 1, NT), NT, 0, st>>>(
         M, N, gp.splits, gp.ws, alpha, beta, gp.Cin ? gp.Cin : C, gp.Cin ? gp.ldcin : ldc, C, ldc);

@@ -1,0 +1,461 @@
+// pico_amd/csrc/gemm_split.h -- the fp32 product on the bf16 matrix cores.
+// Part of gemm_split.hip (included inside its anonymous namespace).
+//
+// The fp32 matrix cores are 16 times slower than the bf16 ones, and a SIMD's
+// vector instructions do not overlap fp32 matrix instructions while they do
+// overlap bf16 ones (up to about six per 32x32x16 instruction, measured with
+// independent streams of both).  So an fp32 operand is taken as the exact sum
+// of three bf16 parts, x = h + m + l (8 significant bits each, rounded to
+// nearest, 24 in all), on its way to LDS, and
+//     a.b = hh + hm + mh + mm + hl + lh
+// in six matrix instructions per 16 k; ml, lm and ll, together below 2^-24 of
+// |a||b|, are left out.  Nothing is held in less than fp32's 24 bits, and the
+// sums are fp32.  Against float64 the error is below that of the fp32 matrix
+// instructions (which round after every k): normal operands, relative
+// 2-norm, K 768 / 2048 / 4096: 2.9e-7 / 6.9e-7 / 9.7e-7 against 5.0e-7 /
+// 8.1e-7 / 1.15e-6.
+//  * Range: operands are scaled by 2^16, so that the parts of every normal and
+//    subnormal fp32 number are exact bf16 numbers (l of a 2^-126 would need
+//    2^-149), and the sums by 2^-32 at the end.  What overflows (values above
+//    2^111, sums above 2^96, infinities) or is NaN leaves a non-finite sum: a
+//    wave that sees one computes its tile again on the fp32 cores, from global
+//    memory (exact_tile).
+//  * Sign: the matrix unit drops the low bits of products much smaller than the
+//    accumulator towards minus infinity.  One sum loses less than its
+//    roundings, but the loss has the same sign in every output, so it would
+//    add up in a sum over outputs (a bias gradient, an attention average:
+//    the mean error of [8192, 2304] outputs with K 768 was 2e-6 of the value
+//    in such a sum).  So the parts of op(A) change sign with the sums every
+//    128 k (K group by K group where a workgroup splits K), and the loss
+//    cancels: mean error below 2e-9 of the root mean square.
+//  * Bound: 6 instructions of 32 cycles per 32x32 block and 16 k, 2.5 PFLOP/s /
+//    6 = 417 TFLOP/s at the nominal clock; the card settles near 2.06 GHz under
+//    bf16 matrix load (358).  The split costs 6.5 vector instructions per staged
+//    value, 1.1-4.6 per matrix instruction depending on the tile.  Splitting
+//    when the fragments are read instead would stage 4 bytes a value, but each
+//    value is read by several waves.
+//  * Tiles: at least two waves per SIMD, so that one wave's staging and LDS
+//    latency hides under the other's matrix work; where a tile has only four
+//    waves, G groups of them take every G-th slice of K into LDS buffers of
+//    their own and add their sums at the end (256x96: 166 -> 197 TFLOP/s at
+//    [8192, 768] K 2304; 64x64 with G 4: 84 -> 114 at 1024^3).
+//  * A slice is 16 k.  Its first half multiplies m.m, m.h, h.m while l is read,
+//    the next slice is split and stored and the slice after it fetched; one
+//    barrier; then h.l, l.h, h.h while the next slice's m and h are read into
+//    the fragments that are free by then.
+//  * Loads go through buffer resources that end where the operand ends, 128 bits
+//    at any 4-byte alignment, so ragged sizes take the same path: what lies
+//    behind the end reads as zero, and only a partial last slice is masked.
+//    (The per-element edge path this replaces: 2000x1503x1001 at 58 TFLOP/s,
+//    now 105.)
+//
+// 4096^3 A.B / A.B^T / A^T.B 244-246 TFLOP/s (149 on the fp32 cores), 8192^3
+// 237-243 (151), 2048^3 186-189 (142).
+
+// A tile shape: WM x WN waves, each TM x TN blocks of 32 x 32; WPS waves per SIMD.
+template <int WM_, int WN_, int TM_, int TN_, int G_, int WPS_, int PF_>
+struct SplitTile {
+    static constexpr int WGM = WM_, WGN = WN_, TM = TM_, TN = TN_, G = G_;
+    static constexpr int WPS = WPS_, PF = PF_;
+    static constexpr int BM = WM_ * TM_ * 32, BN = WN_ * TN_ * 32;
+    static constexpr int WAVES = WM_ * WN_;                    // of one K group
+    static constexpr int GTHREADS = 64 * WAVES, THREADS = GTHREADS * G_;
+};
+
+constexpr int SK = 16;  // k per slice: one v_mfma_f32_32x32x16_bf16 step
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+
+// One operand's R x 16 slice as staged by THREADS threads: items of KPI
+// consecutive k of one row, ITEMS per thread (threads past the last item
+// repeat an earlier one).
+template <bool KFAST, int R, int THREADS>
+struct SplitOperand {
+    static constexpr int KPI = KFAST ? 4 : (R * 2 >= THREADS ? 8 : 4);
+    static constexpr int COUNT = R * SK / KPI;
+    static constexpr int ITEMS = (COUNT + THREADS - 1) / THREADS;
+    static constexpr int LOADS = KFAST ? 1 : KPI;
+
+    static __device__ __forceinline__ void origin(int item, int& rr, int& kk) {
+        int u = threadIdx.x % THREADS + item * THREADS;
+        if(ITEMS * THREADS != COUNT) u %= COUNT;
+        if(KFAST) {
+            rr = u >> 2;
+            kk = (u & 3) * 4;
+        } else {
+            rr = u % R;
+            kk = (u / R) * KPI;
+        }
+    }
+};
+
+// The operand as buffer loads see it: bytes from `base` to its end.
+struct SplitSource {
+    const char* base;  // element (first row of the tile, k 0)
+    int64_t left;      // bytes from base to the end of the operand
+    int64_t kstep;     // bytes per k
+};
+
+template <bool KFAST, bool EDGE, int R, int THREADS, bool PAIR>
+__device__ __forceinline__ void split_load(const SplitSource& src, int64_t ld, int64_t k0,
+                                           int64_t shift,
+                                           float (&v)[SplitOperand<KFAST, R, THREADS>::ITEMS]
+                                                     [SplitOperand<KFAST, R, THREADS>::KPI]) {
+    using O = SplitOperand<KFAST, R, THREADS>;
+    const int64_t off = k0 * src.kstep;
+    const int64_t left = src.left - off;
+    const unsigned num = EDGE ? (left <= 0 ? 0u : left > 0xfffffff0ll ? 0xfffffff0u : (unsigned)left)
+                              : 0xfffffff0u;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(src.base + off), (short)0, (int)num, 0x00020000);
+#pragma unroll
+    for(int i = 0; i < O::ITEMS; ++i) {
+        int rr, kk;
+        O::origin(i, rr, kk);
+        const unsigned row = (unsigned)rr + (PAIR && rr >= R / 2 ? (unsigned)shift : 0u);
+        if(KFAST) {
+            const int voff = (int)((row * (unsigned)ld + kk) * 4u);
+            const f32x4 x =
+                __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, 0, 0));
+#pragma unroll
+            for(int t = 0; t < 4; ++t) v[i][t] = x[t];
+        } else {
+            const int voff = (int)((kk * (unsigned)ld + row) * 4u);
+#pragma unroll
+            for(int t = 0; t < O::KPI; ++t)
+                v[i][t] = __builtin_bit_cast(
+                    float, __builtin_amdgcn_raw_buffer_load_b32(rs, voff, (int)(t * (unsigned)ld * 4u), 0));
+        }
+    }
+}
+
+// zero the values at k >= limit (limit < 16: the last, partial slice)
+template <bool KFAST, int R, int THREADS>
+__device__ __forceinline__ void split_mask(int limit,
+                                           float (&v)[SplitOperand<KFAST, R, THREADS>::ITEMS]
+                                                     [SplitOperand<KFAST, R, THREADS>::KPI]) {
+    using O = SplitOperand<KFAST, R, THREADS>;
+#pragma unroll
+    for(int i = 0; i < O::ITEMS; ++i) {
+        int rr, kk;
+        O::origin(i, rr, kk);
+#pragma unroll
+        for(int t = 0; t < O::KPI; ++t) v[i][t] = kk + t < limit ? v[i][t] : 0.0f;
+    }
+}
+
+// two values as three bf16 pairs: x * scale = h + m + l exactly (scale a power of two)
+__device__ __forceinline__ void split3(float x0, float x1, float scale, int& h, int& m, int& l) {
+    const f32x2 x = {x0 * scale, x1 * scale};
+    const bf16x2 hv = __builtin_convertvector(x, bf16x2);
+    const f32x2 r = {x[0] - (float)hv[0], x[1] - (float)hv[1]};
+    const bf16x2 mv = __builtin_convertvector(r, bf16x2);
+    const f32x2 q = {r[0] - (float)mv[0], r[1] - (float)mv[1]};
+    const bf16x2 lv = __builtin_convertvector(q, bf16x2);
+    h = __builtin_bit_cast(int, hv);
+    m = __builtin_bit_cast(int, mv);
+    l = __builtin_bit_cast(int, lv);
+}
+
+// LDS: [part][row][16 k], rows of 32 bytes whose two 16-byte halves swap places
+// every 4 rows, so the 8 lanes of a 128-bit access phase (8 rows 32 bytes
+// apart) fall in distinct banks.  Offset in 16-bit elements of (row, k):
+__device__ __forceinline__ int split_off(int row, int k) {
+    return row * SK + ((((k >> 3) ^ (row >> 2)) & 1) << 3) + (k & 7);
+}
+
+template <bool KFAST, int R, int THREADS, int PART>
+__device__ __forceinline__ void split_store(short* lds,
+                                            const float (&v)[SplitOperand<KFAST, R, THREADS>::ITEMS]
+                                                            [SplitOperand<KFAST, R, THREADS>::KPI],
+                                            float scale) {
+    using O = SplitOperand<KFAST, R, THREADS>;
+#pragma unroll
+    for(int i = 0; i < O::ITEMS; ++i) {
+        int rr, kk;
+        O::origin(i, rr, kk);
+        const int off = split_off(rr, kk);
+        int w[3][O::KPI / 2];
+#pragma unroll
+        for(int t = 0; t < O::KPI / 2; ++t)
+            split3(v[i][2 * t], v[i][2 * t + 1], scale, w[0][t], w[1][t], w[2][t]);
+#pragma unroll
+        for(int q = 0; q < 3; ++q) {
+            if constexpr(O::KPI == 8)
+                *reinterpret_cast<i32x4*>(lds + q * PART + off) =
+                    i32x4{w[q][0], w[q][1], w[q][2], w[q][3]};
+            else
+                *reinterpret_cast<i32x2*>(lds + q * PART + off) = i32x2{w[q][0], w[q][1]};
+        }
+    }
+}
+
+template <int TM, int TN>
+struct SplitFrag {
+    bf16x8 a[TM], b[TN];
+};
+
+// the wave's tile again on the fp32 matrix cores, straight from global memory
+// with 64-bit addresses: for a wave whose split sums are not finite, and for
+// operands whose rows are too far apart for buffer offsets
+template <bool TA, bool TB, bool PAIR, class T>
+__device__ __forceinline__ void exact_tile(const GemmParams& p, const TileJob& j,
+                                                     f32x16 (&acc)[T::TM][T::TN], int ar0, int br0,
+                                                     int lr, int lh) {
+    constexpr int TM = T::TM, TN = T::TN;
+#pragma unroll
+    for(int i = 0; i < TM; ++i)
+#pragma unroll
+        for(int jj = 0; jj < TN; ++jj)
+#pragma unroll
+            for(int r = 0; r < 16; ++r) acc[i][jj][r] = 0.0f;
+#pragma unroll 1
+    for(int64_t k0 = j.kbeg; k0 < j.kend; k0 += 8) {
+        const int64_t k = k0 + lh * 4;
+        float fa[TM][4], fb[TN][4];
+#pragma unroll
+        for(int i = 0; i < TM; ++i) {
+            const int64_t r = min(j.row0 + ar0 + i * 32 + lr, p.M - 1);
+#pragma unroll
+            for(int t = 0; t < 4; ++t) {
+                const int64_t kc = min(k + t, j.kend - 1);
+                const float x = j.A[TA ? kc * p.lda + r : r * p.lda + kc];
+                fa[i][t] = k + t < j.kend ? x : 0.0f;
+            }
+        }
+#pragma unroll
+        for(int jj = 0; jj < TN; ++jj) {
+            const int c = br0 + jj * 32 + lr;
+            const int64_t n = min(j.col0 + c + (PAIR && c >= T::BN / 2 ? p.pair_F - T::BN / 2 : 0),
+                                  p.N - 1);
+#pragma unroll
+            for(int t = 0; t < 4; ++t) {
+                const int64_t kc = min(k + t, j.kend - 1);
+                const float x = j.B[TB ? n * p.ldb + kc : kc * p.ldb + n];
+                fb[jj][t] = k + t < j.kend ? x : 0.0f;
+            }
+        }
+#pragma unroll
+        for(int t = 0; t < 4; ++t)
+#pragma unroll
+            for(int i = 0; i < TM; ++i)
+#pragma unroll
+                for(int jj = 0; jj < TN; ++jj)
+                    acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][t], fb[jj][t],
+                                                                      acc[i][jj], 0, 0, 0);
+    }
+}
+
+// one MFMA, then its share of the phase's other instructions
+template <int N, int DSR, int VALU, int DSW, int VM, int I = 0>
+__device__ __forceinline__ void split_sched() {
+    if constexpr(I < N) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        constexpr int r = (I + 1) * DSR / N - I * DSR / N, v = (I + 1) * VALU / N - I * VALU / N,
+                      w = (I + 1) * DSW / N - I * DSW / N, g = (I + 1) * VM / N - I * VM / N;
+        if constexpr(r > 0) __builtin_amdgcn_sched_group_barrier(0x100, r, 0);
+        if constexpr(v > 0) __builtin_amdgcn_sched_group_barrier(0x002, v, 0);
+        if constexpr(w > 0) __builtin_amdgcn_sched_group_barrier(0x200, w, 0);
+        if constexpr(g > 0) __builtin_amdgcn_sched_group_barrier(0x020, g, 0);
+        split_sched<N, DSR, VALU, DSW, VM, I + 1>();
+    }
+}
+
+template <bool TA, bool TB, bool EDGE, class T, int EPI>
+__global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmParams p) {
+    constexpr int BM = T::BM, BN = T::BN, TM = T::TM, TN = T::TN, NT_ = T::GTHREADS, G = T::G;
+    constexpr bool AK = !TA, BKF = TB, PAIR = EPI == kEpiSwigluFwd;
+    using OA = SplitOperand<AK, BM, NT_>;
+    using OB = SplitOperand<BKF, BN, NT_>;
+    constexpr int PART = (BM + BN) * SK, STAGE = 3 * PART;  // 16-bit elements
+    __shared__ __attribute__((aligned(16))) short lds_all[G * 2 * STAGE];
+
+    const TileJob job = tile_job<T>(p);
+    if(job.skip) return;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), l = threadIdx.x % 64;
+    const int g = G > 1 ? wv / T::WAVES : 0, w = G > 1 ? wv % T::WAVES : wv;
+    const int wm = w / T::WGN, wn = w % T::WGN;
+    const int lr = l & 31, lh = l >> 5;
+    const int ar0 = wm * TM * 32, br0 = wn * TN * 32;
+    short* const lds = lds_all + g * 2 * STAGE;
+    // slices per group, an even number
+    const int nslices =
+        p.exact_only ? 0 : (int)((job.kend - job.kbeg + 2 * G * SK - 1) / (2 * G * SK)) * 2;
+
+    f32x16 acc[TM][TN];
+#pragma unroll
+    for(int i = 0; i < TM; ++i)
+#pragma unroll
+        for(int j = 0; j < TN; ++j)
+#pragma unroll
+            for(int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+    // the scale of op(A)'s parts, whose sign the sums share
+    float scale = G > 1 && (g & 1) ? -0x1p16f : 0x1p16f;
+    if(nslices > 0) {
+        const SplitSource sa = {reinterpret_cast<const char*>(job.A + (AK ? job.row0 * p.lda : job.row0)),
+                                4 * ((AK ? (p.M - 1 - job.row0) * p.lda + p.K
+                                         : (p.K - 1) * p.lda + p.M - job.row0)),
+                                AK ? 4 : p.lda * 4};
+        const SplitSource sb = {reinterpret_cast<const char*>(job.B + (BKF ? job.col0 * p.ldb : job.col0)),
+                                4 * ((BKF ? (p.N - 1 - job.col0) * p.ldb + p.K
+                                          : (p.K - 1) * p.ldb + p.N - job.col0)),
+                                BKF ? 4 : p.ldb * 4};
+        const int64_t shift = p.pair_F - BN / 2;
+        constexpr int PF = T::PF;
+        struct Regs {
+            float a[OA::ITEMS][OA::KPI], b[OB::ITEMS][OB::KPI];
+        };
+        Regs r0, r1;
+        const int64_t klen = job.kend - job.kbeg;
+        auto load = [&](Regs& r, int s) {
+            const int64_t k0 = job.kbeg + ((int64_t)(EDGE ? s : min(s, nslices - 1)) * G + g) * SK;
+            split_load<AK, EDGE, BM, NT_, false>(sa, p.lda, k0, 0, r.a);
+            split_load<BKF, EDGE, BN, NT_, PAIR>(sb, p.ldb, k0, shift, r.b);
+        };
+        auto store = [&](const Regs& r, int stage, float scale_a) {
+            split_store<AK, BM, NT_, PART>(lds + stage * STAGE, r.a, scale_a);
+            split_store<BKF, BN, NT_, PART>(lds + stage * STAGE + BM * SK, r.b, 0x1p16f);
+        };
+        auto mask = [&](Regs& r, int s) {
+            if constexpr(EDGE) {
+                const int64_t limit = klen - ((int64_t)s * G + g) * SK;
+                if(limit < SK) {
+                    split_mask<AK, BM, NT_>((int)max(limit, (int64_t)0), r.a);
+                    split_mask<BKF, BN, NT_>((int)max(limit, (int64_t)0), r.b);
+                }
+            }
+        };
+        const int fo = lr * SK + ((lh ^ (lr >> 2)) & 1) * 8;
+        auto read = [&](SplitFrag<TM, TN>& f, int stage, int part) {
+            const short* t = lds + stage * STAGE + part * PART + fo;
+#pragma unroll
+            for(int i = 0; i < TM; ++i)
+                f.a[i] = *reinterpret_cast<const bf16x8*>(t + (ar0 + i * 32) * SK);
+#pragma unroll
+            for(int j = 0; j < TN; ++j)
+                f.b[j] = *reinterpret_cast<const bf16x8*>(t + (BM + br0 + j * 32) * SK);
+        };
+        auto mma = [&](const SplitFrag<TM, TN>& x, const SplitFrag<TM, TN>& y) {
+#pragma unroll
+            for(int i = 0; i < TM; ++i)
+#pragma unroll
+                for(int j = 0; j < TN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.a[i], y.b[j], acc[i][j], 0,
+                                                                        0, 0);
+        };
+        load(r0, 0);
+        mask(r0, 0);
+        store(r0, 0, scale);
+        load(PF == 2 ? r1 : r0, 1);
+        if constexpr(PF == 2) load(r0, 2);
+        __syncthreads();
+        SplitFrag<TM, TN> f0, f1, m;
+        read(f0, 0, 0);
+        read(m, 0, 1);
+        constexpr int NB = TM * TN, RD = TM + TN;
+        constexpr int CV = (OA::ITEMS * OA::KPI + OB::ITEMS * OB::KPI) * 13 / 2;
+        constexpr int WR = 3 * (OA::ITEMS + OB::ITEMS);
+        constexpr int LD = OA::ITEMS * OA::LOADS + OB::ITEMS * OB::LOADS;
+        auto slice = [&](int s, int cur, float scale_a, Regs& r, SplitFrag<TM, TN>& h,
+                         SplitFrag<TM, TN>& q) {
+            mask(r, s + 1);
+            read(q, cur, 2);
+            store(r, cur ^ 1, scale_a);
+            load(r, s + 1 + PF);
+            mma(m, m);
+            mma(m, h);
+            mma(h, m);
+            split_sched<3 * NB, RD, CV, WR, LD>();
+            __builtin_amdgcn_sched_barrier(0);
+            __syncthreads();
+            read(m, cur ^ 1, 1);
+            mma(h, q);
+            mma(q, h);
+            split_sched<2 * NB, RD, 0, 0, 0>();
+            __builtin_amdgcn_sched_barrier(0);
+            read(q, cur ^ 1, 0);
+            mma(h, h);
+            split_sched<NB, RD, 0, 0, 0>();
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        int flip = 4;
+#pragma unroll 1
+        for(int s = 0; s < nslices; s += 2) {
+            slice(s, 0, scale, PF == 2 ? r1 : r0, f0, f1);
+            const bool turn = G == 1 && s + 2 == flip;
+            if(turn) scale = -scale;
+            slice(s + 1, 1, scale, r0, f1, f0);
+            if(turn) {
+                flip += 8;
+#pragma unroll
+                for(int i = 0; i < TM; ++i)
+#pragma unroll
+                    for(int j = 0; j < TN; ++j) acc[i][j] = -acc[i][j];
+            }
+        }
+    }
+    const float unscale = scale * 0x1p-48f;
+    if constexpr(G > 1) {
+        // the groups' sums meet in LDS: group b % G finishes block b, adding in
+        // group order
+#pragma unroll
+        for(int i = 0; i < TM; ++i)
+#pragma unroll
+            for(int j = 0; j < TN; ++j) acc[i][j] *= unscale;
+        f32x4* red = reinterpret_cast<f32x4*>(lds_all);
+        constexpr int BLK = T::WAVES * TM * TN * 4 * 64;  // f32x4 of one group's tile
+        auto slot = [&](int from, int b, int r) {
+            return ((from * T::WAVES + w) * TM * TN + b) * 4 * 64 + r * 64 + l;
+        };
+        static_assert((G - 1) * BLK * 16 <= (int)sizeof(lds_all), "partial tiles fit");
+        __syncthreads();
+#pragma unroll
+        for(int b = 0; b < TM * TN; ++b) {
+            const int owner = b % G;
+            if(g != owner) {
+                const int from = (g - owner + G) % G - 1;
+#pragma unroll
+                for(int r = 0; r < 4; ++r) {
+                    f32x16& a = acc[b / TN][b % TN];
+                    red[slot(from, b, r)] = f32x4{a[4 * r], a[4 * r + 1], a[4 * r + 2], a[4 * r + 3]};
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for(int b = 0; b < TM * TN; ++b) {
+            if(g == b % G) {
+#pragma unroll
+                for(int from = 0; from < G - 1; ++from)
+#pragma unroll
+                    for(int r = 0; r < 4; ++r) {
+                        const f32x4 x = red[slot(from, b, r)];
+#pragma unroll
+                        for(int e = 0; e < 4; ++e) acc[b / TN][b % TN][4 * r + e] += x[e];
+                    }
+            }
+        }
+    }
+    float sum = 0.0f;
+#pragma unroll
+    for(int i = 0; i < TM; ++i)
+#pragma unroll
+        for(int j = 0; j < TN; ++j)
+            if(G == 1 || g == (i * TN + j) % G)
+#pragma unroll
+            for(int r = 0; r < 16; ++r) {
+                if(G == 1) acc[i][j][r] *= unscale;
+                sum = fmaf(acc[i][j][r], 0.0f, sum);
+            }
+    if(p.exact_only || __any(sum != 0.0f))
+        exact_tile<TA, TB, PAIR, T>(p, job, acc, ar0, br0, lr, lh);
+
+    if constexpr(EPI == kEpiPlain)
+        store_tile<EDGE ? kEdgeScalar : kEdgeNone, TM, TN, G>(p, job, acc, ar0, br0, lr, lh, g);
+    else
+        staged_epilogue<EPI, T, (int)sizeof(lds_all) / 4>(p, job, acc, reinterpret_cast<float*>(lds_all),
+                                                         ar0, br0, lr, lh, g);
+}

@@ -1,0 +1,134 @@
+"""The fp32 product on the bf16 matrix cores (gemm_split.h): every operand is
+the exact sum of three bf16 parts, six of whose nine products are added.
+
+Bound of a sum over K terms: a matrix instruction of 16 k rounds its fp32
+accumulator at most 4 times, six of them per 16 k, each rounding at most
+2^-24 of the partial sums' bound sum |a||b|; the three products left out are
+below 2^-24 of |a||b| together, and the K groups and the scaling add a few
+more: |error| <= (1.5 K + 8) 2^-24 sum |a||b|.
+"""
+import numpy as np
+import pytest
+import torch
+
+from pico_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+
+
+def _gen(seed):
+    return torch.Generator(device="cuda:0").manual_seed(seed)
+
+
+def _product(ta, tb, A, B, C, **kw):
+    return K.gemm(ta, tb, A if ta == "N" else A.t().contiguous(),
+                  B if tb == "N" else B.t().contiguous(), C, **kw)
+
+
+def _within_bound(C, A, B):
+    a, b = A.double(), B.double()
+    err = (C.double() - a @ b).abs()
+    return bool((err <= (1.5 * A.shape[1] + 8) * 2.0 ** -24 * (a.abs() @ b.abs())).all())
+
+
+# whole and ragged sizes of every tile: 256 x 256, 128 x 128, 256 x 96, 128 x 96, 64 x 64; K of a
+# part of a slice, one slice, an odd number of slices, and past a sign change of the sums
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("N", "T"), ("T", "N"), ("T", "T")])
+@pytest.mark.parametrize("M,N,Kd", [(4096, 4096, 64), (4096, 4099, 200), (2048, 2048, 32),
+                                    (2047, 1985, 17), (8192, 768, 64), (8191, 768, 130),
+                                    (4096, 768, 64), (4095, 768, 49), (1024, 1024, 128),
+                                    (1023, 1021, 131), (515, 2047, 1), (700, 600, 1100)])
+def test_within_fp32_bound(dev, ta, tb, M, N, Kd):
+    g = _gen(M + N + Kd)
+    A = torch.randn(M, Kd, device=dev, generator=g)
+    B = torch.rand(Kd, N, device=dev, generator=g)
+    C = torch.full((M, N), float("nan"), device=dev)
+    _product(ta, tb, A, B, C)
+    assert _within_bound(C, A, B)
+
+
+@pytest.mark.parametrize("M,N,Kd", [(4096, 4096, 768), (2048, 2048, 2048), (8192, 768, 768)])
+def test_errors_do_not_share_a_sign(dev, M, N, Kd):
+    """the matrix unit drops bits of small products towards minus infinity; the
+    alternating sign of the sums keeps that out of the result, so the mean
+    error over M N outputs is that of independent errors (here 8 of their
+    standard errors, and a tenth of the root mean square error at most)"""
+    g = _gen(5)
+    A = torch.randn(M, Kd, device=dev, generator=g)
+    B = torch.randn(Kd, N, device=dev, generator=g)
+    C = torch.empty(M, N, device=dev)
+    K.gemm("N", "N", A, B, C)
+    e = C.double() - A.double() @ B.double()
+    rms = float(e.square().mean().sqrt())
+    cols = e.mean(0)
+    assert abs(float(e.mean())) <= 0.01 * rms
+    assert float(cols.square().mean().sqrt()) <= 2 * rms / M ** 0.5
+
+
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("T", "N")])
+def test_every_float_passes_exactly(dev, ta, tb):
+    """times the identity, any finite float (subnormal and near the largest
+    among them) comes back bit for bit: the three parts hold all 24 bits, and
+    what overflows the scaled sums is computed again on the fp32 cores"""
+    bits = torch.randint(0, 1 << 32, (600, 1040), generator=_gen(1), device=dev, dtype=torch.int64)
+    A = (bits - (1 << 31)).to(torch.int32).view(torch.float32)
+    A = torch.where(torch.isfinite(A), A, torch.ones_like(A))
+    one = torch.eye(1040, device=dev)
+    for rows in (A, torch.ldexp(A.sign(), torch.randint(-149, 128, A.shape, generator=_gen(2),
+                                                        device=dev).float())):
+        # one magnitude per row and group of columns, so the sums are single values
+        C = torch.empty(600, 1040, device=dev)
+        _product(ta, tb, rows, one, C)
+        assert torch.equal(C, rows + 0.0)
+
+
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("N", "T"), ("T", "N")])
+def test_infinities_and_nan(dev, ta, tb):
+    M, N, Kd = 1100, 700, 1500
+    g = _gen(3)
+    A = torch.randn(M, Kd, device=dev, generator=g)
+    B = torch.randn(Kd, N, device=dev, generator=g)
+    A[3, 7], A[500, 1499], A[1099, 0] = float("inf"), float("nan"), float("-inf")
+    A[200, 5] = 3e38  # rounds to an infinite bf16
+    B[7, 11] = 0.0
+    C = torch.empty(M, N, device=dev)
+    _product(ta, tb, A, B, C)
+    R = A.double() @ B.double()
+    assert torch.equal(torch.isnan(C), torch.isnan(R))
+    assert bool(torch.isnan(C[500]).all()) and bool(torch.isnan(C[3, 11]))
+    inf = torch.isinf(R) | (R.abs() > 3.4028235e38)
+    assert torch.equal(C[inf].double().sign(), R[inf].sign()) and bool(torch.isinf(C[inf]).all())
+    fine = torch.ones(M, dtype=torch.bool, device=dev)
+    fine[[3, 200, 500, 1099]] = False
+    assert _within_bound(C[fine], A[fine], B)
+
+
+def test_rows_too_far_apart_for_buffer_offsets(dev):
+    """a leading dimension above 2^21 floats: 64-bit addresses"""
+    ld, M, N, Kd = (1 << 21) + 8, 3, 5, 1500
+    big = torch.zeros(M, ld, device=dev)
+    A = big[:, :Kd]
+    A.copy_(torch.randn(M, Kd, device=dev, generator=_gen(4)))
+    B = torch.randn(Kd, N, device=dev, generator=_gen(5))
+    C = torch.empty(M, N, device=dev)
+    K.gemm("N", "N", A, B, C)
+    assert _within_bound(C, A, B)
+
+
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("T", "N"), ("N", "T")])
+def test_ragged_operands_end_where_they_end(dev, ta, tb):
+    """strided, ragged operands inside buffers of NaN: nothing outside them
+    reaches the result"""
+    M, N, Kd = 517, 1031, 1203
+    g = _gen(6)
+    A = torch.randn(M, Kd, device=dev, generator=g)
+    B = torch.randn(Kd, N, device=dev, generator=g)
+
+    def inside(x):
+        buf = torch.full((x.shape[0] + 64, x.shape[1] + 3), float("nan"), device=dev)
+        buf[:x.shape[0], :x.shape[1]] = x
+        return buf[:x.shape[0], :x.shape[1]]
+
+    C = torch.full((M, N), float("nan"), device=dev)
+    K.gemm(ta, tb, inside(A if ta == "N" else A.t()), inside(B if tb == "N" else B.t()), C)
+    assert np.isfinite(C.cpu().numpy()).all() and _within_bound(C, A, B)
