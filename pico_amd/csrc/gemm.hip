@@ -37,6 +37,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -1060,6 +1061,75 @@ int choose_splits(int64_t M, int64_t N, int64_t K, bool ta, bool fp32, int64_t* 
     return (int)((K + chunk - 1) / chunk);
 }
 
+// fp32 products (gemm_split.h): tile shape and K split together, by the
+// estimated time of the busiest CU -- its workgroups, ceil(tiles * splits / 256
+// CUs), each `per_k` per k of its range plus `fixed` for its prologue and
+// epilogue -- plus, for a split, a read of every partial plane and a write at
+// 5 TB/s and a launch.  Measured in microseconds on whole tiles (each shape
+// where it fills the CUs once: 4096^3 on 256x256, [8192, 768] K 32000 on 256x96,
+// 2048^3 on 128x128, [4096, 512] K 8192 on 128x64, [768, 768] K 8192 on 64x64),
+// fixed from the same at K 512-1024.  Over 45 shapes of a transformer step,
+// squares and ragged sizes the pick ran within 8 % of the best shape timed.
+// Examples: 4096^2 -> 256x256; [8192, 768] and [8192, 2304] -> 256x96;
+// 2048^2 -> 128x128; [4096, 512] -> 128x64; 1024^2 -> 64x64; the weight gradient
+// [768, 768] K 8192 -> 128x128 in 7 splits, [768, 2304] 256x256 in 9.
+struct SplitShape {
+    TileKind kind;
+    int bm, bn;
+    double per_k, fixed;
+};
+constexpr SplitShape kSplitShapes[] = {{kTile128, 128, 128, 0.0400, 4.0},
+                                       {kTile256, 256, 256, 0.1370, 11.0},
+                                       {kTile256x96, 256, 96, 0.0610, 6.5},
+                                       {kTile128x64, 128, 64, 0.0252, 3.5},
+                                       {kTile64, 64, 64, 0.0145, 3.0}};
+
+struct SplitPlan {
+    TileChoice tile;
+    int splits;
+    int64_t kchunk;
+};
+
+// allow_split: choose_splits has the say on whether a shape splits at all, and
+// on the scratch it may take: a split that fits pk_gemm_noalloc_f32's array
+// keeps fitting
+constexpr size_t kNoAllocScratchBytes = (size_t)128 << 20;
+
+SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int64_t batch, bool allow_all, bool ta,
+                     bool allow_split) {
+    SplitPlan best = {{kTile128, 128, 128}, 1, K};
+    double c = -1.0;
+    int64_t s_max = 1, old_chunk;
+    size_t cap = ~(size_t)0;
+    if(allow_split) {
+        const int old = choose_splits(M, N, K, ta, true, &old_chunk);
+        if(old > 1) {
+            s_max = std::min<int64_t>(64, K / (K >= 1024 ? 256 : 128));
+            if((size_t)old * M * N * sizeof(float) <= kNoAllocScratchBytes) cap = kNoAllocScratchBytes;
+        }
+    }
+    const double plane = (double)M * (double)N * 4.0 / 5e6;
+    for(const SplitShape& t : kSplitShapes) {
+        if(!allow_all && t.kind != kTile128) continue;
+        if(t.kind == kTile256x96 && N % 96 != 0) continue;
+        const int64_t tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * batch;
+        const int64_t step = 32 * split_groups(t.kind);
+        for(int64_t s = 1; s <= s_max; ++s) {
+            const int64_t chunk = s == 1 ? K : ((K + s - 1) / s + step - 1) / step * step;
+            const int64_t splits = s == 1 ? 1 : (K + chunk - 1) / chunk;
+            if(splits > 1 && (size_t)splits * M * N * sizeof(float) > cap) break;
+            const int64_t rounds = (tiles * splits + kCUs - 1) / kCUs;
+            const double ck = (double)rounds * (t.per_k * (double)chunk + t.fixed) +
+                              (splits > 1 ? (double)(splits + 1) * plane + 3.0 : 0.0);
+            if(c < 0.0 || ck < c) {
+                c = ck;
+                best = {{t.kind, t.bm, t.bn}, (int)splits, chunk};
+            }
+        }
+    }
+    return best;
+}
+
 enum Precision { kFp32 = 0, kBf16 = 1, kBf16x3 = 2, kFp8 = 3 };
 
 template <bool TA, bool TB, class T, int EDGE, int EPI>
@@ -1272,13 +1342,18 @@ int gemm_impl(char ta, char tb, int64_t M, int64_t N, int64_t K, float alpha, co
     gp.splits = 1;
     gp.kchunk = K;
     gp.ws = nullptr;
-    if(batch == 1 && causal == 0 && ws && K > 0 && !swiglu && !sfwd) {
-        int64_t kchunk;
-        const int S = choose_splits(M, N, K, TA, prec == kFp32, &kchunk);
+    const bool may_split = batch == 1 && causal == 0 && ws && K > 0 && !swiglu && !sfwd;
+    SplitPlan plan = {{kTile128, 128, 128}, 1, K};
+    if(prec == kFp32) plan = plan_split(M, N, K, batch, causal == 0, TA, may_split);
+    if(may_split) {
+        int64_t kchunk = plan.kchunk;
+        const int S = prec == kFp32 ? plan.splits : choose_splits(M, N, K, TA, false, &kchunk);
         if(S > 1 && ws_bytes >= (size_t)S * (size_t)M * (size_t)N * sizeof(float)) {
             gp.splits = S;
             gp.kchunk = kchunk;
             gp.ws = ws;
+        } else if(S > 1 && prec == kFp32) {
+            plan = plan_split(M, N, K, batch, true, TA, false);
         }
     }
     auto v4 = [](const void* q, int64_t ld) {
@@ -1295,9 +1370,9 @@ int gemm_impl(char ta, char tb, int64_t M, int64_t N, int64_t K, float alpha, co
     if(tc.bm == 0)
         return pk::fail("pk_gemm_swiglu_fwd_f32: F=%lld is not a multiple of 32 (no tile holds "
                         "whole gate/up column pairs)", (long long)gp.pair_F);
-    // fp32: the SwiGLU-forward product takes the plain product's shape (its
-    // tiles may hold partial columns), so both add K in the same order
-    if(prec == kFp32 && gp.pair_F) tc = pick_tile(M, N, batch, causal == 0);
+    // fp32: a shape for M, N and K alone (the SwiGLU-forward product's tiles may
+    // hold partial columns), so every epilogue adds K in the same order
+    if(prec == kFp32) tc = plan.tile;
     const int64_t tiles_m = (M + tc.bm - 1) / tc.bm,
                   tiles_n = gp.pair_F ? (gp.pair_F + tc.bn / 2 - 1) / (tc.bn / 2)
                                       : (N + tc.bn - 1) / tc.bn;
@@ -1375,14 +1450,18 @@ extern "C" int pk_gemm_f32(char ta, char tb, int64_t M, int64_t N, int64_t K, fl
 // the split-K partials of op(A) . op(B) for one layout of A
 static size_t gemm_workspace(int64_t M, int64_t N, int64_t K, bool ta) {
     if(M <= 0 || N <= 0 || K <= 0) return 0;
-    int64_t kchunk;
-    const int S = choose_splits(M, N, K, ta, true, &kchunk);
+    const int S = plan_split(M, N, K, 1, true, ta, true).splits;
     return S > 1 ? (size_t)S * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
-// any layout: A^T.B splits whenever another layout of the shape does
+// any layout (A^T.B splits whenever another layout of the shape does) and any
+// precision: the opt-in ones split by choose_splits alone
 extern "C" size_t pk_gemm_workspace_f32(int64_t M, int64_t N, int64_t K) {
-    return gemm_workspace(M, N, K, true);
+    if(M <= 0 || N <= 0 || K <= 0) return 0;
+    int64_t kchunk;
+    const int S = choose_splits(M, N, K, true, true, &kchunk);
+    return std::max(gemm_workspace(M, N, K, true),
+                    S > 1 ? (size_t)S * (size_t)M * (size_t)N * sizeof(float) : 0);
 }
 
 extern "C" int pk_gemm_ex_f32(char ta, char tb, int64_t M, int64_t N, int64_t K, float alpha,
@@ -1591,7 +1670,6 @@ extern "C" int pk_gemm_swiglu_fwd_f32(char ta, char tb, int64_t M, int64_t N, in
 // copy at its own address).  Calls that overlap on one GPU (two streams, two
 // threads) share that GPU's array and race.
 namespace {
-constexpr size_t kNoAllocScratchBytes = size_t(128) << 20;
 constexpr int kMaxDevices = 64;
 }  // namespace
 
@@ -1629,11 +1707,15 @@ extern "C" size_t pk_gemm_noalloc_scratch_bytes(void) { return kNoAllocScratchBy
 extern "C" int pk_gemm_noalloc_f32(char ta, char tb, int64_t M, int64_t N, int64_t K, float alpha,
                                    const float* A, int64_t lda, const float* B, int64_t ldb,
                                    float beta, float* C, int64_t ldc, pk_stream_t stream) {
-    const size_t need = gemm_workspace(M, N, K, ta == 'T' || ta == 't');
-    if(need > kNoAllocScratchBytes)
+    const bool TA = ta == 'T' || ta == 't';
+    int64_t kchunk;
+    const int S = M > 0 && N > 0 && K > 0 ? choose_splits(M, N, K, TA, true, &kchunk) : 1;
+    const size_t most = S > 1 ? (size_t)S * (size_t)M * (size_t)N * sizeof(float) : 0;
+    if(most > kNoAllocScratchBytes)
         return pk::fail("pk_gemm_noalloc_f32: this product's split-K partials need %zu bytes, "
                         "above the %zu-byte static scratch (use pk_gemm_ex_f32 with a workspace)",
-                        need, kNoAllocScratchBytes);
+                        most, kNoAllocScratchBytes);
+    const size_t need = gemm_workspace(M, N, K, TA);
     float* ws = nullptr;
     if(need > 0 && !(ws = scratch_on_current_device())) return PK_EINVAL;
     // every partial-plane element the reduction reads is written by its split

@@ -293,7 +293,8 @@ __device__ __forceinline__ void staged_epilogue(const GemmParams& p, const TileJ
     }
 }
 
-enum TileKind { kTile128, kTile96, kTile256, kTile64, kTile256x96 };
+// (128x96 tiles: the opt-in precisions' kernels only; 128x64: fp32 only)
+enum TileKind { kTile128, kTile96, kTile256, kTile64, kTile256x96, kTile128x64 };
 
 
 // the fp32 product (gemm_split.hip): K groups a shape's workgroups split K into,

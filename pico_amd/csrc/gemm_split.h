@@ -46,11 +46,11 @@
 //  * Loads go through buffer resources that end where the operand ends, 128 bits
 //    at any 4-byte alignment, so ragged sizes take the same path: what lies
 //    behind the end reads as zero, and only a partial last slice is masked.
-//    (The per-element edge path this replaces: 2000x1503x1001 at 58 TFLOP/s,
-//    now 105.)
+//    (The per-element edge path this replaces ran 2000x1503x1001, forward and
+//    backward, at 59 TFLOP/s; now 130.)
 //
 // 4096^3 A.B / A.B^T / A^T.B 244-246 TFLOP/s (149 on the fp32 cores), 8192^3
-// 237-243 (151), 2048^3 186-189 (142).
+// 237-243 (151), 2048^3 188-193 (142), 1024^3 114-117 (105-115).
 
 // A tile shape: WM x WN waves, each TM x TN blocks of 32 x 32; WPS waves per SIMD.
 template <int WM_, int WN_, int TM_, int TN_, int G_, int WPS_, int PF_>
@@ -322,9 +322,10 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmPara
         auto mask = [&](Regs& r, int s) {
             if constexpr(EDGE) {
                 const int64_t limit = klen - ((int64_t)s * G + g) * SK;
-                if(limit < SK) {
-                    split_mask<AK, BM, NT_>((int)max(limit, (int64_t)0), r.a);
-                    split_mask<BKF, BN, NT_>((int)max(limit, (int64_t)0), r.b);
+                // (k rows of a row-contiguous operand past K lie behind its end)
+                if((AK || BKF) && limit < SK) {
+                    if(AK) split_mask<AK, BM, NT_>((int)max(limit, (int64_t)0), r.a);
+                    if(BKF) split_mask<BKF, BN, NT_>((int)max(limit, (int64_t)0), r.b);
                 }
             }
         };

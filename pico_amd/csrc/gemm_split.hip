@@ -9,9 +9,9 @@ using namespace pkg;
 
 // the fp32 products' shapes of the same names (gemm_split.h)
 using Split256 = SplitTile<2, 4, 4, 2, 1, 2, 1>;
-using Split128 = SplitTile<2, 4, 2, 1, 1, 4, 1>;
+using Split128 = SplitTile<2, 4, 2, 1, 2, 4, 1>;
 using Split256x96 = SplitTile<4, 1, 2, 3, 2, 2, 1>;
-using Split96 = SplitTile<4, 1, 1, 3, 2, 2, 1>;
+using Split128x64 = SplitTile<2, 2, 2, 1, 2, 4, 1>;
 using Split64 = SplitTile<2, 2, 1, 1, 4, 4, 2>;
 
 template <bool TA, bool TB, bool EDGE, class T>
@@ -50,7 +50,7 @@ int launch_layout(const GemmParams& gp, int64_t batch, bool edge, TileKind kind,
     switch(kind) {
     case kTile256: return launch_split_tile<TA, TB, Split256>(gp, batch, edge, st);
     case kTile256x96: return launch_split_tile<TA, TB, Split256x96>(gp, batch, edge, st);
-    case kTile96: return launch_split_tile<TA, TB, Split96>(gp, batch, edge, st);
+    case kTile128x64: return launch_split_tile<TA, TB, Split128x64>(gp, batch, edge, st);
     case kTile64: return launch_split_tile<TA, TB, Split64>(gp, batch, edge, st);
     default: return launch_split_tile<TA, TB, Split128>(gp, batch, edge, st);
     }
@@ -61,7 +61,7 @@ int launch_layout(const GemmParams& gp, int64_t batch, bool edge, TileKind kind,
 namespace pkg {
 
 int split_groups(TileKind kind) {
-    return kind == kTile64 ? Split64::G : kind == kTile96 || kind == kTile256x96 ? 2 : 1;
+    return kind == kTile64 ? Split64::G : kind == kTile256 ? Split256::G : 2;
 }
 
 int launch_split(bool ta, bool tb, const GemmParams& gp, int64_t batch, bool edge, TileKind kind,
