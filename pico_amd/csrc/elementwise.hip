@@ -9,6 +9,8 @@
 // reference's CPU results.
 #include <math.h>
 
+#include <algorithm>
+
 #include "pk_common.h"
 
 #pragma clang fp contract(off)
@@ -57,6 +59,72 @@ __global__ void binary_same4(int op, int64_t n4, const f32x4* __restrict__ a,
         r[3] = bin_apply(op, x[3], y[3]);
         out[i] = r;
     }
+}
+
+// Two-dimensional broadcasts: out is [R, C] contiguous, and an operand's element
+// (r, c) is at r * sr + c * sc with sc 0 or 1 (a bias row, a column of row
+// factors, a scalar, a padded matrix).  `tx` threads (a power of two) walk a
+// row's columns in units of W, NT / tx rows at a time, so no index is divided;
+// binary_general spends two 64-bit divisions per dim and element ([4096, 2048]
+// with a [2048] row: 25 us, here 14).
+struct Plane {
+    const float* p;
+    int64_t sr;
+    int sc;
+};
+
+template <int W>
+__device__ __forceinline__ f32x4 plane_load(const Plane& a, int64_t r, int64_t c) {
+    const float* q = a.p + r * a.sr;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if(a.sc == 0) {
+        v[0] = v[1] = v[2] = v[3] = *q;
+    } else if(W == 4) {
+        v = *reinterpret_cast<const f32x4*>(q + c);
+    } else {
+        v[0] = q[c];
+    }
+    return v;
+}
+
+template <int W>
+__global__ void binary_plane(int op, int64_t R, int64_t C, int tx, Plane a, Plane b,
+                             float* __restrict__ out) {
+    const int ty = NT / tx, x = threadIdx.x & (tx - 1), y = threadIdx.x / tx;
+    for(int64_t r = (int64_t)blockIdx.y * ty + y; r < R; r += (int64_t)gridDim.y * ty)
+        for(int64_t c = ((int64_t)blockIdx.x * tx + x) * W; c < C; c += (int64_t)gridDim.x * tx * W) {
+            const f32x4 u = plane_load<W>(a, r, c), v = plane_load<W>(b, r, c);
+            if(W == 4) {
+                f32x4 w;
+#pragma unroll
+                for(int e = 0; e < 4; ++e) w[e] = bin_apply(op, u[e], v[e]);
+                *reinterpret_cast<f32x4*>(out + r * C + c) = w;
+            } else {
+                out[r * C + c] = bin_apply(op, u[0], v[0]);
+            }
+        }
+}
+
+// mul's gradient of an operand that has the output's shape and layout, the other
+// operand broadcast: gx (+)= g * other
+template <int W>
+__global__ void mul_bwd_plane(int64_t R, int64_t C, int tx, const float* __restrict__ g, Plane other,
+                              float* __restrict__ gx, int accum) {
+    const int ty = NT / tx, x = threadIdx.x & (tx - 1), y = threadIdx.x / tx;
+    for(int64_t r = (int64_t)blockIdx.y * ty + y; r < R; r += (int64_t)gridDim.y * ty)
+        for(int64_t c = ((int64_t)blockIdx.x * tx + x) * W; c < C; c += (int64_t)gridDim.x * tx * W) {
+            const f32x4 o = plane_load<W>(other, r, c);
+            float* q = gx + r * C + c;
+            if(W == 4) {
+                const f32x4 gv = *reinterpret_cast<const f32x4*>(g + r * C + c);
+                f32x4 acc = accum ? *reinterpret_cast<f32x4*>(q) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for(int e = 0; e < 4; ++e) acc[e] = acc[e] + gv[e] * o[e];
+                *reinterpret_cast<f32x4*>(q) = acc;
+            } else {
+                *q = (accum ? *q : 0.0f) + g[r * C + c] * o[0];
+            }
+        }
 }
 
 // Gradient of one operand x.  The output dims split into "kept" dims (x has
@@ -148,6 +216,146 @@ __global__ void binary_bwd_rows(int op, int which, int64_t R, int64_t C,
     }
 }
 
+// The reductions of a broadcast operand's gradient, one running sum per element
+// of x as pico adds them (term r after term r - 1), but with the memory traffic
+// off the adds' chain: a workgroup owns JB elements, its 256 threads fetch
+// chunks of terms into LDS two chunks ahead, and the JB lanes of wave 0 add
+// them, four terms per LDS read.
+//   term(j, r) = g[j * gj + r * gr] (* other[j * oj + r * orr] for mul)
+// with gj == 1 (x broadcast over leading dims: a bias) or gr == 1 (over trailing
+// ones: a row factor).  binary_bwd_rows keeps one thread's loads eight ahead
+// of its adds, which leaves 2048 columns to 32 waves: a [4096, 2048] bias
+// gradient 142 us (mul 257), here 31 (44); binary_bwd_reduce divides indexes per
+// term and reads a row per thread: a [4096, 1] factor's 598 us (1032), here 13 (21).
+// Terms past the end are -0, which changes no sum.
+struct OrderedSum {
+    const float *g, *other;
+    float* gx;
+    int64_t J, Rn, gj, gr, oj, orr, xj;
+    int negate, accum, vec;
+};
+
+constexpr int kOsQuads = 4;  // float4 of terms per thread and chunk
+
+template <int JB, int kOsThreads, bool COLS, bool MUL>
+__global__ __launch_bounds__(kOsThreads) void ordered_sum_kernel(OrderedSum p) {
+    constexpr int TR = kOsThreads * kOsQuads * 4 / JB;  // terms per chunk
+    constexpr int LD = TR + 4;                          // 16 bytes off per lane: no bank conflicts
+    __shared__ __attribute__((aligned(16))) float lds[2][JB * LD];
+    const int64_t j0 = (int64_t)blockIdx.x * JB;
+    const int jn = (int)min((int64_t)JB, p.J - j0);
+    const int64_t chunks = (p.Rn + TR - 1) / TR;
+    auto place = [&](int q, int& j, int& r) {
+        const int u = threadIdx.x + q * kOsThreads;
+        if(COLS) {
+            j = u % JB;
+            r = u / JB * 4;
+        } else {
+            j = u / (TR / 4);
+            r = u % (TR / 4) * 4;
+        }
+    };
+    auto load4 = [&](const float* base, int64_t sj, int64_t sr, int64_t j, int64_t r) {
+        f32x4 v = {-0.f, -0.f, -0.f, -0.f};
+        const float* q = base + j * sj + r * sr;
+        if(!COLS && sr == 1 && p.vec && r + 3 < p.Rn) return *reinterpret_cast<const f32x4*>(q);
+#pragma unroll
+        for(int e = 0; e < 4; ++e)
+            if(r + e < p.Rn) v[e] = q[e * sr];
+        return v;
+    };
+    f32x4 ga[kOsQuads], gb[kOsQuads], oa[MUL ? kOsQuads : 1], ob[MUL ? kOsQuads : 1];
+    auto fetch = [&](f32x4 (&g)[kOsQuads], f32x4 (&o)[MUL ? kOsQuads : 1], int64_t c) {
+#pragma unroll
+        for(int q = 0; q < kOsQuads; ++q) {
+            int j, r;
+            place(q, j, r);
+            const int64_t rr = c * TR + r;
+            g[q] = f32x4{-0.f, -0.f, -0.f, -0.f};
+            if(MUL) o[q] = f32x4{1.f, 1.f, 1.f, 1.f};
+            if(j < jn && rr < p.Rn) {
+                g[q] = load4(p.g, p.gj, p.gr, j0 + j, rr);
+                if(MUL) o[q] = load4(p.other, p.oj, p.orr, j0 + j, rr);
+            }
+        }
+    };
+    auto put = [&](const f32x4 (&g)[kOsQuads], const f32x4 (&o)[MUL ? kOsQuads : 1], int64_t c) {
+        float* t = lds[c & 1];
+#pragma unroll
+        for(int q = 0; q < kOsQuads; ++q) {
+            int j, r;
+            place(q, j, r);
+            f32x4 v;
+#pragma unroll
+            for(int e = 0; e < 4; ++e) {
+                float x = g[q][e];
+                if(MUL) x = c * TR + r + e < p.Rn ? x * o[q][e] : -0.0f;
+                else if(p.negate) x = c * TR + r + e < p.Rn ? -x : -0.0f;
+                v[e] = x;
+            }
+            *reinterpret_cast<f32x4*>(t + j * LD + r) = v;
+        }
+    };
+    const int lane = threadIdx.x;
+    float acc = 0.0f;
+    if(p.accum && lane < jn) acc = p.gx[(j0 + lane) * p.xj];
+    fetch(ga, oa, 0);
+    fetch(gb, ob, 1);
+    put(ga, oa, 0);
+    __syncthreads();
+    auto step = [&](int64_t c, f32x4 (&g0)[kOsQuads], f32x4 (&o0)[MUL ? kOsQuads : 1],
+                    f32x4 (&g1)[kOsQuads], f32x4 (&o1)[MUL ? kOsQuads : 1]) {
+        fetch(g0, o0, c + 2);
+        if(lane < jn) {
+            const float* t = lds[c & 1] + lane * LD;
+            // eight reads ahead of the adds
+            f32x4 v[8], n[8];
+#pragma unroll
+            for(int e = 0; e < 8; ++e) v[e] = *reinterpret_cast<const f32x4*>(t + 4 * e);
+#pragma unroll 1
+            for(int r = 32; r <= TR; r += 32) {
+                const int rn = r < TR ? r : 0;
+#pragma unroll
+                for(int e = 0; e < 8; ++e) n[e] = *reinterpret_cast<const f32x4*>(t + rn + 4 * e);
+#pragma unroll
+                for(int e = 0; e < 8; ++e) {
+                    acc += v[e][0];
+                    acc += v[e][1];
+                    acc += v[e][2];
+                    acc += v[e][3];
+                }
+#pragma unroll
+                for(int e = 0; e < 8; ++e) v[e] = n[e];
+            }
+        }
+        put(g1, o1, c + 1);
+        __syncthreads();
+    };
+    for(int64_t c = 0; c < chunks; c += 2) {
+        step(c, ga, oa, gb, ob);
+        if(c + 1 < chunks) step(c + 1, gb, ob, ga, oa);
+    }
+    if(lane < jn) p.gx[(j0 + lane) * p.xj] = acc;
+}
+
+// fewest terms and most columns that take the ordered sums
+constexpr int64_t kOrderedMin = 32, kOrderedMost = 8192;
+
+template <bool COLS, bool MUL>
+void launch_ordered_sum(const OrderedSum& p, hipStream_t st) {
+    // 16 elements per workgroup until that gives every CU two workgroups; while it
+    // gives every CU one at most, long sums take chunks four times as long, so
+    // fewer barriers cut their chain ([4096, 2048] 57 -> 31 us; 512 workgroups
+    // of [8192, 4096] row factors are faster with short chunks, 35 against 52)
+    const unsigned g16 = (unsigned)((p.J + 15) / 16), g64 = (unsigned)((p.J + 63) / 64);
+    if(p.J <= 16 * 256 && p.Rn > 512)
+        ordered_sum_kernel<16, 1024, COLS, MUL><<<g16, 1024, 0, st>>>(p);
+    else if(p.J <= 16 * 512)
+        ordered_sum_kernel<16, 256, COLS, MUL><<<g16, 256, 0, st>>>(p);
+    else
+        ordered_sum_kernel<64, 256, COLS, MUL><<<g64, 256, 0, st>>>(p);
+}
+
 // ---------------------------------------------------------------- unary
 __device__ __forceinline__ float un_apply(int op, float x) {
     switch(op) {
@@ -180,12 +388,17 @@ __global__ void unary_kernel(int op, int64_t n, const float* __restrict__ x, flo
         y[i] = un_apply(op, x[i]);
 }
 
+// sqrt and tanh read y only, the others x only
 __global__ void unary_bwd_kernel(int op, int64_t n, const float* __restrict__ x,
                                  const float* __restrict__ y, const float* __restrict__ gy,
                                  float* __restrict__ gx, int accum) {
+    const bool use_y = op == 0 || op == 4;
+    const float* __restrict__ s = use_y ? y : x;
     for(int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-        i += (int64_t)gridDim.x * blockDim.x)
-        gx[i] = un_bwd(op, accum ? gx[i] : 0.0f, x[i], y[i], gy[i]);
+        i += (int64_t)gridDim.x * blockDim.x) {
+        const float v = s[i];
+        gx[i] = un_bwd(op, accum ? gx[i] : 0.0f, v, v, gy[i]);
+    }
 }
 
 // ------------------------------------------------------------------ relu
@@ -596,6 +809,89 @@ bool valid_op(int op, int hi) { return op >= 0 && op <= hi; }
 
 // ======================================================================= C-ABI
 
+namespace {
+
+// [R, C] of a broadcast's dims: those of size 1 dropped, neighbours that every
+// operand steps through alike joined.  False when more than two are left.
+struct PlaneDims {
+    int64_t R, C;
+    int64_t sr[2], sc[2];
+};
+bool plane_dims(int ndim, const int64_t* shape, const int64_t* s0, const int64_t* s1, PlaneDims& d) {
+    int64_t sh[2], st[2][2];
+    int n = 0;
+    for(int k = 0; k < ndim; ++k) {
+        if(shape[k] == 1) continue;
+        const int64_t v[2] = {s0[k], s1[k]};
+        if(n && st[n - 1][0] == v[0] * shape[k] && st[n - 1][1] == v[1] * shape[k]) {
+            sh[n - 1] *= shape[k];
+        } else {
+            if(n == 2) return false;
+            sh[n++] = shape[k];
+        }
+        st[n - 1][0] = v[0];
+        st[n - 1][1] = v[1];
+    }
+    d.C = n ? sh[n - 1] : 1;
+    d.R = n == 2 ? sh[0] : 1;
+    for(int o = 0; o < 2; ++o) {
+        d.sc[o] = n ? st[n - 1][o] : 0;
+        d.sr[o] = n == 2 ? st[0][o] : 0;
+        if(d.sc[o] != 0 && d.sc[o] != 1) return false;
+    }
+    return true;
+}
+
+struct PlaneGrid {
+    dim3 grid;
+    int tx;
+};
+PlaneGrid plane_grid(int64_t R, int64_t C, int W) {
+    const int64_t units = (C + W - 1) / W;
+    int tx = 1;
+    while(tx < NT && tx < units) tx *= 2;
+    const int64_t gx = std::min<int64_t>((units + tx - 1) / tx, 64);
+    const int64_t rows = (R + NT / tx - 1) / (NT / tx);
+    return {dim3((unsigned)gx, (unsigned)std::max<int64_t>(1, std::min<int64_t>(rows, 4096 / gx))), tx};
+}
+
+bool plane_vec(const Plane& a) { return a.sc == 0 || (pk::aligned16(a.p) && a.sr % 4 == 0); }
+
+bool launch_binary_plane(int op, const Strides& s, const float* a, const float* b, float* out,
+                         hipStream_t st) {
+    PlaneDims d;
+    if(!plane_dims(s.ndim, s.shape, s.sa, s.sb, d)) return false;
+    const Plane pa = {a, d.sr[0], (int)d.sc[0]}, pb = {b, d.sr[1], (int)d.sc[1]};
+    if(d.C % 4 == 0 && pk::aligned16(out) && plane_vec(pa) && plane_vec(pb)) {
+        const PlaneGrid g = plane_grid(d.R, d.C, 4);
+        binary_plane<4><<<g.grid, NT, 0, st>>>(op, d.R, d.C, g.tx, pa, pb, out);
+    } else {
+        const PlaneGrid g = plane_grid(d.R, d.C, 1);
+        binary_plane<1><<<g.grid, NT, 0, st>>>(op, d.R, d.C, g.tx, pa, pb, out);
+    }
+    return true;
+}
+
+// neighbouring dims that the output, the other operand and x step through alike
+// become one
+int merge_dims(int n, int64_t* shape, int64_t* a, int64_t* b, int64_t* c) {
+    int m = 0;
+    for(int k = 0; k < n; ++k) {
+        if(m && a[m - 1] == a[k] * shape[k] && b[m - 1] == b[k] * shape[k] &&
+           (!c || c[m - 1] == c[k] * shape[k])) {
+            shape[m - 1] *= shape[k];
+        } else {
+            shape[m++] = shape[k];
+        }
+        a[m - 1] = a[k];
+        b[m - 1] = b[k];
+        if(c) c[m - 1] = c[k];
+    }
+    return m;
+}
+
+}  // namespace
+
 extern "C" int pk_binary_f32(int op, int ndim, const int64_t* out_shape, const int64_t* a_strides,
                              const int64_t* b_strides, const float* a, const float* b, float* out,
                              pk_stream_t stream) {
@@ -622,7 +918,7 @@ extern "C" int pk_binary_f32(int op, int ndim, const int64_t* out_shape, const i
     if(same && n % 4 == 0 && pk::aligned16(a) && pk::aligned16(b) && pk::aligned16(out))
         binary_same4<<<pk::grid_for(n / 4, NT), NT, 0, st>>>(
             op, n / 4, (const f32x4*)a, (const f32x4*)b, (f32x4*)out);
-    else
+    else if(!launch_binary_plane(op, s, a, b, out, st))
         binary_general<<<pk::grid_for(n, NT), NT, 0, st>>>(op, s, n, a, b, out);
     return pk::launch_status("pk_binary_f32");
 }
@@ -684,9 +980,51 @@ extern "C" int pk_binary_bwd_f32(int op, int which, int ndim, const int64_t* out
             op, which, x_numel / 4, (const f32x4*)gout, (const f32x4*)other, (f32x4*)gx, accum);
         return pk::launch_status("pk_binary_bwd_f32");
     }
+    // a long reduction over one run of dims, x's elements another: ordered sums
+    // (columns up to 8192: [4096, 4096] 64 us against 420 with a thread a column,
+    // mul 114 against 517; [4096, 20000] 287 against 349, but mul 529 against 399.
+    // Fewer than 32 terms are a launch's time either way)
+    if(d.nr > 0 && d.red_numel >= kOrderedMin) {
+        OrderedSum p = {gout, other, gx, 1, d.red_numel, 0, 0, 0, 0, 0, op == 1 && which == 1, accum, 0};
+        BwdDesc m = d;
+        m.nk = merge_dims(d.nk, m.kshape, m.kout, m.koth, m.kx);
+        m.nr = merge_dims(d.nr, m.rshape, m.rout, m.roth, nullptr);
+        if(m.nk <= 1 && m.nr == 1) {
+            p.gr = m.rout[0];
+            p.orr = m.roth[0];
+            if(m.nk) {
+                p.J = m.kshape[0];
+                p.gj = m.kout[0];
+                p.oj = m.koth[0];
+                p.xj = m.kx[0];
+            }
+            const bool cols = p.gr != 1;
+            p.vec = !cols && pk::aligned16(gout) && p.gj % 4 == 0 &&
+                    (op != 2 || (pk::aligned16(other) && p.oj % 4 == 0));
+            if(p.J <= kOrderedMost || !cols) {
+                if(cols) op == 2 ? launch_ordered_sum<true, true>(p, st) : launch_ordered_sum<true, false>(p, st);
+                else op == 2 ? launch_ordered_sum<false, true>(p, st) : launch_ordered_sum<false, false>(p, st);
+                return pk::launch_status("pk_binary_bwd_f32");
+            }
+        }
+    }
     if(kept_like_out && reduced_first) {  // R = 1 when nothing is reduced
         binary_bwd_rows<<<pk::grid_for(x_numel, NT), NT, 0, st>>>(op, which, d.red_numel, x_numel,
                                                                   gout, other, gx, accum);
+        return pk::launch_status("pk_binary_bwd_f32");
+    }
+    PlaneDims pd;
+    if(op == 2 && d.nr == 0 && plane_dims(ndim, out_shape, other_strides, x_strides, pd) &&
+       pd.sc[1] == 1 && (pd.R == 1 || pd.sr[1] == pd.C)) {
+        // x laid out like the output, the other operand broadcast
+        const Plane po = {other, pd.sr[0], (int)pd.sc[0]};
+        if(pd.C % 4 == 0 && pk::aligned16(gout) && pk::aligned16(gx) && plane_vec(po)) {
+            const PlaneGrid g = plane_grid(pd.R, pd.C, 4);
+            mul_bwd_plane<4><<<g.grid, NT, 0, st>>>(pd.R, pd.C, g.tx, gout, po, gx, accum);
+        } else {
+            const PlaneGrid g = plane_grid(pd.R, pd.C, 1);
+            mul_bwd_plane<1><<<g.grid, NT, 0, st>>>(pd.R, pd.C, g.tx, gout, po, gx, accum);
+        }
         return pk::launch_status("pk_binary_bwd_f32");
     }
     binary_bwd_reduce<<<pk::grid_for(x_numel, NT), NT, 0, st>>>(op, which, d, x_numel, gout,
