@@ -494,6 +494,21 @@ int pk_attn_causal_bwd_f32(int64_t B, int64_t H, int64_t T, int64_t hd, int64_t 
                            float scale, const float* q, const float* k, const float* v,
                            const float* P, const float* dout, float* dq, float* dk, float* dv,
                            float* dP_ws, int flags, pk_stream_t stream);
+/* Fused causal attention for head sizes 32, 96 and 128 (any T), fp32 products:
+ * the layouts, alignments, lse, write order and accumulate flags of the head-size-64
+ * functions below.  pk_flash_wide_supported(T, hd) says whether these apply; the
+ * backward needs pk_flash_wide_bwd_workspace(B, H, T) bytes (row constants, and
+ * dS tiles of about 2*B*H*T^2 bytes). */
+int pk_flash_wide_supported(int64_t T, int64_t hd);
+size_t pk_flash_wide_bwd_workspace(int64_t B, int64_t H, int64_t T);
+int pk_flash_wide_fwd_f32(int64_t B, int64_t H, int64_t T, int64_t hd, int64_t ld, float scale,
+                          const float* q, const float* k, const float* v, float* o, float* lse,
+                          pk_stream_t stream);
+int pk_flash_wide_bwd_f32(int64_t B, int64_t H, int64_t T, int64_t hd, int64_t ld, float scale,
+                          const float* q, const float* k, const float* v, const float* o,
+                          const float* lse, const float* dout, float* dq, float* dk, float* dv,
+                          void* workspace, size_t workspace_bytes, int flags, pk_stream_t stream);
+
 /* Fused causal attention for head size 64 (any T): the scores
  * are never written to memory.  Same layouts and lse as above; q, k, v, o,
  * dout, dq, dk, dv 16-byte aligned and ld a multiple of 4.

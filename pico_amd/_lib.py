@@ -122,6 +122,11 @@ PK_SIGNATURES = {
                                c_p, c_p],
     "pk_attn_causal_bwd_f32": [c_i64, c_i64, c_i64, c_i64, c_i64, c_f, c_p, c_p, c_p, c_p, c_p,
                                c_p, c_p, c_p, c_p, c_int, c_p],
+    "pk_flash_wide_supported": [c_i64, c_i64],
+    "pk_flash_wide_bwd_workspace": [c_i64, c_i64, c_i64],
+    "pk_flash_wide_fwd_f32": [c_i64, c_i64, c_i64, c_i64, c_i64, c_f, c_p, c_p, c_p, c_p, c_p, c_p],
+    "pk_flash_wide_bwd_f32": [c_i64, c_i64, c_i64, c_i64, c_i64, c_f, c_p, c_p, c_p, c_p, c_p, c_p,
+                              c_p, c_p, c_p, c_p, c_size, c_int, c_p],
     "pk_flash_attn_supported": [c_i64, c_i64],
     "pk_flash_attn_fwd_f32": [c_i64, c_i64, c_i64, c_i64, c_i64, c_f, c_p, c_p, c_p, c_p, c_p,
                               c_p],
@@ -151,6 +156,7 @@ PK_SIGNATURES = {
 _RESTYPES = {"pk_last_error": ctypes.c_char_p, "pk_rmsnorm_bwd_workspace": c_size,
              "pk_gemm_workspace_f32": c_size, "pk_flash_attn_bwd_workspace": c_size,
              "pk_flash_attn_bwd_workspace_recompute": c_size,
+             "pk_flash_wide_bwd_workspace": c_size,
              "pk_embed_bwd_workspace": c_size, "pk_gemm_noalloc_scratch_bytes": c_size,
              "pk_fp8_quantized_bytes": c_size, "pk_mx8_bytes": c_size,
              "pk_gemm_mx8_workspace": c_size, "pk_bf16q_bytes": c_size,

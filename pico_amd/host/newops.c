@@ -262,9 +262,10 @@ struct PicoTensor* pico_swiglu(struct PicoTensor* a, struct PicoTensor* u) {
  * of each head's causal triangle in a workspace of about 2*B*H*T^2 bytes.  Above
  * attn_ds_cap() bytes of tiles the fp32 backward recomputes dQ's scores
  * instead (PK_FLASH_RECOMPUTE: a workspace of 8*B*H*T bytes, the same
- * results).  Otherwise the chain of
- * batched GEMMs and causal-softmax kernels runs and saves the probabilities
- * P [B*H, T, T] (arena device memory). */
+ * results).  Head sizes 32, 96 and 128 run the fused kernels of their own
+ * (pk_flash_wide_*, fp32) while their dS tiles fit that cap.  Otherwise the
+ * chain of batched GEMMs and causal-softmax kernels runs and saves the
+ * probabilities P [B*H, T, T] (arena device memory). */
 enum { AS_LSE = 0, AS_P = 1 };
 /* largest dS-tile workspace the fused backward takes: 4 GiB (B*H*T^2 up to
  * about 2^31; 8 x 12 heads at T 8192 recompute), or PICO_ATTN_DS_CAP bytes
@@ -281,6 +282,8 @@ static size_t attn_ds_cap(void) {
 /* AI_PREC: the products' precision, 0 fp32, 1 bf16, 2 fp8 (flash only); an
  * fp8 node keeps max|q|, max|k|, max|v| for the backward in saved[AS_P] */
 enum { AI_B = 0, AI_H = 1, AI_FLASH = 2, AI_PREC = 3 };
+/* AI_FLASH */
+enum { ATTN_CHAIN = 0, ATTN_FLASH = 1, ATTN_WIDE = 2 };
 enum { ATTN_F32 = 0, ATTN_BF16 = 1, ATTN_FP8 = 2, ATTN_BF16X3 = 3 };
 
 static void attn_backward(struct PicoTensor* self) {
@@ -291,9 +294,11 @@ static void attn_backward(struct PicoTensor* self) {
     int64_t B = n->ival[AI_B], H = n->ival[AI_H];
     int64_t T = q->shape[0] / B, hd = q->shape[1] / H, ld = q->strides[0];
     const int flash = (int)n->ival[AI_FLASH], prec = flash ? (int)n->ival[AI_PREC] : ATTN_F32;
-    size_t ws_bytes = flash ? pk_flash_attn_bwd_workspace(B, H, T)
-                            : sizeof(float) * (size_t)(B * H * T * T);
-    const int recompute = flash && prec == ATTN_F32 && ws_bytes > attn_ds_cap();
+    const int wide = flash == ATTN_WIDE;
+    size_t ws_bytes = wide    ? pk_flash_wide_bwd_workspace(B, H, T)
+                      : flash ? pk_flash_attn_bwd_workspace(B, H, T)
+                              : sizeof(float) * (size_t)(B * H * T * T);
+    const int recompute = flash && !wide && prec == ATTN_F32 && ws_bytes > attn_ds_cap();
     if(recompute) ws_bytes = pk_flash_attn_bwd_workspace_recompute(B, H, T);
     void* ws = pkh_workspace(ws_bytes);
     if(!ws) {
@@ -319,6 +324,10 @@ static void attn_backward(struct PicoTensor* self) {
                                        self->data, (const float*)n->saved[AS_LSE], dout, q->grad,
                                        k->grad, v->grad, (float*)n->saved[AS_P], ws, ws_bytes,
                                        flags, pkh_stream());
+    else if(wide)
+        st = pk_flash_wide_bwd_f32(B, H, T, hd, ld, n->fval[0], q->data, k->data, v->data,
+                                   self->data, (const float*)n->saved[AS_LSE], dout, q->grad,
+                                   k->grad, v->grad, ws, ws_bytes, flags, pkh_stream());
     else if(flash)
         st = (prec == ATTN_BF16     ? pk_flash_attn_bwd_bf16_f32
               : prec == ATTN_BF16X3 ? pk_flash_attn_bwd_bf16x3_f32
@@ -331,6 +340,24 @@ static void attn_backward(struct PicoTensor* self) {
                                     (const float*)n->saved[AS_P], dout, q->grad, k->grad, v->grad,
                                     (float*)ws, flags, pkh_stream());
     pkh_status("pico_attention_causal_backward", st);
+}
+
+/* the fused kernels of head sizes 32, 96 and 128: 16-byte aligned tensors, a
+ * sequence within 32-bit byte offsets, and a dS workspace within the cap (the
+ * chain's probabilities and scratch would take four times that).  Few long
+ * rows of 128 dims run faster as a chain, whose products spread over the chip
+ * (forward + backward, us, fused against chain: 192 blocks of 64 rows at T 2048
+ * 549 / 438, 128 at T 1024 279 / 221, 256 at T 1024 288 / 275, 264 at T 700
+ * 209 / 208, 512 at T 1000 347 / 457; T 128 55 / 59); 32 and 96 dims gain at
+ * every size timed, from one head of T 2048 (179 / 308) up */
+static int wide_applies(struct PicoTensor* const* xs, int64_t B, int64_t H, int64_t T, int64_t hd) {
+    if(!pk_flash_wide_supported(T, hd)) return 0;
+    if(hd == 128 && T > 128 && B * H * ((T + 63) / 64) < 384) return 0;
+    for(int i = 0; i < 3; i++)
+        if(((uintptr_t)xs[i]->data | (uintptr_t)xs[i]->grad) & 15) return 0;
+    const int64_t ld = xs[0]->strides[0];
+    return (T + 64) * ld * 4 <= INT32_MAX && B * H * ((T + 31) / 32) <= INT32_MAX &&
+           pk_flash_wide_bwd_workspace(B, H, T) <= attn_ds_cap();
 }
 
 struct PicoTensor* pico_attention_causal(struct PicoTensor* q, struct PicoTensor* k,
@@ -358,11 +385,13 @@ struct PicoTensor* pico_attention_causal(struct PicoTensor* q, struct PicoTensor
     struct PicoTensor* out = pkh_new_tensor(arena, q->shape, 2);
     if(!out) return NULL;
     struct PkNode* n = pkh_node(out);
-    const int flash = pk_flash_attn_supported(T, hd);
+    const int flash = pk_flash_attn_supported(T, hd) ? ATTN_FLASH
+                      : wide_applies(xs, B, H, T, hd) ? ATTN_WIDE
+                                                      : ATTN_CHAIN;
     /* the matmul precision switch covers attention's products too; the
      * backward uses the precision the forward ran in */
     const int mp = pico_get_matmul_precision();
-    const int prec = !flash                     ? ATTN_F32
+    const int prec = flash != ATTN_FLASH        ? ATTN_F32
                      : mp == PICO_MATMUL_FP8    ? ATTN_FP8
                      : mp == PICO_MATMUL_BF16   ? ATTN_BF16
                      : mp == PICO_MATMUL_BF16X3 ? ATTN_BF16X3
@@ -384,6 +413,9 @@ struct PicoTensor* pico_attention_causal(struct PicoTensor* q, struct PicoTensor
     if(prec == ATTN_FP8)
         st = pk_flash_attn_fwd_fp8_f32(B, H, T, hd, ld, n->fval[0], q->data, k->data, v->data,
                                        out->data, lse, P, pkh_stream());
+    else if(flash == ATTN_WIDE)
+        st = pk_flash_wide_fwd_f32(B, H, T, hd, ld, n->fval[0], q->data, k->data, v->data,
+                                   out->data, lse, pkh_stream());
     else if(flash)
         st = (prec == ATTN_BF16     ? pk_flash_attn_fwd_bf16_f32
               : prec == ATTN_BF16X3 ? pk_flash_attn_fwd_bf16x3_f32
