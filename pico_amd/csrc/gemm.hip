@@ -1099,31 +1099,37 @@ SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int64_t batch, bool allow_
                      bool allow_split) {
     SplitPlan best = {{kTile128, 128, 128}, 1, K};
     double c = -1.0;
-    int64_t s_max = 1, old_chunk;
+    int s_max = 1;
+    int64_t old_chunk;
     size_t cap = ~(size_t)0;
     if(allow_split) {
         const int old = choose_splits(M, N, K, ta, true, &old_chunk);
-        if(old > 1) {
-            s_max = std::min<int64_t>(64, K / (K >= 1024 ? 256 : 128));
+        if(old > 1 && K < (int64_t)1 << 30) {
+            s_max = (int)std::min<int64_t>(64, K / (K >= 1024 ? 256 : 128));
             if((size_t)old * M * N * sizeof(float) <= kNoAllocScratchBytes) cap = kNoAllocScratchBytes;
         }
     }
     const double plane = (double)M * (double)N * 4.0 / 5e6;
+    // (a few dozen counts and 32-bit divisions: this runs on the host for every
+    // product, and all 64 counts in 64-bit took 10 us)
+    static constexpr int kCounts[] = {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 14, 16, 18, 21, 24, 28, 32, 40, 48, 64};
+    const uint32_t k32 = (uint32_t)std::min<int64_t>(K, (int64_t)1 << 30);
     for(const SplitShape& t : kSplitShapes) {
         if(!allow_all && t.kind != kTile128) continue;
         if(t.kind == kTile256x96 && N % 96 != 0) continue;
         const int64_t tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * batch;
-        const int64_t step = 32 * split_groups(t.kind);
-        for(int64_t s = 1; s <= s_max; ++s) {
-            const int64_t chunk = s == 1 ? K : ((K + s - 1) / s + step - 1) / step * step;
-            const int64_t splits = s == 1 ? 1 : (K + chunk - 1) / chunk;
+        const uint32_t step = 32 * split_groups(t.kind);
+        for(const int s : kCounts) {
+            if(s > s_max) break;
+            const uint32_t chunk = s == 1 ? k32 : ((k32 + s - 1) / s + step - 1) / step * step;
+            const uint32_t splits = s == 1 ? 1 : (k32 + chunk - 1) / chunk;
             if(splits > 1 && (size_t)splits * M * N * sizeof(float) > cap) break;
             const int64_t rounds = (tiles * splits + kCUs - 1) / kCUs;
             const double ck = (double)rounds * (t.per_k * (double)chunk + t.fixed) +
                               (splits > 1 ? (double)(splits + 1) * plane + 3.0 : 0.0);
             if(c < 0.0 || ck < c) {
                 c = ck;
-                best = {{t.kind, t.bm, t.bn}, (int)splits, chunk};
+                best = {{t.kind, t.bm, t.bn}, (int)splits, splits == 1 ? K : (int64_t)chunk};
             }
         }
     }
