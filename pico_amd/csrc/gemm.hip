@@ -47,12 +47,10 @@ namespace {
 
 using namespace pkg;
 
-constexpr int KF = BK + 4;  // row stride of a k-contiguous LDS tile [rows][36]
 constexpr int64_t kCUs = 256;  // MI355X
 
-// One operand's R x BK slice, staged into a k-contiguous LDS tile [R][KF].
-// Each staging item is 4 consecutive k of one row, held as one float4 and
-// stored to LDS as one 128-bit write; R/32 items per thread.
+// One operand's R x BK slice, staged into a k-contiguous LDS tile.  Each staging
+// item is 4 consecutive k of one row, held as one float4; R/32 items per thread.
 //  * k-contiguous in memory (KFAST: op(A) when A is not transposed, op(B)^T
 //    when B is): the item is one 128-bit load.
 //  * row-contiguous in memory: the item is four 32-bit loads, one per k, and
@@ -66,7 +64,6 @@ struct Operand {
     static constexpr int ITEMS = R * BK / 4 / NT;
     static constexpr int F4 = ITEMS;            // float4 registers per thread
     static constexpr int OPS = KFAST ? 2 : 5;   // memory instructions per item (loads + store)
-    static constexpr int FLOATS = R * KF;       // LDS floats of one stage
 };
 
 // A tile shape: WGM x (4 / WGM) waves, each TM x TN blocks of 32 x 32.
@@ -209,9 +206,9 @@ __device__ __forceinline__ void load_item(const float* __restrict__ base, int64_
     }
 }
 
-// Row stride (elements) of a k-contiguous LDS tile: fp32 [rows][36]; bf16
-// [rows][40] (80 bytes: the 16-lane passes of 128-bit reads down a column of
-// rows touch 16 distinct 4-bank groups).
+// Row stride (elements) of a k-contiguous bf16 LDS tile: 80 bytes, so the
+// 16-lane passes of 128-bit reads down a column of rows touch 16 distinct
+// 4-bank groups.
 constexpr int KFB = BK + 8;
 // An e4m3 element of an fp8 tile (OCP FP8 E4M3: bias 7, 3 mantissa bits,
 // largest finite 448), one byte.  fp8 tiles have rows of KF8 = 48 bytes:
@@ -232,7 +229,7 @@ __shared__ float g_fp8_scale[2];
 
 template <class E>
 constexpr int lds_stride() {
-    return sizeof(E) == 4 ? KF : sizeof(E) == 1 ? KF8 : KFB;
+    return sizeof(E) == 1 ? KF8 : KFB;
 }
 
 // x rounded to e4m3 (nearest even) after clamping to the finite range, so
@@ -254,17 +251,6 @@ struct SplitBf16 {
     __bf16 hi;
 };
 
-template <int LO>
-__device__ __forceinline__ void put_split(__bf16* t, int off, const float* w, int n) {
-#pragma unroll
-    for(int e = 0; e < 4; ++e) {
-        if(e >= n) break;
-        const __bf16 h = (__bf16)w[e];
-        t[off + e] = h;
-        t[off + LO + e] = (__bf16)(w[e] - (float)h);
-    }
-}
-
 // store 4 consecutive k of one row; a bf16 tile gets them rounded to nearest
 // even, a split tile their hi and lo parts
 template <int LO>
@@ -280,6 +266,11 @@ __device__ __forceinline__ void put4(SplitBf16<LO>* lds, int off, f32x4 w) {
     *reinterpret_cast<bf16x4*>(t + off + LO) = l;
 }
 
+__device__ __forceinline__ void put4(__bf16* lds, int off, f32x4 w) {
+    const bf16x4 b = {(__bf16)w[0], (__bf16)w[1], (__bf16)w[2], (__bf16)w[3]};
+    *reinterpret_cast<bf16x4*>(lds + off) = b;
+}
+
 template <int OP>
 __device__ __forceinline__ void put4(Fp8T<OP>* lds, int off, f32x4 w) {
     const float sc = g_fp8_scale[OP];
@@ -287,22 +278,11 @@ __device__ __forceinline__ void put4(Fp8T<OP>* lds, int off, f32x4 w) {
     *reinterpret_cast<int*>(reinterpret_cast<unsigned char*>(lds) + off) = v;
 }
 
-template <class E>
-__device__ __forceinline__ void put4(E* lds, int off, f32x4 w) {
-    if constexpr(sizeof(E) == 4) {
-        *reinterpret_cast<f32x4*>(lds + off) = w;
-    } else {
-        const bf16x4 b = {(__bf16)w[0], (__bf16)w[1], (__bf16)w[2], (__bf16)w[3]};
-        *reinterpret_cast<bf16x4*>(lds + off) = b;
-    }
-}
-
 template <bool KFAST, int R, class E>
 __device__ __forceinline__ void store_item(E* lds, int item, const f32x4* v) {
-    constexpr int LS = lds_stride<E>();
     int rr, kk;
     item_origin<KFAST, R>(item, rr, kk);
-    put4(lds, rr * LS + kk, v[0]);
+    put4(lds, rr * lds_stride<E>() + kk, v[0]);
 }
 
 // Scheduling hints for one k-group: NMEM memory instructions (LDS or global)
@@ -399,13 +379,15 @@ __device__ __forceinline__ void prologue(const GemmParams& p, const TileJob& j, 
                                           &rb[e], p.pair_F - T::BN / 2);
 }
 
-// The same product with bf16 multiplies: op(A) and op(B) are rounded to bf16
+// The product with bf16 multiplies: op(A) and op(B) are rounded to bf16
 // (nearest even) on their way to LDS and multiplied by
 // v_mfma_f32_32x32x16_bf16 (32768 FLOP per instruction, eight times the fp32
 // rate), accumulating in fp32.  A 32-wide k slice is two MFMA steps of k 16, the
 // second step's fragments read under the first step's MFMAs and the next
 // slice's first fragments under the second.  A lane's 8 k of a step are k
-// 16t + 8*(lane/32) .. +7, the same for both operands.
+// 16t + 8*(lane/32) .. +7, the same for both operands.  Whole tiles only, and
+// of those the ones this is the faster kernel for (narrow_here below); the
+// others' kernel, gemm_narrow.hip, adds the same products in the same order.
 template <int NB>
 __device__ __forceinline__ void read_step(const __bf16* lds, int r0, int lr, int lh, int t,
                                           bf16x8 (&f)[NB]) {
@@ -424,9 +406,10 @@ __device__ __forceinline__ void mfma_step(f32x16 (&acc)[TM][TN], const bf16x8 (&
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
 }
 
-template <bool TA, bool TB, int EDGE, class T, bool SPLIT, int EPI>
+template <bool TA, bool TB, class T, bool SPLIT, int EPI>
 __global__ __launch_bounds__(NT, T::OCC) void gemm_bf16_kernel(GemmParams p) {
     constexpr int BM = T::BM, BN = T::BN, TM = T::TM, TN = T::TN, WGN = T::WGN;
+    constexpr int EDGE = kEdgeNone;
     constexpr bool AK = !TA, BKF = TB;
     using OA = Operand<AK, BM>;
     using OB = Operand<BKF, BN>;
@@ -1061,6 +1044,8 @@ int choose_splits(int64_t M, int64_t N, int64_t K, bool ta, bool fp32, int64_t* 
     return (int)((K + chunk - 1) / chunk);
 }
 
+enum Precision { kFp32 = 0, kBf16 = 1, kBf16x3 = 2, kFp8 = 3 };
+
 // fp32 products (gemm_split.h): tile shape and K split together, by the
 // estimated time of the busiest CU -- its workgroups, ceil(tiles * splits / 256
 // CUs), each `per_k` per k of its range plus `fixed` for its prologue and
@@ -1078,11 +1063,38 @@ struct SplitShape {
     int bm, bn;
     double per_k, fixed;
 };
-constexpr SplitShape kSplitShapes[] = {{kTile128, 128, 128, 0.0400, 4.0},
-                                       {kTile256, 256, 256, 0.1370, 11.0},
-                                       {kTile256x96, 256, 96, 0.0610, 6.5},
-                                       {kTile128x64, 128, 64, 0.0252, 3.5},
-                                       {kTile64, 64, 64, 0.0145, 3.0}};
+constexpr SplitShape kSplitShapes[5] = {{kTile128, 128, 128, 0.0400, 4.0},
+                                        {kTile256, 256, 256, 0.1370, 11.0},
+                                        {kTile256x96, 256, 96, 0.0610, 6.5},
+                                        {kTile128x64, 128, 64, 0.0252, 3.5},
+                                        {kTile64, 64, 64, 0.0145, 3.0}};
+// The same for bf16 and split-bf16 multiplies: 4096^3 takes 256x256, [8192, 768]
+// 256x96, [4096, 768] 128x96, 2048^3 128x128, 1024^3 64x64.  A split keeps to
+// 256x256, 128x128 and 64x64, and A^T.B to those altogether, whose operand
+// traffic the 96-column tiles double: the gradient [768, 4096] with K 8192 runs
+// in 4 splits of 256x256 (bf16 130 -> 97 us, split bf16 200 -> 164, in 8 of
+// 128x128 before), [768, 2304] in 8 (107 -> 80, 127 -> 98).
+constexpr SplitShape kNarrowShapes[2][5] = {{{kTile128, 128, 128, 0.0160, 2.5},
+                                             {kTile256, 256, 256, 0.0430, 8.0},
+                                             {kTile256x96, 256, 96, 0.0205, 3.5},
+                                             {kTile96, 128, 96, 0.0125, 2.5},
+                                             {kTile64, 64, 64, 0.0075, 2.5}},
+                                            {{kTile128, 128, 128, 0.0285, 2.5},
+                                             {kTile256, 256, 256, 0.0840, 11.0},
+                                             {kTile256x96, 256, 96, 0.0385, 4.0},
+                                             {kTile96, 128, 96, 0.0215, 2.5},
+                                             {kTile64, 64, 64, 0.0115, 2.5}}};
+
+// Whether a whole-tile bf16 or split-bf16 product runs on the four-wave kernel
+// of this file rather than gemm_narrow.hip's: the 96-column tiles (64x96 per
+// wave; eight waves of 32x96 read LDS faster than it delivers: [8192, 768] K
+// 2048 83 against 91 us split, 48.4 against 48.8 bf16; [8192, 2304] K 768 101
+// against 113, 55 against 58), and split bf16, whose products hide the staging
+// of four waves (2048^3 64.9 against 67.2, 1024^3 18.9 against 19.6; bf16 41.1
+// against 39.0 and 13.1 against 12.9 stays there).
+bool narrow_here(int prec, TileKind kind) {
+    return kind == kTile256x96 || kind == kTile96 || prec == kBf16x3;
+}
 
 struct SplitPlan {
     TileChoice tile;
@@ -1095,15 +1107,17 @@ struct SplitPlan {
 // keeps fitting
 constexpr size_t kNoAllocScratchBytes = (size_t)128 << 20;
 
-SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int64_t batch, bool allow_all, bool ta,
-                     bool allow_split) {
+SplitPlan plan_split(int prec, int64_t M, int64_t N, int64_t K, int64_t batch, bool allow_all,
+                     bool ta, bool allow_split, bool allow_96 = true) {
+    const bool fp32 = prec == kFp32;
+    const SplitShape* const shapes = fp32 ? kSplitShapes : kNarrowShapes[prec - kBf16];
     SplitPlan best = {{kTile128, 128, 128}, 1, K};
     double c = -1.0;
     int s_max = 1;
     int64_t old_chunk;
     size_t cap = ~(size_t)0;
     if(allow_split) {
-        const int old = choose_splits(M, N, K, ta, true, &old_chunk);
+        const int old = choose_splits(M, N, K, ta, fp32, &old_chunk);
         if(old > 1 && K < (int64_t)1 << 30) {
             s_max = (int)std::min<int64_t>(64, K / (K >= 1024 ? 256 : 128));
             if((size_t)old * M * N * sizeof(float) <= kNoAllocScratchBytes) cap = kNoAllocScratchBytes;
@@ -1114,13 +1128,15 @@ SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int64_t batch, bool allow_
     // product, and all 64 counts in 64-bit took 10 us)
     static constexpr int kCounts[] = {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 14, 16, 18, 21, 24, 28, 32, 40, 48, 64};
     const uint32_t k32 = (uint32_t)std::min<int64_t>(K, (int64_t)1 << 30);
-    for(const SplitShape& t : kSplitShapes) {
+    for(int i = 0; i < 5; ++i) {
+        const SplitShape& t = shapes[i];
+        const bool n96 = t.bn == 96;
         if(!allow_all && t.kind != kTile128) continue;
-        if(t.kind == kTile256x96 && N % 96 != 0) continue;
+        if(n96 && (N % 96 != 0 || (!fp32 && (ta || !allow_96 || M % t.bm != 0)))) continue;
         const int64_t tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * batch;
-        const uint32_t step = 32 * split_groups(t.kind);
+        const uint32_t step = fp32 ? 32 * split_groups(t.kind) : 32;
         for(const int s : kCounts) {
-            if(s > s_max) break;
+            if(s > (n96 && !fp32 ? 1 : s_max)) break;
             const uint32_t chunk = s == 1 ? k32 : ((k32 + s - 1) / s + step - 1) / step * step;
             const uint32_t splits = s == 1 ? 1 : (k32 + chunk - 1) / chunk;
             if(splits > 1 && (size_t)splits * M * N * sizeof(float) > cap) break;
@@ -1136,16 +1152,15 @@ SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int64_t batch, bool allow_
     return best;
 }
 
-enum Precision { kFp32 = 0, kBf16 = 1, kBf16x3 = 2, kFp8 = 3 };
-
 template <bool TA, bool TB, class T, int EDGE, int EPI>
 void launch_epi(const GemmParams& gp, dim3 grid, int prec, hipStream_t st) {
+    constexpr bool T96 = T::BN == 96;
     if(prec == kFp8)
         gemm_fp8_kernel<TA, TB, EDGE, T, EPI><<<grid, NT, 0, st>>>(gp);
-    else if(prec == kBf16)
-        gemm_bf16_kernel<TA, TB, EDGE, T, false, EPI><<<grid, NT, 0, st>>>(gp);
-    else if(prec == kBf16x3)
-        gemm_bf16_kernel<TA, TB, EDGE, T, true, EPI><<<grid, NT, 0, st>>>(gp);
+    else if constexpr(EDGE == kEdgeNone) {
+        if(prec == kBf16x3) gemm_bf16_kernel<TA, TB, T, true, EPI><<<grid, NT, 0, st>>>(gp);
+        else if constexpr(T96) gemm_bf16_kernel<TA, TB, T, false, EPI><<<grid, NT, 0, st>>>(gp);
+    }
 }
 
 // The staged epilogues are instantiated only where they are used: the
@@ -1175,8 +1190,7 @@ int launch_tile(const GemmParams& gp, int64_t batch, int edge, int prec, hipStre
         launch_kernel<TA, TB, T, kEdgeScalar>(gp, grid, prec, st);
     return pk::launch_status(prec == kBf16     ? "pk_gemm_bf16_f32"
                              : prec == kBf16x3 ? "pk_gemm_bf16x3_f32"
-                             : prec == kFp8    ? "pk_gemm_fp8_f32"
-                                               : "pk_gemm_f32");
+                                               : "pk_gemm_fp8_f32");
 }
 
 template <bool TA, bool TB>
@@ -1189,6 +1203,14 @@ int launch(const GemmParams& gp, int64_t batch, int edge, TileKind kind, int pre
     case kTile64: return launch_tile<TA, TB, Tile64>(gp, batch, edge, prec, st);
     default: return launch_tile<TA, TB, Tile128>(gp, batch, edge, prec, st);
     }
+}
+
+int launch_layout(bool ta, bool tb, const GemmParams& gp, int64_t batch, int edge, TileKind kind,
+                  int prec, hipStream_t st) {
+    if(!ta && !tb) return launch<false, false>(gp, batch, edge, kind, prec, st);
+    if(!ta && tb) return launch<false, true>(gp, batch, edge, kind, prec, st);
+    if(ta && !tb) return launch<true, false>(gp, batch, edge, kind, prec, st);
+    return launch<true, true>(gp, batch, edge, kind, prec, st);
 }
 
 // what a product's tiles write besides alpha * op(A) . op(B): the beta term's
@@ -1349,18 +1371,39 @@ int gemm_impl(char ta, char tb, int64_t M, int64_t N, int64_t K, float alpha, co
     gp.kchunk = K;
     gp.ws = nullptr;
     const bool may_split = batch == 1 && causal == 0 && ws && K > 0 && !swiglu && !sfwd;
+    // a tile's loads reach 32-bit byte offsets: 256 rows of a k-contiguous
+    // operand, 16 (fp32) or 32 k rows of the other kind
+    const int64_t near_k = (int64_t)1 << 21, near_r = (int64_t)1 << (prec == kFp32 ? 25 : 24);
+    gp.exact_only = lda > (TA ? near_r : near_k) || ldb > (TB ? near_k : near_r);
     SplitPlan plan = {{kTile128, 128, 128}, 1, K};
-    if(prec == kFp32) plan = plan_split(M, N, K, batch, causal == 0, TA, may_split);
-    if(may_split) {
-        int64_t kchunk = plan.kchunk;
-        const int S = prec == kFp32 ? plan.splits : choose_splits(M, N, K, TA, false, &kchunk);
-        if(S > 1 && ws_bytes >= (size_t)S * (size_t)M * (size_t)N * sizeof(float)) {
-            gp.splits = S;
-            gp.kchunk = kchunk;
-            gp.ws = ws;
-        } else if(S > 1 && prec == kFp32) {
-            plan = plan_split(M, N, K, batch, true, TA, false);
-        }
+    // fp8 and the four-wave bf16 kernel: float4 loads need 16-byte aligned operands
+    // and leading dimensions and batch strides that are multiples of 4; the
+    // unchecked path also needs whole tiles, loaded through buffer resources with
+    // 32-bit offsets from each operand's start: op(A) and op(B) must each span
+    // less than 2^31 bytes
+    const bool vec = (lda % 4) == 0 && (ldb % 4) == 0 && (sA_outer % 4) == 0 &&
+                     (sA_inner % 4) == 0 && (sB_outer % 4) == 0 && (sB_inner % 4) == 0 &&
+                     pk::aligned16(A) && pk::aligned16(B);
+    auto extent = [K](bool kfast, int64_t rows, int64_t ld) {
+        return 4 * (kfast ? (rows - 1) * ld + K : (K - 1) * ld + rows);
+    };
+    const bool small = extent(!TA, M, lda) < INT32_MAX && extent(TB, N, ldb) < INT32_MAX;
+    const bool fast = vec && small && K % BK == 0;
+    if(prec != kFp8) {
+        const bool use96 = fast && (gp.pair_F == 0 || gp.pair_F % 48 == 0);
+        plan = plan_split(prec, M, N, K, batch, causal == 0, TA, may_split, use96);
+        if(plan.splits > 1 && ws_bytes < (size_t)plan.splits * (size_t)M * (size_t)N * sizeof(float))
+            plan = plan_split(prec, M, N, K, batch, true, TA, false, use96);
+        if(prec != kFp32 && gp.exact_only) plan.tile = {kTile64, 64, 64};
+    } else if(may_split) {
+        plan.splits = choose_splits(M, N, K, TA, false, &plan.kchunk);
+        if(ws_bytes < (size_t)plan.splits * (size_t)M * (size_t)N * sizeof(float))
+            plan.splits = 1;
+    }
+    if(plan.splits > 1) {
+        gp.splits = plan.splits;
+        gp.kchunk = plan.kchunk;
+        gp.ws = ws;
     }
     auto v4 = [](const void* q, int64_t ld) {
         return q == nullptr || (pk::aligned16(q) && ld % 4 == 0);
@@ -1368,17 +1411,17 @@ int gemm_impl(char ta, char tb, int64_t M, int64_t N, int64_t K, float alpha, co
     gp.epi_vec = v4(C, ldc) && v4(gp.Cin, gp.ldcin) && v4(gp.sg_a, gp.sg_lda) &&
                  v4(gp.sg_u, gp.sg_ldu) && v4(gp.sg_da, gp.sg_ldd) && v4(gp.sg_du, gp.sg_ldd) &&
                  v4(gp.sf_h, gp.sf_ldh) && (gp.splits == 1 || v4(gp.ws, N));
-    // split products keep 128x128 tiles (the split count is sized for them);
-    // causal products keep 128-row tiles (the attention chain's diagonal logic
-    // is exercised at that size)
+    // fp8: split products keep 128x128 tiles (the split count is sized for them);
+    // causal products of any precision keep 128-row tiles (the attention chain's
+    // diagonal logic is exercised at that size)
     TileChoice tc = gp.splits > 1 ? TileChoice{kTile128, 128, 128}
                                   : pick_tile(M, N, batch, causal == 0, gp.pair_F);
     if(tc.bm == 0)
         return pk::fail("pk_gemm_swiglu_fwd_f32: F=%lld is not a multiple of 32 (no tile holds "
                         "whole gate/up column pairs)", (long long)gp.pair_F);
-    // fp32: a shape for M, N and K alone (the SwiGLU-forward product's tiles may
-    // hold partial columns), so every epilogue adds K in the same order
-    if(prec == kFp32) tc = plan.tile;
+    // the others: a shape for M, N and K alone (the SwiGLU-forward product's tiles
+    // may hold partial columns), so every epilogue adds K in the same order
+    if(prec != kFp8) tc = plan.tile;
     const int64_t tiles_m = (M + tc.bm - 1) / tc.bm,
                   tiles_n = gp.pair_F ? (gp.pair_F + tc.bn / 2 - 1) / (tc.bn / 2)
                                       : (N + tc.bn - 1) / tc.bn;
@@ -1388,40 +1431,22 @@ int gemm_impl(char ta, char tb, int64_t M, int64_t N, int64_t K, float alpha, co
     gp.tiles_n = (int)tiles_n;
     const TileKind kind = tc.kind;
     int rc;
-    if(prec == kFp32) {
-        const int64_t kstep = 32 * split_groups(kind);
+    if(prec != kFp8) {
+        const int64_t kstep = prec == kFp32 ? 32 * split_groups(kind) : 32;
         const bool whole = M % tc.bm == 0 && K % kstep == 0 && gp.kchunk % kstep == 0 &&
                            (gp.pair_F ? gp.pair_F % (tc.bn / 2) == 0 : N % tc.bn == 0);
-        // a tile's loads reach 32-bit byte offsets: 256 rows of a k-contiguous
-        // operand, 16 k rows of the other kind
-        const int64_t near_k = (int64_t)1 << 21, near_r = (int64_t)1 << 25;
-        gp.exact_only = lda > (TA ? near_r : near_k) || ldb > (TB ? near_k : near_r);
-        rc = launch_split(TA, TB, gp, batch, !whole, kind, st);
+        if(prec == kFp32)
+            rc = launch_split(TA, TB, gp, batch, !whole, kind, st);
+        else if(whole && fast && narrow_here(prec, kind))
+            rc = launch_layout(TA, TB, gp, batch, kEdgeNone, kind, prec, st);
+        else
+            rc = launch_narrow(TA, TB, prec, gp, batch, !whole, kind, st);
     } else {
-        // float4 loads need 16-byte aligned operands and leading dimensions and
-        // batch strides that are multiples of 4; the unchecked path also needs
-        // whole tiles
-        const bool vec = (lda % 4) == 0 && (ldb % 4) == 0 && (sA_outer % 4) == 0 &&
-                         (sA_inner % 4) == 0 && (sB_outer % 4) == 0 && (sB_inner % 4) == 0 &&
-                         pk::aligned16(A) && pk::aligned16(B);
-        const bool whole = (M % tc.bm) == 0 && (N % tc.bn) == 0 && (K % BK) == 0;
-        // whole tiles load through buffer resources with 32-bit offsets from each
-        // operand's start: op(A) and op(B) must each span less than 2^31 bytes
-        auto extent = [K](bool kfast, int64_t rows, int64_t ld) {
-            return 4 * (kfast ? (rows - 1) * ld + K : (K - 1) * ld + rows);
-        };
-        const bool small = extent(!TA, M, lda) < INT32_MAX && extent(TB, N, ldb) < INT32_MAX;
-        const int edge = vec && whole && small ? kEdgeNone
+        const bool whole = (M % tc.bm) == 0 && (N % tc.bn) == 0;
+        const int edge = fast && whole ? kEdgeNone
                          : vec && (M % 4) == 0 && (N % 4) == 0 && (K % 4) == 0 ? kEdgeVec
                                                                                : kEdgeScalar;
-        if(!TA && !TB)
-            rc = launch<false, false>(gp, batch, edge, kind, prec, st);
-        else if(!TA && TB)
-            rc = launch<false, true>(gp, batch, edge, kind, prec, st);
-        else if(TA && !TB)
-            rc = launch<true, false>(gp, batch, edge, kind, prec, st);
-        else
-            rc = launch<true, true>(gp, batch, edge, kind, prec, st);
+        rc = launch_layout(TA, TB, gp, batch, edge, kind, prec, st);
     }
     if(rc || gp.splits == 1) return rc;
     splitk_reduce<<<pk::grid_for(M * N / 4 + 1, NT), NT, 0, st>>>(
@@ -1454,20 +1479,22 @@ extern "C" int pk_gemm_f32(char ta, char tb, int64_t M, int64_t N, int64_t K, fl
 }
 
 // the split-K partials of op(A) . op(B) for one layout of A
-static size_t gemm_workspace(int64_t M, int64_t N, int64_t K, bool ta) {
+static size_t gemm_workspace(int prec, int64_t M, int64_t N, int64_t K, bool ta) {
     if(M <= 0 || N <= 0 || K <= 0) return 0;
-    const int S = plan_split(M, N, K, 1, true, ta, true).splits;
+    const int S = plan_split(prec, M, N, K, 1, true, ta, true).splits;
     return S > 1 ? (size_t)S * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
 // any layout (A^T.B splits whenever another layout of the shape does) and any
-// precision: the opt-in ones split by choose_splits alone
+// precision: fp8 splits by choose_splits alone
 extern "C" size_t pk_gemm_workspace_f32(int64_t M, int64_t N, int64_t K) {
     if(M <= 0 || N <= 0 || K <= 0) return 0;
     int64_t kchunk;
     const int S = choose_splits(M, N, K, true, true, &kchunk);
-    return std::max(gemm_workspace(M, N, K, true),
-                    S > 1 ? (size_t)S * (size_t)M * (size_t)N * sizeof(float) : 0);
+    size_t most = S > 1 ? (size_t)S * (size_t)M * (size_t)N * sizeof(float) : 0;
+    for(const int prec : {kFp32, kBf16, kBf16x3})
+        most = std::max(most, gemm_workspace(prec, M, N, K, true));
+    return most;
 }
 
 extern "C" int pk_gemm_ex_f32(char ta, char tb, int64_t M, int64_t N, int64_t K, float alpha,
@@ -1721,7 +1748,7 @@ extern "C" int pk_gemm_noalloc_f32(char ta, char tb, int64_t M, int64_t N, int64
         return pk::fail("pk_gemm_noalloc_f32: this product's split-K partials need %zu bytes, "
                         "above the %zu-byte static scratch (use pk_gemm_ex_f32 with a workspace)",
                         most, kNoAllocScratchBytes);
-    const size_t need = gemm_workspace(M, N, K, TA);
+    const size_t need = gemm_workspace(kFp32, M, N, K, TA);
     float* ws = nullptr;
     if(need > 0 && !(ws = scratch_on_current_device())) return PK_EINVAL;
     // every partial-plane element the reduction reads is written by its split

@@ -293,7 +293,7 @@ __device__ __forceinline__ void staged_epilogue(const GemmParams& p, const TileJ
     }
 }
 
-// (128x96 tiles: the opt-in precisions' kernels only; 128x64: fp32 only)
+// (128x96 tiles: fp8 only; 128x64: fp32 only)
 enum TileKind { kTile128, kTile96, kTile256, kTile64, kTile256x96, kTile128x64 };
 
 
@@ -302,5 +302,10 @@ enum TileKind { kTile128, kTile96, kTile256, kTile64, kTile256x96, kTile128x64 }
 int split_groups(TileKind kind);
 int launch_split(bool ta, bool tb, const GemmParams& gp, int64_t batch, bool edge, TileKind kind,
                  hipStream_t st);
+
+// the bf16 (parts 1) and split-bf16 (parts 2) products (gemm_narrow.hip); with
+// gp.exact_only, 64x64 tiles only
+int launch_narrow(bool ta, bool tb, int parts, const GemmParams& gp, int64_t batch, bool edge,
+                  TileKind kind, hipStream_t st);
 
 }  // namespace pkg

@@ -1,5 +1,6 @@
 // pico_amd/csrc/gemm_split.h -- the fp32 product on the bf16 matrix cores.
-// Part of gemm_split.hip (included inside its anonymous namespace).
+// Included inside the anonymous namespace of gemm_split.hip, which launches it,
+// and of gemm_narrow.hip, whose kernel shares the staging.
 //
 // The fp32 matrix cores are 16 times slower than the bf16 ones, and a SIMD's
 // vector instructions do not overlap fp32 matrix instructions while they do
@@ -68,13 +69,13 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x2 __attribute__((ext_vector_type(2)));
 
-// One operand's R x 16 slice as staged by THREADS threads: items of KPI
+// One operand's R x W slice as staged by THREADS threads: items of KPI
 // consecutive k of one row, ITEMS per thread (threads past the last item
 // repeat an earlier one).
-template <bool KFAST, int R, int THREADS>
+template <bool KFAST, int R, int THREADS, int W = SK>
 struct SplitOperand {
-    static constexpr int KPI = KFAST ? 4 : (R * 2 >= THREADS ? 8 : 4);
-    static constexpr int COUNT = R * SK / KPI;
+    static constexpr int KPI = KFAST ? 4 : (R * W / 8 >= THREADS ? 8 : 4);
+    static constexpr int COUNT = R * W / KPI;
     static constexpr int ITEMS = (COUNT + THREADS - 1) / THREADS;
     static constexpr int LOADS = KFAST ? 1 : KPI;
 
@@ -82,8 +83,8 @@ struct SplitOperand {
         int u = threadIdx.x % THREADS + item * THREADS;
         if(ITEMS * THREADS != COUNT) u %= COUNT;
         if(KFAST) {
-            rr = u >> 2;
-            kk = (u & 3) * 4;
+            rr = u / (W / 4);
+            kk = u % (W / 4) * 4;
         } else {
             rr = u % R;
             kk = (u / R) * KPI;
@@ -98,12 +99,12 @@ struct SplitSource {
     int64_t kstep;     // bytes per k
 };
 
-template <bool KFAST, bool EDGE, int R, int THREADS, bool PAIR>
+template <bool KFAST, bool EDGE, int R, int THREADS, bool PAIR, int W = SK>
 __device__ __forceinline__ void split_load(const SplitSource& src, int64_t ld, int64_t k0,
                                            int64_t shift,
-                                           float (&v)[SplitOperand<KFAST, R, THREADS>::ITEMS]
-                                                     [SplitOperand<KFAST, R, THREADS>::KPI]) {
-    using O = SplitOperand<KFAST, R, THREADS>;
+                                           float (&v)[SplitOperand<KFAST, R, THREADS, W>::ITEMS]
+                                                     [SplitOperand<KFAST, R, THREADS, W>::KPI]) {
+    using O = SplitOperand<KFAST, R, THREADS, W>;
     const int64_t off = k0 * src.kstep;
     const int64_t left = src.left - off;
     const unsigned num = EDGE ? (left <= 0 ? 0u : left > 0xfffffff0ll ? 0xfffffff0u : (unsigned)left)
@@ -131,12 +132,12 @@ __device__ __forceinline__ void split_load(const SplitSource& src, int64_t ld, i
     }
 }
 
-// zero the values at k >= limit (limit < 16: the last, partial slice)
-template <bool KFAST, int R, int THREADS>
+// zero the values at k >= limit (limit < W: the last, partial slice)
+template <bool KFAST, int R, int THREADS, int W = SK>
 __device__ __forceinline__ void split_mask(int limit,
-                                           float (&v)[SplitOperand<KFAST, R, THREADS>::ITEMS]
-                                                     [SplitOperand<KFAST, R, THREADS>::KPI]) {
-    using O = SplitOperand<KFAST, R, THREADS>;
+                                           float (&v)[SplitOperand<KFAST, R, THREADS, W>::ITEMS]
+                                                     [SplitOperand<KFAST, R, THREADS, W>::KPI]) {
+    using O = SplitOperand<KFAST, R, THREADS, W>;
 #pragma unroll
     for(int i = 0; i < O::ITEMS; ++i) {
         int rr, kk;
@@ -166,23 +167,36 @@ __device__ __forceinline__ int split_off(int row, int k) {
     return row * SK + ((((k >> 3) ^ (row >> 2)) & 1) << 3) + (k & 7);
 }
 
-template <bool KFAST, int R, int THREADS, int PART>
+// P parts of every value into [k / 16][part][row][16]: 3 as above, 2 hi and lo
+// (lo = bf16(x - hi)), 1 rounded to bf16
+template <int P, bool KFAST, int R, int THREADS, int PART, int W = SK>
 __device__ __forceinline__ void split_store(short* lds,
-                                            const float (&v)[SplitOperand<KFAST, R, THREADS>::ITEMS]
-                                                            [SplitOperand<KFAST, R, THREADS>::KPI],
+                                            const float (&v)[SplitOperand<KFAST, R, THREADS, W>::ITEMS]
+                                                            [SplitOperand<KFAST, R, THREADS, W>::KPI],
                                             float scale) {
-    using O = SplitOperand<KFAST, R, THREADS>;
+    using O = SplitOperand<KFAST, R, THREADS, W>;
 #pragma unroll
     for(int i = 0; i < O::ITEMS; ++i) {
         int rr, kk;
         O::origin(i, rr, kk);
-        const int off = split_off(rr, kk);
+        const int off = split_off(rr, kk % SK) + kk / SK * (P * PART);
         int w[3][O::KPI / 2];
 #pragma unroll
-        for(int t = 0; t < O::KPI / 2; ++t)
-            split3(v[i][2 * t], v[i][2 * t + 1], scale, w[0][t], w[1][t], w[2][t]);
+        for(int t = 0; t < O::KPI / 2; ++t) {
+            if constexpr(P == 3) {
+                split3(v[i][2 * t], v[i][2 * t + 1], scale, w[0][t], w[1][t], w[2][t]);
+            } else {
+                const f32x2 x = {v[i][2 * t], v[i][2 * t + 1]};
+                const bf16x2 h = __builtin_convertvector(x, bf16x2);
+                w[0][t] = __builtin_bit_cast(int, h);
+                if constexpr(P == 2) {
+                    const f32x2 r = {x[0] - (float)h[0], x[1] - (float)h[1]};
+                    w[1][t] = __builtin_bit_cast(int, __builtin_convertvector(r, bf16x2));
+                }
+            }
+        }
 #pragma unroll
-        for(int q = 0; q < 3; ++q) {
+        for(int q = 0; q < P; ++q) {
             if constexpr(O::KPI == 8)
                 *reinterpret_cast<i32x4*>(lds + q * PART + off) =
                     i32x4{w[q][0], w[q][1], w[q][2], w[q][3]};
@@ -316,8 +330,8 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmPara
             split_load<BKF, EDGE, BN, NT_, PAIR>(sb, p.ldb, k0, shift, r.b);
         };
         auto store = [&](const Regs& r, int stage, float scale_a) {
-            split_store<AK, BM, NT_, PART>(lds + stage * STAGE, r.a, scale_a);
-            split_store<BKF, BN, NT_, PART>(lds + stage * STAGE + BM * SK, r.b, 0x1p16f);
+            split_store<3, AK, BM, NT_, PART>(lds + stage * STAGE, r.a, scale_a);
+            split_store<3, BKF, BN, NT_, PART>(lds + stage * STAGE + BM * SK, r.b, 0x1p16f);
         };
         auto mask = [&](Regs& r, int s) {
             if constexpr(EDGE) {
