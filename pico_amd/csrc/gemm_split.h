@@ -106,11 +106,15 @@ __device__ __forceinline__ void split_load(const SplitSource& src, int64_t ld, i
                                                      [SplitOperand<KFAST, R, THREADS, W>::KPI]) {
     using O = SplitOperand<KFAST, R, THREADS, W>;
     const int64_t off = k0 * src.kstep;
-    const int64_t left = src.left - off;
-    const unsigned num = EDGE ? (left <= 0 ? 0u : left > 0xfffffff0ll ? 0xfffffff0u : (unsigned)left)
-                              : 0xfffffff0u;
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char*>(src.base + off), (short)0, (int)num, 0x00020000);
+    // the operand from `skip` bytes past the slice's first value on
+    auto rest = [&](int64_t skip) {
+        const int64_t left = src.left - off - skip;
+        const unsigned num = EDGE ? (left <= 0 ? 0u : left > 0xfffffff0ll ? 0xfffffff0u : (unsigned)left)
+                                  : 0xfffffff0u;
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(src.base + off + skip), (short)0,
+                                                 (int)num, 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t rs = rest(0);
 #pragma unroll
     for(int i = 0; i < O::ITEMS; ++i) {
         int rr, kk;
@@ -123,11 +127,25 @@ __device__ __forceinline__ void split_load(const SplitSource& src, int64_t ld, i
 #pragma unroll
             for(int t = 0; t < 4; ++t) v[i][t] = x[t];
         } else {
-            const int voff = (int)((kk * (unsigned)ld + row) * 4u);
+            // whole tiles reach their k rows by the scalar offset; bounded loads do
+            // not, as only the vector offset is sure to be checked.  Slices of 16 k
+            // add it up anew each time (kept over the loop, the offsets spill in
+            // 256-row tiles), those of 32 k, with no vector register to spare, take
+            // a resource per k row (which would spill scalar registers in the other)
+            unsigned voff = (kk * (unsigned)ld + row) * 4u;
+            const unsigned step = (unsigned)ld * 4u;
+            if(EDGE && W == SK) asm volatile("" : "+v"(voff));
 #pragma unroll
-            for(int t = 0; t < O::KPI; ++t)
-                v[i][t] = __builtin_bit_cast(
-                    float, __builtin_amdgcn_raw_buffer_load_b32(rs, voff, (int)(t * (unsigned)ld * 4u), 0));
+            for(int t = 0; t < O::KPI; ++t) {
+                int x;
+                if(!EDGE)
+                    x = __builtin_amdgcn_raw_buffer_load_b32(rs, (int)voff, (int)(t * step), 0);
+                else if(W == SK)
+                    x = __builtin_amdgcn_raw_buffer_load_b32(rs, (int)(voff + t * step), 0, 0);
+                else
+                    x = __builtin_amdgcn_raw_buffer_load_b32(rest(t * src.kstep), (int)voff, 0, 0);
+                v[i][t] = __builtin_bit_cast(float, x);
+            }
         }
     }
 }
