@@ -382,41 +382,95 @@ __device__ __forceinline__ float un_bwd(int op, float gx, float x, float y, floa
     }
 }
 
-__global__ void unary_kernel(int op, int64_t n, const float* __restrict__ x, float* __restrict__ y) {
-    for(int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-        i += (int64_t)gridDim.x * blockDim.x)
-        y[i] = un_apply(op, x[i]);
+// W elements per load, the last n % W one to a thread.  tanh is bound by the
+// double-precision function, its gradient by HBM ([4096, 2048]: 52 and 19 us an
+// element at a time with the op tested per element, 44 and 17 four at a time).
+template <int W>
+using vecw = float __attribute__((ext_vector_type(W)));
+
+template <int OP, int W>
+__global__ void unary_kernel(int64_t n, const float* __restrict__ x, float* __restrict__ y) {
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, nv = n / W;
+    for(int64_t i = t; i < nv; i += (int64_t)gridDim.x * blockDim.x) {
+        vecw<W> v = reinterpret_cast<const vecw<W>*>(x)[i];
+#pragma unroll
+        for(int e = 0; e < W; ++e) v[e] = un_apply(OP, v[e]);
+        reinterpret_cast<vecw<W>*>(y)[i] = v;
+    }
+    if(W > 1 && nv * W + t < n) y[nv * W + t] = un_apply(OP, x[nv * W + t]);
 }
 
 // sqrt and tanh read y only, the others x only
-__global__ void unary_bwd_kernel(int op, int64_t n, const float* __restrict__ x,
+template <int OP, int W>
+__global__ void unary_bwd_kernel(int64_t n, const float* __restrict__ x,
                                  const float* __restrict__ y, const float* __restrict__ gy,
                                  float* __restrict__ gx, int accum) {
-    const bool use_y = op == 0 || op == 4;
-    const float* __restrict__ s = use_y ? y : x;
-    for(int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-        i += (int64_t)gridDim.x * blockDim.x) {
-        const float v = s[i];
-        gx[i] = un_bwd(op, accum ? gx[i] : 0.0f, v, v, gy[i]);
+    const float* __restrict__ s = OP == 0 || OP == 4 ? y : x;
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, nv = n / W;
+    for(int64_t i = t; i < nv; i += (int64_t)gridDim.x * blockDim.x) {
+        const vecw<W> v = reinterpret_cast<const vecw<W>*>(s)[i];
+        const vecw<W> g = reinterpret_cast<const vecw<W>*>(gy)[i];
+        vecw<W> r;
+        if(accum) {
+            r = reinterpret_cast<const vecw<W>*>(gx)[i];
+        } else {
+#pragma unroll
+            for(int e = 0; e < W; ++e) r[e] = 0.0f;
+        }
+#pragma unroll
+        for(int e = 0; e < W; ++e) r[e] = un_bwd(OP, r[e], v[e], v[e], g[e]);
+        reinterpret_cast<vecw<W>*>(gx)[i] = r;
     }
+    if(W > 1 && nv * W + t < n) {
+        const int64_t i = nv * W + t;
+        gx[i] = un_bwd(OP, accum ? gx[i] : 0.0f, s[i], s[i], gy[i]);
+    }
+}
+
+// four elements a thread where that still gives every CU four waves of it and
+// the tensors are 16-byte aligned; below, one (the double-precision functions
+// of four elements would follow each other on few waves)
+static bool wide_unary(int64_t n, const void* a, const void* b, const void* c) {
+    return n >= (int64_t)1 << 18 && pk::aligned16(a) && pk::aligned16(b) && pk::aligned16(c);
 }
 
 // ------------------------------------------------------------------ relu
 __device__ __forceinline__ float relu1(float x) { return x > 0.0f ? x : 0.0f; }
 
+template <int W>
 __global__ void relu_kernel(int64_t n, const float* __restrict__ x, float* __restrict__ y) {
-    for(int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-        i += (int64_t)gridDim.x * blockDim.x)
-        y[i] = relu1(x[i]);
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, nv = n / W;
+    for(int64_t i = t; i < nv; i += (int64_t)gridDim.x * blockDim.x) {
+        vecw<W> v = reinterpret_cast<const vecw<W>*>(x)[i];
+#pragma unroll
+        for(int e = 0; e < W; ++e) v[e] = relu1(v[e]);
+        reinterpret_cast<vecw<W>*>(y)[i] = v;
+    }
+    if(W > 1 && nv * W + t < n) y[nv * W + t] = relu1(x[nv * W + t]);
 }
 
+__device__ __forceinline__ float relu_bwd1(float y, float gy, float gx, int accum) {
+    const float gate = (float)(y > 0.0f);
+    const float t = gy * gate;
+    return accum ? gx + t : t;
+}
+
+template <int W>
 __global__ void relu_bwd_kernel(int64_t n, const float* __restrict__ y,
                                 const float* __restrict__ gy, float* __restrict__ gx, int accum) {
-    for(int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-        i += (int64_t)gridDim.x * blockDim.x) {
-        const float gate = (float)(y[i] > 0.0f);
-        const float t = gy[i] * gate;
-        gx[i] = accum ? gx[i] + t : t;
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, nv = n / W;
+    for(int64_t i = t; i < nv; i += (int64_t)gridDim.x * blockDim.x) {
+        const vecw<W> v = reinterpret_cast<const vecw<W>*>(y)[i];
+        const vecw<W> g = reinterpret_cast<const vecw<W>*>(gy)[i];
+        vecw<W> r = g;
+        if(accum) r = reinterpret_cast<const vecw<W>*>(gx)[i];
+#pragma unroll
+        for(int e = 0; e < W; ++e) r[e] = relu_bwd1(v[e], g[e], r[e], accum);
+        reinterpret_cast<vecw<W>*>(gx)[i] = r;
+    }
+    if(W > 1 && nv * W + t < n) {
+        const int64_t i = nv * W + t;
+        gx[i] = relu_bwd1(y[i], gy[i], accum ? gx[i] : 0.0f, accum);
     }
 }
 
@@ -1036,7 +1090,18 @@ extern "C" int pk_unary_f32(int op, int64_t n, const float* x, float* y, pk_stre
     if(!valid_op(op, 5)) return pk::fail("pk_unary_f32: op %d not in 0..5", op);
     if(n <= 0) return n < 0 ? pk::fail("pk_unary_f32: negative n") : PK_OK;
     if(!x || !y) return pk::fail("pk_unary_f32: NULL pointer");
-    unary_kernel<<<pk::grid_for(n, NT), NT, 0, pk::as_stream(stream)>>>(op, n, x, y);
+    hipStream_t st = pk::as_stream(stream);
+    const bool wide = wide_unary(n, x, y, nullptr);
+    const unsigned grid = pk::grid_for(wide ? n / 4 : n, NT);
+    switch(op) {
+#define PK_UNARY(OP)                                                      \
+    case OP:                                                              \
+        if(wide) unary_kernel<OP, 4><<<grid, NT, 0, st>>>(n, x, y);       \
+        else unary_kernel<OP, 1><<<grid, NT, 0, st>>>(n, x, y);           \
+        break;
+        PK_UNARY(0) PK_UNARY(1) PK_UNARY(2) PK_UNARY(3) PK_UNARY(4) PK_UNARY(5)
+#undef PK_UNARY
+    }
     return pk::launch_status("pk_unary_f32");
 }
 
@@ -1045,15 +1110,28 @@ extern "C" int pk_unary_bwd_f32(int op, int64_t n, const float* x, const float* 
     if(!valid_op(op, 5)) return pk::fail("pk_unary_bwd_f32: op %d not in 0..5", op);
     if(n <= 0) return n < 0 ? pk::fail("pk_unary_bwd_f32: negative n") : PK_OK;
     if(!x || !y || !gy || !gx) return pk::fail("pk_unary_bwd_f32: NULL pointer");
-    unary_bwd_kernel<<<pk::grid_for(n, NT), NT, 0, pk::as_stream(stream)>>>(op, n, x, y, gy, gx,
-                                                                           flags & PK_ACCUM);
+    hipStream_t st = pk::as_stream(stream);
+    const int accum = flags & PK_ACCUM;
+    const bool wide = wide_unary(n, op == 0 || op == 4 ? y : x, gy, gx);
+    const unsigned grid = pk::grid_for(wide ? n / 4 : n, NT);
+    switch(op) {
+#define PK_UNARY(OP)                                                                   \
+    case OP:                                                                           \
+        if(wide) unary_bwd_kernel<OP, 4><<<grid, NT, 0, st>>>(n, x, y, gy, gx, accum); \
+        else unary_bwd_kernel<OP, 1><<<grid, NT, 0, st>>>(n, x, y, gy, gx, accum);     \
+        break;
+        PK_UNARY(0) PK_UNARY(1) PK_UNARY(2) PK_UNARY(3) PK_UNARY(4) PK_UNARY(5)
+#undef PK_UNARY
+    }
     return pk::launch_status("pk_unary_bwd_f32");
 }
 
 extern "C" int pk_relu_f32(int64_t n, const float* x, float* y, pk_stream_t stream) {
     if(n <= 0) return n < 0 ? pk::fail("pk_relu_f32: negative n") : PK_OK;
     if(!x || !y) return pk::fail("pk_relu_f32: NULL pointer");
-    relu_kernel<<<pk::grid_for(n, NT), NT, 0, pk::as_stream(stream)>>>(n, x, y);
+    hipStream_t st = pk::as_stream(stream);
+    if(wide_unary(n, x, y, nullptr)) relu_kernel<4><<<pk::grid_for(n / 4, NT), NT, 0, st>>>(n, x, y);
+    else relu_kernel<1><<<pk::grid_for(n, NT), NT, 0, st>>>(n, x, y);
     return pk::launch_status("pk_relu_f32");
 }
 
@@ -1061,8 +1139,12 @@ extern "C" int pk_relu_bwd_f32(int64_t n, const float* y, const float* gy, float
                                pk_stream_t stream) {
     if(n <= 0) return n < 0 ? pk::fail("pk_relu_bwd_f32: negative n") : PK_OK;
     if(!y || !gy || !gx) return pk::fail("pk_relu_bwd_f32: NULL pointer");
-    relu_bwd_kernel<<<pk::grid_for(n, NT), NT, 0, pk::as_stream(stream)>>>(n, y, gy, gx,
-                                                                          flags & PK_ACCUM);
+    hipStream_t st = pk::as_stream(stream);
+    const int accum = flags & PK_ACCUM;
+    if(wide_unary(n, y, gy, gx))
+        relu_bwd_kernel<4><<<pk::grid_for(n / 4, NT), NT, 0, st>>>(n, y, gy, gx, accum);
+    else
+        relu_bwd_kernel<1><<<pk::grid_for(n, NT), NT, 0, st>>>(n, y, gy, gx, accum);
     return pk::launch_status("pk_relu_bwd_f32");
 }
 
