@@ -1,5 +1,5 @@
 // pico_amd/csrc/attention.hip -- causal self-attention forward and backward as
-// a chain of batched fp32 MFMA GEMMs and causal-softmax row kernels.
+// a chain of batched fp32 GEMMs and causal-softmax row kernels.
 //
 // Heads are addressed in place inside the token-major [B*T, H*hd] activations
 // (a two-level batch: outer stride T*ld per sequence, inner stride hd per
