@@ -192,10 +192,14 @@ __global__ __launch_bounds__(256, KS == 1 || HDT == 32 ? 2 : 1) void wide_fwd(Wi
     f32x16 o[NB];
 #pragma unroll
     for(int cb = 0; cb < NB; ++cb) o[cb] = splat16(0.0f);
-    float m = 0.0f, ls = 0.0f;
+    // m: the running max, raised when a block's max passes it by kTau; ref: what is
+    // subtracted, m or 0 while every score has been -inf
+    float m = -INFINITY, ref = 0.0f, ls = 0.0f;
     auto block = [&](int j, const float* __restrict__ tk, const float* __restrict__ tv) {
-        // scores against the running max m (log2 units)
-        f32x16 s = splat16(-m), s1 = splat16(0.0f);
+        // scores in log2 units.  ref is taken off the finished sum, 16 subtractions a
+        // block: as the sum's start it would absorb the scores of a row whose
+        // first keys lie far below the others
+        f32x16 s = splat16(0.0f), s1 = splat16(0.0f);
         const f32x4* a4 = reinterpret_cast<const f32x4*>(tk + lq * LDT + HDT / 2 * lh);
 #pragma unroll
         for(int i = 0; i < HDT / 8; ++i) {
@@ -214,23 +218,19 @@ __global__ __launch_bounds__(256, KS == 1 || HDT == 32 ? 2 : 1) void wide_fwd(Wi
             if(j == nw - 1 && acc_row(r, lh) > lq) s[r] = -INFINITY;  // the diagonal block
             mx = fmaxf(mx, s[r]);
         }
-        // a wave's first block sets m to its exact row max (its first key is visible
-        // to every query); later ones raise it when they exceed it by kTau
-        if(j < KS || __builtin_amdgcn_ballot_w64(mx > kTau)) {
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const float d = j < KS ? mx : fmaxf(mx, 0.0f);
-            const float alpha = __builtin_amdgcn_exp2f(-d);
+        if(__builtin_amdgcn_ballot_w64(mx > m + kTau)) {
+            mx = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32, 64)));
+            ref = mx == -INFINITY ? 0.0f : mx;
+            const float alpha = __builtin_amdgcn_exp2f(m - ref);
 #pragma unroll
-            for(int r = 0; r < 16; ++r) s[r] -= d;
-            if(j >= KS) {
+            for(int cb = 0; cb < NB; ++cb)
 #pragma unroll
-                for(int cb = 0; cb < NB; ++cb)
-#pragma unroll
-                    for(int r = 0; r < 16; ++r) o[cb][r] *= alpha;
-                ls *= alpha;
-            }
-            m += d;
+                for(int r = 0; r < 16; ++r) o[cb][r] *= alpha;
+            ls *= alpha;
+            m = mx;
         }
+#pragma unroll
+        for(int r = 0; r < 16; ++r) s[r] -= ref;
         float l0 = 0.0f, l1 = 0.0f;
 #pragma unroll
         for(int r = 0; r < 16; r += 2) {
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(256, KS == 1 || HDT == 32 ? 2 : 1) void wide_fwd(Wi
             for(int cb = 0; cb < NB; ++cb)
 #pragma unroll
                 for(int r = 0; r < 16; ++r) mine[(cb * 16 + r) * 64] = o[cb][r];
-            mine[NB * 16 * 64] = nw > 1 ? m : -INFINITY;
+            mine[NB * 16 * 64] = m;
             mine[(NB * 16 + 1) * 64] = ls;
         }
         __syncthreads();

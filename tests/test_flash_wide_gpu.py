@@ -152,3 +152,29 @@ def test_refusals(dev):
     assert L.pk_flash_wide_bwd_f32(1, 1, 64, 96, 96, 1.0, *([_ptr(x)] * 4), _ptr(lse), *([_ptr(x)] * 4),
                                    _ptr(x), 16, 0, None) == -1
     assert not L.pk_flash_wide_supported(64, 64) and L.pk_flash_wide_supported(1, 128)
+
+
+# leading keys (more than a block of them) that no later query sees: scores of -inf, and
+# scores next to which the others' would vanish.  The first 40 rows of the finite case
+# see equal keys only, so their probabilities are equal too
+@pytest.mark.parametrize("hd", [32, 96, 128])
+@pytest.mark.parametrize("B,H,T", [(2, 3, 200), (16, 16, 130)])
+@pytest.mark.parametrize("low", [float("-inf"), -1e30])
+def test_leading_keys_far_below_the_others(dev, hd, B, H, T, low):
+    g = torch.Generator(device=dev).manual_seed(T + hd)
+    D, n = H * hd, 40
+    q, k, v = (torch.randn(B * T, D, device=dev, generator=g) for _ in range(3))
+    q = q.abs() + 0.01
+    k.view(B, T, D)[:, :n] = low
+    o, lse = _fwd(B, H, T, hd, D, q, k, v)
+    x = [t.double().reshape(B, T, H, hd).transpose(1, 2).reshape(B * H, T, hd) for t in (q, k, v)]
+    s = torch.bmm(x[0][:, n:].contiguous(), x[1][:, n:].transpose(1, 2).contiguous()) * hd ** -0.5
+    s = s.masked_fill(~torch.ones(T - n, T - n, dtype=torch.bool, device=dev).tril(), float("-inf"))
+    heads = o.reshape(B, T, H, hd).transpose(1, 2).reshape(B * H, T, hd)
+    _close(heads[:, n:], torch.bmm(torch.softmax(s, -1), x[2][:, n:].contiguous()))
+    _close(lse.reshape(B * H, T)[:, n:], torch.logsumexp(s, -1))
+    if low > float("-inf"):
+        count = torch.arange(1, n + 1, device=dev)[:, None]
+        _close(heads[:, :n], x[2][:, :n].cumsum(1) / count)
+    else:
+        assert bool(torch.isnan(heads[:, :n]).all())
