@@ -18,6 +18,8 @@ SHAPES = [((31, 20), (20,)), ((32, 17), (17,)), ((65, 16), (16,)), ((513, 33), (
           ((600, 4097), (4097,)),
           ((20, 31), (20, 1)), ((17, 33), (17, 1)), ((5, 1030), (5, 1)), ((3, 2052), (3, 1)),
           ((8200, 40), (8200, 1)), ((4100, 513), (4100, 1)),
+          # one row of more than 64 workgroups; rows either side of 70 % of their lanes
+          ((500, 600), (1,)), ((90, 9), (9,)), ((90, 23), (90, 1)), ((90, 22), (22,)), ((9, 257), (9, 1)),
           ((37, 41), (1,)), ((1, 700), (1, 1)), ((6, 50, 7), (50, 7)), ((6, 50, 7), (6, 1, 1)),
           ((6, 50, 7), (50, 1)), ((4, 8, 64), (1, 8, 1)), ((3, 33, 2, 5), (33, 2, 1))]
 
