@@ -14,13 +14,19 @@
 //  * One group of waves per tile, so that every shape and epilogue adds K in the
 //    same order: the composed and fused operations agree bit for bit, and so do
 //    the split product here and on operands split beforehand.
-//  * Ragged sizes go through the buffer resources' own bounds, as there.
+//  * Ragged sizes go through the buffer resources' own bounds, as there; those of
+//    a row-contiguous operand, which cost a resource per k row, only in the last
+//    slices (bounded in every slice, scalar instructions were the bound: A^T.B
+//    of [192, 6464], K 1984, bf16 73 -> 41 us, [266, 1340], K 5136, A.B split 130 ->
+//    98).
 //
 // Bf16 against the four-wave kernel it replaces, us: 4096^3 A.B / A.B^T / A^T.B
 // 173 / 145 / 190 -> 166 / 136 / 175, [8192, 4096] K 768 87 -> 79.  Ragged:
 // [2000, 1503] K 1001 54 -> 26 (split bf16 64 -> 35), its A.B^T 73 -> 34 (77 ->
 // 38), [333, 517] K 1201 32 -> 16 (35 -> 18).  gemm.hip keeps that kernel for
 // the whole tiles where it is the faster one (narrow_here).
+#include <type_traits>
+
 #include "gemm_common.h"
 
 namespace {
@@ -92,23 +98,42 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_narrow_kernel(GemmPar
                                           : (p.K - 1) * p.ldb + p.N - job.col0)),
                                 BKF ? 4 : p.ldb * 4};
         const int64_t shift = p.pair_F - BN / 2;
+        // the slices before this one lie inside the operands with their whole
+        // tile rows: a row-contiguous operand's rows past its last one are read
+        // from the next k rows, `past` of them behind the end
+        // (a loop of their own, which the split-bf16 256x256 and A^T.B 128x128 tiles
+        // have no registers for)
+        constexpr bool TWO = EDGE == kPartial && !(AK && BKF) &&
+                             !(P == 2 && (TM * TN == 8 || (TM * TN == 2 && !AK)));
+        int inside = 0;
+        if constexpr(TWO) {
+            auto past = [](int64_t over, int64_t ld) {
+                return over > 0 ? (int)(((unsigned)over + (unsigned)ld - 1) / (unsigned)ld) : 0;
+            };
+            const int pa = AK ? 0 : past(job.row0 + BM - p.M, p.lda);
+            const int pb = BKF ? 0 : past(job.col0 + BN + (PAIR ? shift : 0) - p.N, p.ldb);
+            inside = (int)(max(min(job.kend, p.K - max(pa, pb)) - job.kbeg, (int64_t)0) / W);
+        }
         float ra[OA::ITEMS][OA::KPI], rb[OB::ITEMS][OB::KPI];
-        auto load = [&](int s) {
+        // (TAIL: slices from `inside` on)
+        auto load = [&](int s, auto tail) {
+            constexpr bool TAIL = decltype(tail)::value;
             const int64_t k0 = job.kbeg + (int64_t)min(s, nslices - 1) * W;
             if constexpr(EDGE == kFar) {
                 far_load<AK, BM, NT_, false>(job.A, p.lda, job.row0, p.M, k0, job.kend, 0, ra);
                 far_load<BKF, BN, NT_, PAIR>(job.B, p.ldb, job.col0, p.N, k0, job.kend, shift, rb);
             } else {
-                split_load<AK, EDGE == kPartial, BM, NT_, false, W>(sa, p.lda, k0, 0, ra);
-                split_load<BKF, EDGE == kPartial, BN, NT_, PAIR, W>(sb, p.ldb, k0, shift, rb);
+                constexpr bool EA = EDGE == kPartial && (AK || TAIL), EB = EDGE == kPartial && (BKF || TAIL);
+                split_load<AK, EA, BM, NT_, false, W>(sa, p.lda, k0, 0, ra);
+                split_load<BKF, EB, BN, NT_, PAIR, W>(sb, p.ldb, k0, shift, rb);
             }
         };
         auto store = [&](int stage) {
             split_store<P, AK, BM, NT_, PART, W>(lds + stage * STAGE, ra, 1.0f);
             split_store<P, BKF, BN, NT_, PART, W>(lds + stage * STAGE + BM * SK, rb, 1.0f);
         };
-        auto mask = [&](int s) {
-            if constexpr(EDGE == kPartial && (AK || BKF)) {
+        auto mask = [&](int s, auto tail) {
+            if constexpr(decltype(tail)::value && EDGE == kPartial && (AK || BKF)) {
                 const int64_t limit = job.kend - job.kbeg - (int64_t)min(s, nslices - 1) * W;
                 if(limit < W) {
                     if(AK) split_mask<AK, BM, NT_, W>((int)limit, ra);
@@ -134,10 +159,11 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_narrow_kernel(GemmPar
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.a[i], y.b[j], acc[i][j], 0,
                                                                         0, 0);
         };
-        load(0);
-        mask(0);
+        using Bounded = std::integral_constant<bool, EDGE != kWhole>;
+        load(0, Bounded());
+        mask(0, Bounded());
         store(0);
-        load(1);
+        load(1, Bounded());
         __syncthreads();
         SplitFrag<TM, TN> h0, h1, lo;
         read(h0, 0, 0, 0);
@@ -145,14 +171,13 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_narrow_kernel(GemmPar
         constexpr int CV = (OA::ITEMS * OA::KPI + OB::ITEMS * OB::KPI) * (P == 2 ? 7 : 1) / 2;
         constexpr int WR = P * (OA::ITEMS + OB::ITEMS);
         constexpr int LD = OA::ITEMS * OA::LOADS + OB::ITEMS * OB::LOADS;
-#pragma unroll 1
-        for(int s = 0; s < nslices; ++s) {
+        auto slice = [&](int s, auto tail) {
             const int cur = s & 1;
-            mask(s + 1);
+            mask(s + 1, tail);
             if constexpr(P == 2) read(lo, cur, 0, 1);
             read(h1, cur, 1, 0);
             store(cur ^ 1);
-            load(s + 2);
+            load(s + 2, tail);
             mma(h0, h0);
             if constexpr(P == 2) {
                 mma(h0, lo);
@@ -173,7 +198,14 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_narrow_kernel(GemmPar
             else mma(h1, h1);
             split_sched<NB, RD, 0, 0, 0>();
             __builtin_amdgcn_sched_barrier(0);
+        };
+        int s = 0;
+        if constexpr(TWO) {
+#pragma unroll 1
+            for(; s + 2 < inside; ++s) slice(s, std::false_type());
         }
+#pragma unroll 1
+        for(; s < nslices; ++s) slice(s, Bounded());
     }
     if constexpr(EPI == kEpiPlain)
         store_tile<EDGE == kWhole ? kEdgeNone : kEdgeScalar, TM, TN, 1>(p, job, acc, ar0, br0, lr, lh, 0);

@@ -106,13 +106,14 @@ __device__ __forceinline__ void split_load(const SplitSource& src, int64_t ld, i
                                                      [SplitOperand<KFAST, R, THREADS, W>::KPI]) {
     using O = SplitOperand<KFAST, R, THREADS, W>;
     const int64_t off = k0 * src.kstep;
-    // the operand from `skip` bytes past the slice's first value on
-    auto rest = [&](int64_t skip) {
-        const int64_t left = src.left - off - skip;
-        const unsigned num = EDGE ? (left <= 0 ? 0u : left > 0xfffffff0ll ? 0xfffffff0u : (unsigned)left)
-                                  : 0xfffffff0u;
+    // (2^31 - 1 at most, which no offset of a slice reaches, so that taking k rows
+    // off it stays a 32-bit subtraction)
+    const int num = EDGE ? (int)min(max(src.left - off, (int64_t)0), (int64_t)INT32_MAX) : -16;
+    // the operand from k row t of the slice on
+    auto rest = [&](int t) {
+        const int skip = t * (int)src.kstep;
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(src.base + off + skip), (short)0,
-                                                 (int)num, 0x00020000);
+                                                 EDGE ? max(num - skip, 0) : num, 0x00020000);
     };
     const __amdgpu_buffer_rsrc_t rs = rest(0);
 #pragma unroll
@@ -130,8 +131,9 @@ __device__ __forceinline__ void split_load(const SplitSource& src, int64_t ld, i
             // whole tiles reach their k rows by the scalar offset; bounded loads do
             // not, as only the vector offset is sure to be checked.  Slices of 16 k
             // add it up anew each time (kept over the loop, the offsets spill in
-            // 256-row tiles), those of 32 k, with no vector register to spare, take
-            // a resource per k row (which would spill scalar registers in the other)
+            // 256-row tiles), those of 32 k, with no vector register to spare and
+            // few bounded slices, take a resource per k row (which would spill
+            // scalar registers in the other)
             unsigned voff = (kk * (unsigned)ld + row) * 4u;
             const unsigned step = (unsigned)ld * 4u;
             if(EDGE && W == SK) asm volatile("" : "+v"(voff));
@@ -143,7 +145,7 @@ __device__ __forceinline__ void split_load(const SplitSource& src, int64_t ld, i
                 else if(W == SK)
                     x = __builtin_amdgcn_raw_buffer_load_b32(rs, (int)(voff + t * step), 0, 0);
                 else
-                    x = __builtin_amdgcn_raw_buffer_load_b32(rest(t * src.kstep), (int)voff, 0, 0);
+                    x = __builtin_amdgcn_raw_buffer_load_b32(rest(t), (int)voff, 0, 0);
                 v[i][t] = __builtin_bit_cast(float, x);
             }
         }

@@ -46,7 +46,10 @@ def _inside(x):
 @pytest.mark.parametrize("M,N,Kd", [(4096, 4096, 64), (4095, 4097, 41), (2048, 2048, 96),
                                     (2047, 2049, 15), (8192, 768, 32), (8190, 768, 33),
                                     (1024, 1024, 160), (1023, 1021, 31), (515, 2047, 1),
-                                    (5, 3, 127), (768, 768, 4096), (517, 301, 3001)])
+                                    (5, 3, 127), (768, 768, 4096), (517, 301, 3001),
+                                    # many slices inside the operands, then the bounded ones; rows
+                                    # so short that a tile runs over several k rows
+                                    (2049, 2047, 500), (8, 700, 303), (700, 6, 300), (200, 72, 97)])
 def test_products_at_tile_edges(dev, kind, ta, tb, M, N, Kd):
     g = torch.Generator(device=dev).manual_seed(M + N + Kd)
     A = torch.randn(M, Kd, device=dev, generator=g)
