@@ -38,6 +38,7 @@
 #include <stdio.h>
 
 #include <algorithm>
+#include <iterator>
 #include <mutex>
 #include <type_traits>
 
@@ -1046,44 +1047,49 @@ int choose_splits(int64_t M, int64_t N, int64_t K, bool ta, bool fp32, int64_t* 
 
 enum Precision { kFp32 = 0, kBf16 = 1, kBf16x3 = 2, kFp8 = 3 };
 
-// fp32 products (gemm_split.h): tile shape and K split together, by the
-// estimated time of the busiest CU -- its workgroups, ceil(tiles * splits / 256
-// CUs), each `per_k` per k of its range plus `fixed` for its prologue and
-// epilogue -- plus, for a split, a read of every partial plane and a write at
-// 5 TB/s and a launch.  Measured in microseconds on whole tiles (each shape
-// where it fills the CUs once: 4096^3 on 256x256, [8192, 768] K 32000 on 256x96,
-// 2048^3 on 128x128, [4096, 512] K 8192 on 128x64, [768, 768] K 8192 on 64x64),
-// fixed from the same at K 512-1024.  Over 45 shapes of a transformer step,
-// squares and ragged sizes the pick ran within 8 % of the best shape timed.
-// Examples: 4096^2 -> 256x256; [8192, 768] and [8192, 2304] -> 256x96;
-// 2048^2 -> 128x128; [4096, 512] -> 128x64; 1024^2 -> 64x64; the weight gradient
-// [768, 768] K 8192 -> 128x128 in 7 splits, [768, 2304] 256x256 in 9.
+// fp32 products (gemm_split.h), bf16 and split-bf16 ones (gemm_narrow.hip, or the
+// kernel of this file): tile shape and K split together, by the shortest
+// estimated time.  Of a shape, in microseconds for k of a workgroup's range,
+//     max(one + one_k * k, base + rounds * (round + per_k * k))
+// the first for a CU with one workgroup, bound by its latency, the second for
+// CUs that overlap several; `edge` more for one and for each round of ragged
+// tiles (or K), per_k and one_k `ta` times as long for A^T.B.  rounds is the mean
+// of tiles * splits / 256 CUs and of its ceiling (320 tiles take 1.6 times what 256
+// do: the CUs with a second tile run it faster than two).  A split adds a
+// launch, a step per partial plane in the reduction's chain (longer where
+// N % 4 leaves it scalar) and the planes' traffic.
+//
+// The constants are fits to about 6500 times: 64 to 2048 tiles of every shape, K 3
+// to 2048, three layouts, whole and ragged, root mean square error 4-11 %.  Over
+// 586 random and transformer shapes with every shape and split timed, the pick
+// ran within 0.7 % (fp32), 2.1 % (bf16) and 0.8 % (split bf16) of the best on average.
+// One time per k and round with a fixed part, which stood here before, ran
+// within 2.6 %, 5.7 % and 2.3 %, and far off at K below 256: [1184, 448] K 32 fp32
+// 8.4 us (now 5.2), [1344, 3712] K 64 19.6 (10.8), [7680, 1344] K 96 35 (22); bf16
+// [4096, 1376] A^T.B K 512 37 (30).
+// 96-column tiles take no split but in fp32.
 struct SplitShape {
     TileKind kind;
     int bm, bn;
-    double per_k, fixed;
+    double one, one_k, base, round, per_k, edge, ta;
 };
-constexpr SplitShape kSplitShapes[5] = {{kTile128, 128, 128, 0.0400, 4.0},
-                                        {kTile256, 256, 256, 0.1370, 11.0},
-                                        {kTile256x96, 256, 96, 0.0610, 6.5},
-                                        {kTile128x64, 128, 64, 0.0252, 3.5},
-                                        {kTile64, 64, 64, 0.0145, 3.0}};
-// The same for bf16 and split-bf16 multiplies: 4096^3 takes 256x256, [8192, 768]
-// 256x96, [4096, 768] 128x96, 2048^3 128x128, 1024^3 64x64.  A split keeps to
-// 256x256, 128x128 and 64x64, and A^T.B to those altogether, whose operand
-// traffic the 96-column tiles double: the gradient [768, 4096] with K 8192 runs
-// in 4 splits of 256x256 (bf16 130 -> 97 us, split bf16 200 -> 164, in 8 of
-// 128x128 before), [768, 2304] in 8 (107 -> 80, 127 -> 98).
-constexpr SplitShape kNarrowShapes[2][5] = {{{kTile128, 128, 128, 0.0160, 2.5},
-                                             {kTile256, 256, 256, 0.0430, 8.0},
-                                             {kTile256x96, 256, 96, 0.0205, 3.5},
-                                             {kTile96, 128, 96, 0.0125, 2.5},
-                                             {kTile64, 64, 64, 0.0075, 2.5}},
-                                            {{kTile128, 128, 128, 0.0285, 2.5},
-                                             {kTile256, 256, 256, 0.0840, 11.0},
-                                             {kTile256x96, 256, 96, 0.0385, 4.0},
-                                             {kTile96, 128, 96, 0.0215, 2.5},
-                                             {kTile64, 64, 64, 0.0115, 2.5}}};
+constexpr SplitShape kShapesF32[] = {{kTile128, 128, 128, 6.7, 0.0280, 4.8, 4.1, 0.0391, 2.9, 1.04},
+                                     {kTile256, 256, 256, 10.6, 0.1023, 2.3, 12.0, 0.1370, 7.2, 1.00},
+                                     {kTile256x96, 256, 96, 6.3, 0.0477, 6.1, 4.5, 0.0586, 4.1, 1.07},
+                                     {kTile128x64, 128, 64, 4.9, 0.0220, 5.3, 1.2, 0.0229, 1.6, 1.06},
+                                     {kTile64, 64, 64, 6.1, 0.0106, 3.4, 3.3, 0.0126, 2.7, 1.08},
+                                     {kTile64x2, 64, 64, 4.5, 0.0154, 5.4, 0.31, 0.0137, 1.4, 1.05},
+                                     {kTile64x1, 64, 64, 4.0, 0.0262, 4.9, 0.12, 0.0150, 0.8, 1.02}};
+constexpr SplitShape kShapesBf16[] = {{kTile128, 128, 128, 5.5, 0.0161, 5.7, 1.8, 0.0133, 1.0, 1.18},
+                                      {kTile256, 256, 256, 9.5, 0.0299, 1.3, 13.3, 0.0332, 4.2, 1.14},
+                                      {kTile256x96, 256, 96, 7.2, 0.0205, 5.8, 3.3, 0.0159, 0.0, 1.42},
+                                      {kTile96, 128, 96, 4.9, 0.0146, 5.1, 1.5, 0.0096, 0.0, 1.46},
+                                      {kTile64, 64, 64, 3.8, 0.0101, 4.4, 0.20, 0.0061, 1.0, 1.25}};
+constexpr SplitShape kShapesBf16x3[] = {{kTile128, 128, 128, 6.3, 0.0275, 6.0, 2.0, 0.0238, 0.7, 1.13},
+                                        {kTile256, 256, 256, 12.4, 0.0621, 3.3, 13.6, 0.0737, 3.4, 1.06},
+                                        {kTile256x96, 256, 96, 7.2, 0.0322, 4.9, 4.6, 0.0357, 0.0, 1.32},
+                                        {kTile96, 128, 96, 5.2, 0.0239, 5.1, 1.6, 0.0192, 0.0, 1.17},
+                                        {kTile64, 64, 64, 4.1, 0.0167, 4.6, 0.25, 0.0090, 0.9, 1.19}};
 
 // Whether a whole-tile bf16 or split-bf16 product runs on the four-wave kernel
 // of this file rather than gemm_narrow.hip's: the 96-column tiles (64x96 per
@@ -1110,7 +1116,6 @@ constexpr size_t kNoAllocScratchBytes = (size_t)128 << 20;
 SplitPlan plan_split(int prec, int64_t M, int64_t N, int64_t K, int64_t batch, bool allow_all,
                      bool ta, bool allow_split, bool allow_96 = true) {
     const bool fp32 = prec == kFp32;
-    const SplitShape* const shapes = fp32 ? kSplitShapes : kNarrowShapes[prec - kBf16];
     SplitPlan best = {{kTile128, 128, 128}, 1, K};
     double c = -1.0;
     int s_max = 1;
@@ -1123,26 +1128,34 @@ SplitPlan plan_split(int prec, int64_t M, int64_t N, int64_t K, int64_t batch, b
             if((size_t)old * M * N * sizeof(float) <= kNoAllocScratchBytes) cap = kNoAllocScratchBytes;
         }
     }
-    const double plane = (double)M * (double)N * 4.0 / 5e6;
+    const double plane = (double)M * (double)N * 4.0 / 6.7e6, link = N % 4 ? 1.1 : 0.3;
     // (a few dozen counts and 32-bit divisions: this runs on the host for every
     // product, and all 64 counts in 64-bit took 10 us)
     static constexpr int kCounts[] = {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 14, 16, 18, 21, 24, 28, 32, 40, 48, 64};
     const uint32_t k32 = (uint32_t)std::min<int64_t>(K, (int64_t)1 << 30);
-    for(int i = 0; i < 5; ++i) {
+    const SplitShape* const shapes = fp32 ? kShapesF32 : prec == kBf16 ? kShapesBf16 : kShapesBf16x3;
+    const int n_shapes = fp32 ? (int)std::size(kShapesF32) : (int)std::size(kShapesBf16);
+    static_assert(std::size(kShapesBf16) == std::size(kShapesBf16x3), "one count for both");
+    for(int i = 0; i < n_shapes; ++i) {
         const SplitShape& t = shapes[i];
         const bool n96 = t.bn == 96;
         if(!allow_all && t.kind != kTile128) continue;
-        if(n96 && (N % 96 != 0 || (!fp32 && (ta || !allow_96 || M % t.bm != 0)))) continue;
+        if(n96 && (N % 96 != 0 || (!fp32 && (!allow_96 || M % t.bm != 0)))) continue;
         const int64_t tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * batch;
         const uint32_t step = fp32 ? 32 * split_groups(t.kind) : 32;
+        const bool whole = M % t.bm == 0 && N % t.bn == 0 && K % step == 0;
+        const double edge = whole ? 0.0 : t.edge, ta_k = ta ? t.ta : 1.0;
         for(const int s : kCounts) {
             if(s > (n96 && !fp32 ? 1 : s_max)) break;
             const uint32_t chunk = s == 1 ? k32 : ((k32 + s - 1) / s + step - 1) / step * step;
             const uint32_t splits = s == 1 ? 1 : (k32 + chunk - 1) / chunk;
             if(splits > 1 && (size_t)splits * M * N * sizeof(float) > cap) break;
-            const int64_t rounds = (tiles * splits + kCUs - 1) / kCUs;
-            const double ck = (double)rounds * (t.per_k * (double)chunk + t.fixed) +
-                              (splits > 1 ? (double)(splits + 1) * plane + 3.0 : 0.0);
+            const int64_t n = tiles * splits;
+            const double k = ta_k * (double)chunk,
+                         rounds = 0.5 * ((double)((n + kCUs - 1) / kCUs) + (double)n / kCUs);
+            const double ck = std::max(t.one + edge + t.one_k * k,
+                                       t.base + rounds * (t.round + edge + t.per_k * k)) +
+                              (splits > 1 ? 0.5 + link * splits + (splits + 1) * plane : 0.0);
             if(c < 0.0 || ck < c) {
                 c = ck;
                 best = {{t.kind, t.bm, t.bn}, (int)splits, splits == 1 ? K : (int64_t)chunk};
@@ -1485,15 +1498,15 @@ static size_t gemm_workspace(int prec, int64_t M, int64_t N, int64_t K, bool ta)
     return S > 1 ? (size_t)S * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
-// any layout (A^T.B splits whenever another layout of the shape does) and any
-// precision: fp8 splits by choose_splits alone
+// any layout (A^T.B splits whenever another layout of the shape does, into more
+// or fewer ranges) and any precision: fp8 splits by choose_splits alone
 extern "C" size_t pk_gemm_workspace_f32(int64_t M, int64_t N, int64_t K) {
     if(M <= 0 || N <= 0 || K <= 0) return 0;
     int64_t kchunk;
     const int S = choose_splits(M, N, K, true, true, &kchunk);
     size_t most = S > 1 ? (size_t)S * (size_t)M * (size_t)N * sizeof(float) : 0;
     for(const int prec : {kFp32, kBf16, kBf16x3})
-        most = std::max(most, gemm_workspace(prec, M, N, K, true));
+        for(const bool ta : {false, true}) most = std::max(most, gemm_workspace(prec, M, N, K, ta));
     return most;
 }
 

@@ -293,9 +293,9 @@ __device__ __forceinline__ void staged_epilogue(const GemmParams& p, const TileJ
     }
 }
 
-// (128x96 tiles: fp8 only; 128x64: fp32 only)
-enum TileKind { kTile128, kTile96, kTile256, kTile64, kTile256x96, kTile128x64 };
-
+// (128x96 tiles: not for fp32; 128x64 and 64x64 tiles of two and one wave groups:
+// fp32 only)
+enum TileKind { kTile128, kTile96, kTile256, kTile64, kTile256x96, kTile128x64, kTile64x2, kTile64x1 };
 
 // the fp32 product (gemm_split.hip): K groups a shape's workgroups split K into,
 // and the launch

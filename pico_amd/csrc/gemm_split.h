@@ -53,10 +53,13 @@
 // 4096^3 A.B / A.B^T / A^T.B 244-246 TFLOP/s (149 on the fp32 cores), 8192^3
 // 237-243 (151), 2048^3 188-193 (142), 1024^3 114-117 (105-115).
 
-// A tile shape: WM x WN waves, each TM x TN blocks of 32 x 32; WPS waves per SIMD.
-template <int WM_, int WN_, int TM_, int TN_, int G_, int WPS_, int PF_>
+// A tile shape: WM x WN waves, each TM x TN blocks of 32 x 32; WPS waves per SIMD;
+// G groups of them, each with A sets of sums (slice s of K goes to group s % G and
+// there to set s / G % A).
+template <int WM_, int WN_, int TM_, int TN_, int G_, int WPS_, int PF_, int A_ = 1>
 struct SplitTile {
-    static constexpr int WGM = WM_, WGN = WN_, TM = TM_, TN = TN_, G = G_;
+    static constexpr int WGM = WM_, WGN = WN_, TM = TM_, TN = TN_, G = G_, A = A_;
+    static_assert(A_ == 1 || (TM_ * TN_ == 1 && PF_ == 1), "one block to a wave");
     static constexpr int WPS = WPS_, PF = PF_;
     static constexpr int BM = WM_ * TM_ * 32, BN = WN_ * TN_ * 32;
     static constexpr int WAVES = WM_ * WN_;                    // of one K group
@@ -299,7 +302,8 @@ __device__ __forceinline__ void split_sched() {
 
 template <bool TA, bool TB, bool EDGE, class T, int EPI>
 __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmParams p) {
-    constexpr int BM = T::BM, BN = T::BN, TM = T::TM, TN = T::TN, NT_ = T::GTHREADS, G = T::G;
+    constexpr int BM = T::BM, BN = T::BN, TM = T::TM, TN = T::TN, NT_ = T::GTHREADS, G = T::G,
+                  SETS = T::A;
     constexpr bool AK = !TA, BKF = TB, PAIR = EPI == kEpiSwigluFwd;
     using OA = SplitOperand<AK, BM, NT_>;
     using OB = SplitOperand<BKF, BN, NT_>;
@@ -314,20 +318,25 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmPara
     const int lr = l & 31, lh = l >> 5;
     const int ar0 = wm * TM * 32, br0 = wn * TN * 32;
     short* const lds = lds_all + g * 2 * STAGE;
-    // slices per group, an even number
+    // slices per group, an even number unless one group has several sets of sums
+    constexpr int STEP = G == 1 && SETS > 1 ? 1 : 2;
     const int nslices =
-        p.exact_only ? 0 : (int)((job.kend - job.kbeg + 2 * G * SK - 1) / (2 * G * SK)) * 2;
+        p.exact_only ? 0 : (int)((job.kend - job.kbeg + STEP * G * SK - 1) / (STEP * G * SK)) * STEP;
 
-    f32x16 acc[TM][TN];
+    f32x16 acc[TM][TN], more[SETS > 1 ? SETS - 1 : 1];  // the first set, the others
 #pragma unroll
     for(int i = 0; i < TM; ++i)
 #pragma unroll
         for(int j = 0; j < TN; ++j)
 #pragma unroll
             for(int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+#pragma unroll
+    for(int i = 0; i + 1 < SETS; ++i) more[i] = acc[0][0];
 
-    // the scale of op(A)'s parts, whose sign the sums share
+    // the scale of op(A)'s parts, whose sign the sums share: one sign to a group,
+    // or to a set of sums
     float scale = G > 1 && (g & 1) ? -0x1p16f : 0x1p16f;
+    auto set_sign = [&](int a) { return G == 1 && (a & 1) ? -1.0f : 1.0f; };
     if(nslices > 0) {
         const SplitSource sa = {reinterpret_cast<const char*>(job.A + (AK ? job.row0 * p.lda : job.row0)),
                                 4 * ((AK ? (p.M - 1 - job.row0) * p.lda + p.K
@@ -373,13 +382,12 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmPara
             for(int j = 0; j < TN; ++j)
                 f.b[j] = *reinterpret_cast<const bf16x8*>(t + (BM + br0 + j * 32) * SK);
         };
-        auto mma = [&](const SplitFrag<TM, TN>& x, const SplitFrag<TM, TN>& y) {
+        auto mma = [&](f32x16 (&c)[TM][TN], const SplitFrag<TM, TN>& x, const SplitFrag<TM, TN>& y) {
 #pragma unroll
             for(int i = 0; i < TM; ++i)
 #pragma unroll
                 for(int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.a[i], y.b[j], acc[i][j], 0,
-                                                                        0, 0);
+                    c[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.a[i], y.b[j], c[i][j], 0, 0, 0);
         };
         load(r0, 0);
         mask(r0, 0);
@@ -394,56 +402,82 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmPara
         constexpr int CV = (OA::ITEMS * OA::KPI + OB::ITEMS * OB::KPI) * 13 / 2;
         constexpr int WR = 3 * (OA::ITEMS + OB::ITEMS);
         constexpr int LD = OA::ITEMS * OA::LOADS + OB::ITEMS * OB::LOADS;
+        // scale_a: of the next slice, which is split here
         auto slice = [&](int s, int cur, float scale_a, Regs& r, SplitFrag<TM, TN>& h,
-                         SplitFrag<TM, TN>& q) {
+                         SplitFrag<TM, TN>& q, f32x16 (&c)[TM][TN]) {
             mask(r, s + 1);
             read(q, cur, 2);
             store(r, cur ^ 1, scale_a);
             load(r, s + 1 + PF);
-            mma(m, m);
-            mma(m, h);
-            mma(h, m);
+            mma(c, m, m);
+            mma(c, m, h);
+            mma(c, h, m);
             split_sched<3 * NB, RD, CV, WR, LD>();
             __builtin_amdgcn_sched_barrier(0);
             __syncthreads();
             read(m, cur ^ 1, 1);
-            mma(h, q);
-            mma(q, h);
+            mma(c, h, q);
+            mma(c, q, h);
             split_sched<2 * NB, RD, 0, 0, 0>();
             __builtin_amdgcn_sched_barrier(0);
             read(q, cur ^ 1, 0);
-            mma(h, h);
+            mma(c, h, h);
             split_sched<NB, RD, 0, 0, 0>();
             __builtin_amdgcn_sched_barrier(0);
         };
-        int flip = 4;
+        if constexpr(SETS > 1) {
+            auto set = [&](int a) -> f32x16(&)[TM][TN] {
+                return a == 0 ? acc : reinterpret_cast<f32x16(&)[TM][TN]>(more[a - 1]);
+            };
 #pragma unroll 1
-        for(int s = 0; s < nslices; s += 2) {
-            slice(s, 0, scale, PF == 2 ? r1 : r0, f0, f1);
-            const bool turn = G == 1 && s + 2 == flip;
-            if(turn) scale = -scale;
-            slice(s + 1, 1, scale, r0, f1, f0);
-            if(turn) {
-                flip += 8;
+            for(int s = 0; s < nslices; s += SETS) {
 #pragma unroll
-                for(int i = 0; i < TM; ++i)
+                for(int a = 0; a < SETS; ++a) {
+                    if(a % STEP == 0 && a > 0 && s + a >= nslices) break;
+                    slice(s + a, a & 1, scale * set_sign(a + 1), r0, a & 1 ? f1 : f0,
+                          a & 1 ? f0 : f1, set(a));
+                }
+            }
+        } else {
+            int flip = 4;
+#pragma unroll 1
+            for(int s = 0; s < nslices; s += 2) {
+                slice(s, 0, scale, PF == 2 ? r1 : r0, f0, f1, acc);
+                const bool turn = G == 1 && s + 2 == flip;
+                if(turn) scale = -scale;
+                slice(s + 1, 1, scale, r0, f1, f0, acc);
+                if(turn) {
+                    flip += 8;
 #pragma unroll
-                    for(int j = 0; j < TN; ++j) acc[i][j] = -acc[i][j];
+                    for(int i = 0; i < TM; ++i)
+#pragma unroll
+                        for(int j = 0; j < TN; ++j) acc[i][j] = -acc[i][j];
+                }
             }
         }
     }
     const float unscale = scale * 0x1p-48f;
-    if constexpr(G > 1) {
-        // the groups' sums meet in LDS: group b % G finishes block b, adding in
-        // group order
+    // every set of every group is scaled back, and they are added in the order of
+    // their first slices, so the tile shapes that deal K to four sums agree bit
+    // for bit
+    if constexpr(G > 1 || SETS > 1) {
 #pragma unroll
         for(int i = 0; i < TM; ++i)
 #pragma unroll
             for(int j = 0; j < TN; ++j) acc[i][j] *= unscale;
+#pragma unroll
+        for(int a = 1; a < SETS; ++a) {
+            more[a - 1] *= unscale * set_sign(a);
+            if(G == 1) acc[0][0] += more[a - 1];
+        }
+    }
+    if constexpr(G > 1) {
+        // the groups' sums meet in LDS: group b % G finishes block b, adding in
+        // group order
         f32x4* red = reinterpret_cast<f32x4*>(lds_all);
-        constexpr int BLK = T::WAVES * TM * TN * 4 * 64;  // f32x4 of one group's tile
-        auto slot = [&](int from, int b, int r) {
-            return ((from * T::WAVES + w) * TM * TN + b) * 4 * 64 + r * 64 + l;
+        constexpr int BLK = T::WAVES * TM * TN * SETS * 4 * 64;  // f32x4 of one group's tile
+        auto slot = [&](int from, int b, int a, int r) {
+            return (((from * T::WAVES + w) * TM * TN + b) * SETS + a) * 4 * 64 + r * 64 + l;
         };
         static_assert((G - 1) * BLK * 16 <= (int)sizeof(lds_all), "partial tiles fit");
         __syncthreads();
@@ -453,10 +487,12 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmPara
             if(g != owner) {
                 const int from = (g - owner + G) % G - 1;
 #pragma unroll
-                for(int r = 0; r < 4; ++r) {
-                    f32x16& a = acc[b / TN][b % TN];
-                    red[slot(from, b, r)] = f32x4{a[4 * r], a[4 * r + 1], a[4 * r + 2], a[4 * r + 3]};
-                }
+                for(int a = 0; a < SETS; ++a)
+#pragma unroll
+                    for(int r = 0; r < 4; ++r) {
+                        const f32x16& x = a == 0 ? acc[b / TN][b % TN] : more[a - 1];
+                        red[slot(from, b, a, r)] = f32x4{x[4 * r], x[4 * r + 1], x[4 * r + 2], x[4 * r + 3]};
+                    }
             }
         }
         __syncthreads();
@@ -464,13 +500,17 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmPara
         for(int b = 0; b < TM * TN; ++b) {
             if(g == b % G) {
 #pragma unroll
-                for(int from = 0; from < G - 1; ++from)
+                for(int a = 0; a < SETS; ++a) {
+                    if(a > 0) acc[0][0] += more[a - 1];
 #pragma unroll
-                    for(int r = 0; r < 4; ++r) {
-                        const f32x4 x = red[slot(from, b, r)];
+                    for(int from = 0; from < G - 1; ++from)
 #pragma unroll
-                        for(int e = 0; e < 4; ++e) acc[b / TN][b % TN][4 * r + e] += x[e];
-                    }
+                        for(int r = 0; r < 4; ++r) {
+                            const f32x4 x = red[slot(from, b, a, r)];
+#pragma unroll
+                            for(int e = 0; e < 4; ++e) acc[b / TN][b % TN][4 * r + e] += x[e];
+                        }
+                }
             }
         }
     }
@@ -482,7 +522,7 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmPara
             if(G == 1 || g == (i * TN + j) % G)
 #pragma unroll
             for(int r = 0; r < 16; ++r) {
-                if(G == 1) acc[i][j][r] *= unscale;
+                if(G == 1 && SETS == 1) acc[i][j][r] *= unscale;
                 sum = fmaf(acc[i][j][r], 0.0f, sum);
             }
     if(p.exact_only || __any(sum != 0.0f))

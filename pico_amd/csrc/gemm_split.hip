@@ -13,6 +13,8 @@ using Split128 = SplitTile<2, 4, 2, 1, 2, 4, 1>;
 using Split256x96 = SplitTile<4, 1, 2, 3, 2, 2, 1>;
 using Split128x64 = SplitTile<2, 2, 2, 1, 2, 4, 1>;
 using Split64 = SplitTile<2, 2, 1, 1, 4, 4, 2>;
+using Split64x2 = SplitTile<2, 2, 1, 1, 2, 4, 1, 2>;
+using Split64x1 = SplitTile<2, 2, 1, 1, 1, 4, 1, 4>;
 
 template <bool TA, bool TB, bool EDGE, class T>
 void launch_split_kernel(const GemmParams& gp, dim3 grid, hipStream_t st) {
@@ -52,6 +54,8 @@ int launch_layout(const GemmParams& gp, int64_t batch, bool edge, TileKind kind,
     case kTile256x96: return launch_split_tile<TA, TB, Split256x96>(gp, batch, edge, st);
     case kTile128x64: return launch_split_tile<TA, TB, Split128x64>(gp, batch, edge, st);
     case kTile64: return launch_split_tile<TA, TB, Split64>(gp, batch, edge, st);
+    case kTile64x2: return launch_split_tile<TA, TB, Split64x2>(gp, batch, edge, st);
+    case kTile64x1: return launch_split_tile<TA, TB, Split64x1>(gp, batch, edge, st);
     default: return launch_split_tile<TA, TB, Split128>(gp, batch, edge, st);
     }
 }
@@ -61,7 +65,7 @@ int launch_layout(const GemmParams& gp, int64_t batch, bool edge, TileKind kind,
 namespace pkg {
 
 int split_groups(TileKind kind) {
-    return kind == kTile64 ? Split64::G : kind == kTile256 ? Split256::G : 2;
+    return kind == kTile64 ? Split64::G : kind == kTile256 || kind == kTile64x1 ? 1 : 2;
 }
 
 int launch_split(bool ta, bool tb, const GemmParams& gp, int64_t batch, bool edge, TileKind kind,

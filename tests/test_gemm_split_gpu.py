@@ -31,13 +31,16 @@ def _within_bound(C, A, B):
     return bool((err <= (1.5 * A.shape[1] + 8) * 2.0 ** -24 * (a.abs() @ b.abs())).all())
 
 
-# whole and ragged sizes of every tile: 256 x 256, 128 x 128, 256 x 96, 128 x 96, 64 x 64; K of a
+# whole and ragged sizes of every tile: 256 x 256, 128 x 128, 256 x 96, 64 x 64; K of a
 # part of a slice, one slice, an odd number of slices, and past a sign change of the sums
 @pytest.mark.parametrize("ta,tb", [("N", "N"), ("N", "T"), ("T", "N"), ("T", "T")])
 @pytest.mark.parametrize("M,N,Kd", [(4096, 4096, 64), (4096, 4099, 200), (2048, 2048, 32),
                                     (2047, 1985, 17), (8192, 768, 64), (8191, 768, 130),
                                     (4096, 768, 64), (4095, 768, 49), (1024, 1024, 128),
-                                    (1023, 1021, 131), (515, 2047, 1), (700, 600, 1100)])
+                                    (1023, 1021, 131), (515, 2047, 1), (700, 600, 1100),
+                                    # 64 x 64 tiles with one and two wave groups
+                                    (1184, 448, 32), (601, 930, 10), (1103, 577, 48), (1472, 192, 192),
+                                    (1024, 1024, 256), (601, 930, 200), (601, 930, 257)])
 def test_within_fp32_bound(dev, ta, tb, M, N, Kd):
     g = _gen(M + N + Kd)
     A = torch.randn(M, Kd, device=dev, generator=g)
