@@ -1307,7 +1307,7 @@ int gemm_impl(char ta, char tb, int64_t M, int64_t N, int64_t K, float alpha, co
     gp.pair_F = 0;
     gp.sf_h = nullptr;
     gp.sf_ldh = 0;
-    gp.exact_only = 0;
+    gp.far = 0;
     if(sfwd) {
         if(TA || TB || batch != 1 || causal != 0 || beta != 0.0f || !own_c)
             return pk::fail("pk_gemm_swiglu_fwd_f32: only the plain ('N','N') product is built");
@@ -1387,7 +1387,7 @@ int gemm_impl(char ta, char tb, int64_t M, int64_t N, int64_t K, float alpha, co
     // a tile's loads reach 32-bit byte offsets: 256 rows of a k-contiguous
     // operand, 16 (fp32) or 32 k rows of the other kind
     const int64_t near_k = (int64_t)1 << 21, near_r = (int64_t)1 << (prec == kFp32 ? 25 : 24);
-    gp.exact_only = lda > (TA ? near_r : near_k) || ldb > (TB ? near_k : near_r);
+    gp.far = lda > (TA ? near_r : near_k) || ldb > (TB ? near_k : near_r);
     SplitPlan plan = {{kTile128, 128, 128}, 1, K};
     // fp8 and the four-wave bf16 kernel: float4 loads need 16-byte aligned operands
     // and leading dimensions and batch strides that are multiples of 4; the
@@ -1407,7 +1407,7 @@ int gemm_impl(char ta, char tb, int64_t M, int64_t N, int64_t K, float alpha, co
         plan = plan_split(prec, M, N, K, batch, causal == 0, TA, may_split, use96);
         if(plan.splits > 1 && ws_bytes < (size_t)plan.splits * (size_t)M * (size_t)N * sizeof(float))
             plan = plan_split(prec, M, N, K, batch, true, TA, false, use96);
-        if(prec != kFp32 && gp.exact_only) plan.tile = {kTile64, 64, 64};
+        if(gp.far) plan.tile = {prec == kFp32 ? kTile64x2 : kTile64, 64, 64};
     } else if(may_split) {
         plan.splits = choose_splits(M, N, K, TA, false, &plan.kchunk);
         if(ws_bytes < (size_t)plan.splits * (size_t)M * (size_t)N * sizeof(float))

@@ -44,9 +44,9 @@ struct GemmParams {
     int64_t pair_F;
     float* sf_h;
     int64_t sf_ldh;
-    // fp32 products: 1 runs every tile on the fp32 matrix cores with 64-bit
-    // addresses (an operand whose rows are too far apart for buffer offsets)
-    int exact_only;
+    // 1: an operand's rows are too far apart for buffer offsets, so tiles (64x64
+    // ones only) load with 64-bit addresses
+    int far;
 };
 
 // Bounds handling of a tile's loads and stores: none (whole tiles), per float4
@@ -298,13 +298,13 @@ __device__ __forceinline__ void staged_epilogue(const GemmParams& p, const TileJ
 enum TileKind { kTile128, kTile96, kTile256, kTile64, kTile256x96, kTile128x64, kTile64x2, kTile64x1 };
 
 // the fp32 product (gemm_split.hip): K groups a shape's workgroups split K into,
-// and the launch
+// and the launch; with gp.far, kTile64x2 only
 int split_groups(TileKind kind);
 int launch_split(bool ta, bool tb, const GemmParams& gp, int64_t batch, bool edge, TileKind kind,
                  hipStream_t st);
 
 // the bf16 (parts 1) and split-bf16 (parts 2) products (gemm_narrow.hip); with
-// gp.exact_only, 64x64 tiles only
+// gp.far, 64x64 tiles only
 int launch_narrow(bool ta, bool tb, int parts, const GemmParams& gp, int64_t batch, bool edge,
                   TileKind kind, hipStream_t st);
 

@@ -37,30 +37,6 @@ using namespace pkg;
 
 constexpr int W = 32;  // k per slice
 
-// How a tile's operands are read: buffer loads without bounds (whole tiles),
-// bounded by the operand's end, or one element at a time with 64-bit addresses
-// (leading dimensions beyond the reach of buffer offsets)
-constexpr int kWhole = 0, kPartial = 1, kFar = 2;
-
-template <bool KFAST, int R, int THREADS, bool PAIR>
-__device__ __forceinline__ void far_load(const float* x, int64_t ld, int64_t row0, int64_t rows,
-                                         int64_t k0, int64_t kend, int64_t shift,
-                                         float (&v)[SplitOperand<KFAST, R, THREADS, W>::ITEMS]
-                                                   [SplitOperand<KFAST, R, THREADS, W>::KPI]) {
-    using O = SplitOperand<KFAST, R, THREADS, W>;
-#pragma unroll
-    for(int i = 0; i < O::ITEMS; ++i) {
-        int rr, kk;
-        O::origin(i, rr, kk);
-        const int64_t row = row0 + rr + (PAIR && rr >= R / 2 ? shift : 0);
-#pragma unroll
-        for(int t = 0; t < O::KPI; ++t) {
-            const int64_t k = k0 + kk + t;
-            v[i][t] = row < rows && k < kend ? x[KFAST ? row * ld + k : k * ld + row] : 0.0f;
-        }
-    }
-}
-
 template <bool TA, bool TB, int EDGE, class T, int P, int EPI>
 __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_narrow_kernel(GemmParams p) {
     constexpr int BM = T::BM, BN = T::BN, TM = T::TM, TN = T::TN, NT_ = T::THREADS;
@@ -120,8 +96,8 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_narrow_kernel(GemmPar
             constexpr bool TAIL = decltype(tail)::value;
             const int64_t k0 = job.kbeg + (int64_t)min(s, nslices - 1) * W;
             if constexpr(EDGE == kFar) {
-                far_load<AK, BM, NT_, false>(job.A, p.lda, job.row0, p.M, k0, job.kend, 0, ra);
-                far_load<BKF, BN, NT_, PAIR>(job.B, p.ldb, job.col0, p.N, k0, job.kend, shift, rb);
+                far_load<AK, BM, NT_, false, W>(job.A, p.lda, job.row0, p.M, k0, job.kend, 0, ra);
+                far_load<BKF, BN, NT_, PAIR, W>(job.B, p.ldb, job.col0, p.N, k0, job.kend, shift, rb);
             } else {
                 constexpr bool EA = EDGE == kPartial && (AK || TAIL), EB = EDGE == kPartial && (BKF || TAIL);
                 split_load<AK, EA, BM, NT_, false, W>(sa, p.lda, k0, 0, ra);
@@ -256,7 +232,7 @@ int launch_layout(const GemmParams& gp, int64_t batch, bool edge, TileKind kind,
     switch(kind) {
     case kTile256: launch_narrow_tile<TA, TB, Narrow256, P>(gp, batch, edge, st); break;
     case kTile64: {
-        if(!gp.exact_only) {
+        if(!gp.far) {
             launch_narrow_tile<TA, TB, Narrow64, P>(gp, batch, edge, st);
             break;
         }

@@ -155,6 +155,37 @@ __device__ __forceinline__ void split_load(const SplitSource& src, int64_t ld, i
     }
 }
 
+// How a tile's operands are read: buffer loads without bounds (whole tiles), bounded
+// by the operand's end, or with 64-bit addresses (leading dimensions beyond the
+// reach of buffer offsets)
+constexpr int kWhole = 0, kPartial = 1, kFar = 2;
+
+// the slice at k0 of rows row0.., zeros past `rows` and kend
+template <bool KFAST, int R, int THREADS, bool PAIR, int W>
+__device__ __forceinline__ void far_load(const float* x, int64_t ld, int64_t row0, int64_t rows,
+                                         int64_t k0, int64_t kend, int64_t shift,
+                                         float (&v)[SplitOperand<KFAST, R, THREADS, W>::ITEMS]
+                                                   [SplitOperand<KFAST, R, THREADS, W>::KPI]) {
+    using O = SplitOperand<KFAST, R, THREADS, W>;
+    typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+#pragma unroll
+    for(int i = 0; i < O::ITEMS; ++i) {
+        int rr, kk;
+        O::origin(i, rr, kk);
+        const int64_t row = row0 + rr + (PAIR && rr >= R / 2 ? shift : 0), k = k0 + kk;
+        const float* q = x + (KFAST ? row * ld + k : k * ld + row);
+        if(KFAST && row < rows && k + 3 < kend) {
+            const f32x4 y = *reinterpret_cast<const f32x4u*>(q);
+#pragma unroll
+            for(int t = 0; t < 4; ++t) v[i][t] = y[t];
+            continue;
+        }
+#pragma unroll
+        for(int t = 0; t < O::KPI; ++t)
+            v[i][t] = row < rows && k + t < kend ? q[KFAST ? t : t * ld] : 0.0f;
+    }
+}
+
 // zero the values at k >= limit (limit < W: the last, partial slice)
 template <bool KFAST, int R, int THREADS, int W = SK>
 __device__ __forceinline__ void split_mask(int limit,
@@ -235,8 +266,7 @@ struct SplitFrag {
 };
 
 // the wave's tile again on the fp32 matrix cores, straight from global memory
-// with 64-bit addresses: for a wave whose split sums are not finite, and for
-// operands whose rows are too far apart for buffer offsets
+// with 64-bit addresses: for a wave whose split sums are not finite
 template <bool TA, bool TB, bool PAIR, class T>
 __device__ __forceinline__ void exact_tile(const GemmParams& p, const TileJob& j,
                                                      f32x16 (&acc)[T::TM][T::TN], int ar0, int br0,
@@ -300,7 +330,7 @@ __device__ __forceinline__ void split_sched() {
     }
 }
 
-template <bool TA, bool TB, bool EDGE, class T, int EPI>
+template <bool TA, bool TB, int EDGE, class T, int EPI>
 __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmParams p) {
     constexpr int BM = T::BM, BN = T::BN, TM = T::TM, TN = T::TN, NT_ = T::GTHREADS, G = T::G,
                   SETS = T::A;
@@ -320,8 +350,7 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmPara
     short* const lds = lds_all + g * 2 * STAGE;
     // slices per group, an even number unless one group has several sets of sums
     constexpr int STEP = G == 1 && SETS > 1 ? 1 : 2;
-    const int nslices =
-        p.exact_only ? 0 : (int)((job.kend - job.kbeg + STEP * G * SK - 1) / (STEP * G * SK)) * STEP;
+    const int nslices = (int)((job.kend - job.kbeg + STEP * G * SK - 1) / (STEP * G * SK)) * STEP;
 
     f32x16 acc[TM][TN], more[SETS > 1 ? SETS - 1 : 1];  // the first set, the others
 #pragma unroll
@@ -355,15 +384,20 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmPara
         const int64_t klen = job.kend - job.kbeg;
         auto load = [&](Regs& r, int s) {
             const int64_t k0 = job.kbeg + ((int64_t)(EDGE ? s : min(s, nslices - 1)) * G + g) * SK;
-            split_load<AK, EDGE, BM, NT_, false>(sa, p.lda, k0, 0, r.a);
-            split_load<BKF, EDGE, BN, NT_, PAIR>(sb, p.ldb, k0, shift, r.b);
+            if constexpr(EDGE == kFar) {
+                far_load<AK, BM, NT_, false, SK>(job.A, p.lda, job.row0, p.M, k0, job.kend, 0, r.a);
+                far_load<BKF, BN, NT_, PAIR, SK>(job.B, p.ldb, job.col0, p.N, k0, job.kend, shift, r.b);
+            } else {
+                split_load<AK, EDGE == kPartial, BM, NT_, false>(sa, p.lda, k0, 0, r.a);
+                split_load<BKF, EDGE == kPartial, BN, NT_, PAIR>(sb, p.ldb, k0, shift, r.b);
+            }
         };
         auto store = [&](const Regs& r, int stage, float scale_a) {
             split_store<3, AK, BM, NT_, PART>(lds + stage * STAGE, r.a, scale_a);
             split_store<3, BKF, BN, NT_, PART>(lds + stage * STAGE + BM * SK, r.b, 0x1p16f);
         };
         auto mask = [&](Regs& r, int s) {
-            if constexpr(EDGE) {
+            if constexpr(EDGE == kPartial) {
                 const int64_t limit = klen - ((int64_t)s * G + g) * SK;
                 // (k rows of a row-contiguous operand past K lie behind its end)
                 if((AK || BKF) && limit < SK) {
@@ -525,7 +559,7 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmPara
                 if(G == 1 && SETS == 1) acc[i][j][r] *= unscale;
                 sum = fmaf(acc[i][j][r], 0.0f, sum);
             }
-    if(p.exact_only || __any(sum != 0.0f))
+    if(__any(sum != 0.0f))
         exact_tile<TA, TB, PAIR, T>(p, job, acc, ar0, br0, lr, lh);
 
     if constexpr(EPI == kEpiPlain)

@@ -16,7 +16,7 @@ using Split64 = SplitTile<2, 2, 1, 1, 4, 4, 2>;
 using Split64x2 = SplitTile<2, 2, 1, 1, 2, 4, 1, 2>;
 using Split64x1 = SplitTile<2, 2, 1, 1, 1, 4, 1, 4>;
 
-template <bool TA, bool TB, bool EDGE, class T>
+template <bool TA, bool TB, int EDGE, class T>
 void launch_split_kernel(const GemmParams& gp, dim3 grid, hipStream_t st) {
     if constexpr(!TA && TB) {
         if(gp.sg_a) {
@@ -41,9 +41,9 @@ template <bool TA, bool TB, class T>
 int launch_split_tile(const GemmParams& gp, int64_t batch, bool edge, hipStream_t st) {
     dim3 grid((unsigned)(gp.tiles_m * gp.tiles_n), (unsigned)(gp.splits > 1 ? gp.splits : batch));
     if(edge)
-        launch_split_kernel<TA, TB, true, T>(gp, grid, st);
+        launch_split_kernel<TA, TB, kPartial, T>(gp, grid, st);
     else
-        launch_split_kernel<TA, TB, false, T>(gp, grid, st);
+        launch_split_kernel<TA, TB, kWhole, T>(gp, grid, st);
     return pk::launch_status("pk_gemm_f32");
 }
 
@@ -54,7 +54,13 @@ int launch_layout(const GemmParams& gp, int64_t batch, bool edge, TileKind kind,
     case kTile256x96: return launch_split_tile<TA, TB, Split256x96>(gp, batch, edge, st);
     case kTile128x64: return launch_split_tile<TA, TB, Split128x64>(gp, batch, edge, st);
     case kTile64: return launch_split_tile<TA, TB, Split64>(gp, batch, edge, st);
-    case kTile64x2: return launch_split_tile<TA, TB, Split64x2>(gp, batch, edge, st);
+    case kTile64x2: {
+        if(!gp.far) return launch_split_tile<TA, TB, Split64x2>(gp, batch, edge, st);
+        dim3 grid((unsigned)(gp.tiles_m * gp.tiles_n),
+                  (unsigned)(gp.splits > 1 ? gp.splits : batch));
+        launch_split_kernel<TA, TB, kFar, Split64x2>(gp, grid, st);
+        return pk::launch_status("pk_gemm_f32");
+    }
     case kTile64x1: return launch_split_tile<TA, TB, Split64x1>(gp, batch, edge, st);
     default: return launch_split_tile<TA, TB, Split128>(gp, batch, edge, st);
     }

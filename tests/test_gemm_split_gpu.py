@@ -106,16 +106,28 @@ def test_infinities_and_nan(dev, ta, tb):
     assert _within_bound(C[fine], A[fine], B)
 
 
-def test_rows_too_far_apart_for_buffer_offsets(dev):
-    """a leading dimension above 2^21 floats: 64-bit addresses"""
-    ld, M, N, Kd = (1 << 21) + 8, 3, 5, 1500
-    big = torch.zeros(M, ld, device=dev)
-    A = big[:, :Kd]
-    A.copy_(torch.randn(M, Kd, device=dev, generator=_gen(4)))
+@pytest.mark.parametrize("ta,tb,M,N,Kd", [("N", "N", 3, 5, 1500), ("N", "T", 70, 130, 1503),
+                                          ("N", "N", 128, 64, 4096), ("T", "N", 67, 70, 35)])
+def test_rows_too_far_apart_for_buffer_offsets(dev, ta, tb, M, N, Kd):
+    """a leading dimension above 2^21 (k-contiguous) or 2^25 floats: 64-bit
+    addresses, also with K split and a residual"""
+    ld = (1 << 21) + 8 if ta == "N" else (1 << 25) + 4
+    A = torch.randn(M, Kd, device=dev, generator=_gen(4))
     B = torch.randn(Kd, N, device=dev, generator=_gen(5))
-    C = torch.empty(M, N, device=dev)
-    K.gemm("N", "N", A, B, C)
-    assert _within_bound(C, A, B)
+    a = A if ta == "N" else A.t()
+    far = torch.full((a.shape[0], ld), float("nan"), device=dev)[:, :a.shape[1]]
+    far.copy_(a)
+    b = B if tb == "N" else B.t().contiguous()
+    for ws in (None, torch.full((K.gemm_workspace(M, N, Kd) // 4 + 4,), float("nan"), device=dev)):
+        C = torch.full((M, N), 3.0, device=dev)
+        if ws is None:
+            K.gemm(ta, tb, far, b, C)
+        else:
+            K.gemm_ex(ta, tb, far, b, C, beta=1.0, ws=ws)
+            C = C.double() - 3.0
+        a64, b64 = A.double(), B.double()
+        err = (C.double() - a64 @ b64).abs()
+        assert bool((err <= (1.5 * Kd + 10) * 2.0 ** -24 * (a64.abs() @ b64.abs() + 3.0)).all())
 
 
 @pytest.mark.parametrize("ta,tb", [("N", "N"), ("T", "N"), ("N", "T")])
