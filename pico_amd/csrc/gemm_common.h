@@ -118,36 +118,42 @@ __device__ __forceinline__ TileJob tile_job(const GemmParams& p) {
     return j;
 }
 
-// C tile = alpha * acc (+ beta * C).  32x32 block accumulator r of lane l is
+// C block = alpha * acc (+ beta * C).  32x32 block accumulator r of lane l is
 // row 8*(r/4) + 4*(l/32) + r%4, column l%32: each half-wave writes 128
 // contiguous bytes per register.
+template <int EDGE, bool NT_STORE>
+__device__ __forceinline__ void store_block(const GemmParams& p, const TileJob& j, const f32x16& acc,
+                                            int ar, int br, int lr, int lh) {
+    const int64_t col = j.col0 + br + lr;
+#pragma unroll
+    for(int r = 0; r < 16; ++r) {
+        const int64_t row = j.row0 + ar + (r >> 2) * 8 + lh * 4 + (r & 3);
+        if(EDGE != kEdgeNone && (row >= p.M || col >= p.N)) continue;
+        float v = j.alpha * acc[r];
+        float* c = j.C + row * j.ldc + col;
+        if(j.beta != 0.0f) v += j.beta * *c;
+        // 64x64 tiles (products of about 1024^2 outputs, where the
+        // launch's end is a large share of its time) store C
+        // non-temporally: 1024^3 1.1-1.6 % and 768^3 0.6-1.1 % faster,
+        // config-4 and config-5 steps unchanged (same box, alternating);
+        // for every tile they cost a config-5 step 0.05 ms
+        if constexpr(NT_STORE) __builtin_nontemporal_store(v, c);
+        else *c = v;
+    }
+}
+
+// The tile's blocks but those of the bits of `skip`.
 // G > 1: of the tile's blocks, the K group g stores those it finished.
 template <int EDGE, int TM, int TN, int G = 1>
 __device__ __forceinline__ void store_tile(const GemmParams& p, const TileJob& j,
                                            const f32x16 (&acc)[TM][TN], int ar0, int br0, int lr,
-                                           int lh, int g = 0) {
+                                           int lh, int g = 0, unsigned skip = 0) {
 #pragma unroll
-    for(int i = 0; i < TM; ++i)
-#pragma unroll
-        for(int jj = 0; jj < TN; ++jj) {
-            if(G > 1 && (i * TN + jj) % G != g) continue;
-            const int64_t col = j.col0 + br0 + jj * 32 + lr;
-#pragma unroll
-            for(int r = 0; r < 16; ++r) {
-                const int64_t row = j.row0 + ar0 + i * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
-                if(EDGE != kEdgeNone && (row >= p.M || col >= p.N)) continue;
-                float v = j.alpha * acc[i][jj][r];
-                float* c = j.C + row * j.ldc + col;
-                if(j.beta != 0.0f) v += j.beta * *c;
-                // 64x64 tiles (products of about 1024^2 outputs, where the
-                // launch's end is a large share of its time) store C
-                // non-temporally: 1024^3 1.1-1.6 % and 768^3 0.6-1.1 % faster,
-                // config-4 and config-5 steps unchanged (same box, alternating);
-                // for every tile they cost a config-5 step 0.05 ms
-                if constexpr(TM * TN == 1) __builtin_nontemporal_store(v, c);
-                else *c = v;
-            }
-        }
+    for(int b = 0; b < TM * TN; ++b) {
+        if((G > 1 && b % G != g) || (skip >> b & 1)) continue;
+        store_block<EDGE, TM * TN == 1>(p, j, acc[b / TN][b % TN], ar0 + b / TN * 32,
+                                        br0 + b % TN * 32, lr, lh);
+    }
 }
 
 // Epilogues that read other matrices: the tile goes through LDS (free once
@@ -217,15 +223,26 @@ __device__ __forceinline__ void epi_four(const GemmParams& p, const TileJob& j, 
     }
 }
 
-template <int EPI, class T, int LDS_FLOATS>
+// Blocks of the bits of `skip` come from block(index) instead of acc.
+struct NoBlock {
+    __device__ f32x16 operator()(int) const { return f32x16{}; }
+};
+
+template <int EPI, class T, int LDS_FLOATS, class Block = NoBlock>
 __device__ __forceinline__ void staged_epilogue(const GemmParams& p, const TileJob& j,
                                                 const f32x16 (&acc)[T::TM][T::TN], float* lds,
-                                                int ar0, int br0, int lr, int lh, int g = 0) {
+                                                int ar0, int br0, int lr, int lh, int g = 0,
+                                                unsigned skip = 0, const Block& block = Block()) {
     constexpr int BN = T::BN, LDE = BN + 4, TM = T::TM, TN = T::TN, NTHR = T::THREADS;
     // rows per pass: whole 32-row blocks that fit in the operand buffers
     constexpr int rp = (LDS_FLOATS / LDE) / 32 * 32 < T::BM ? (LDS_FLOATS / LDE) / 32 * 32 : T::BM;
     static_assert(rp >= 32, "the staging buffer must hold at least one 32-row block");
     __syncthreads();  // every wave is done reading the operand tiles
+    auto put = [&](const f32x16& x, int row, int col) {
+#pragma unroll
+        for(int r = 0; r < 16; ++r)
+            lds[(row + (r >> 2) * 8 + lh * 4 + (r & 3)) * LDE + col + lr] = x[r];
+    };
     for(int lo = 0; lo < T::BM; lo += rp) {
 #pragma unroll
         for(int i = 0; i < TM; ++i) {
@@ -233,12 +250,13 @@ __device__ __forceinline__ void staged_epilogue(const GemmParams& p, const TileJ
             if(rb < lo || rb >= lo + rp) continue;
 #pragma unroll
             for(int jj = 0; jj < TN; ++jj) {
-                if(T::G > 1 && (i * TN + jj) % T::G != g) continue;
-#pragma unroll
-                for(int r = 0; r < 16; ++r)
-                    lds[(rb - lo + (r >> 2) * 8 + lh * 4 + (r & 3)) * LDE + br0 + jj * 32 + lr] =
-                        acc[i][jj][r];
+                if((T::G > 1 && (i * TN + jj) % T::G != g) || (skip >> (i * TN + jj) & 1)) continue;
+                put(acc[i][jj], rb - lo, br0 + jj * 32);
             }
+        }
+        for(unsigned left = skip; left; left &= left - 1) {
+            const int b = __builtin_ctz(left), rb = ar0 + b / TN * 32;
+            if(rb >= lo && rb < lo + rp) put(block(b), rb - lo, br0 + b % TN * 32);
         }
         __syncthreads();
         const int rows = rp < T::BM - lo ? rp : T::BM - lo;

@@ -19,8 +19,8 @@
 //    subnormal fp32 number are exact bf16 numbers (l of a 2^-126 would need
 //    2^-149), and the sums by 2^-32 at the end.  What overflows (values above
 //    2^111, sums above 2^96, infinities) or is NaN leaves a non-finite sum: a
-//    wave that sees one computes its tile again on the fp32 cores, from global
-//    memory (exact_tile).
+//    wave that sees one computes that 32x32 block again on the fp32 cores, from
+//    global memory (exact_block).
 //  * Sign: the matrix unit drops the low bits of products much smaller than the
 //    accumulator towards minus infinity.  One sum loses less than its
 //    roundings, but the loss has the same sign in every output, so it would
@@ -265,54 +265,74 @@ struct SplitFrag {
     bf16x8 a[TM], b[TN];
 };
 
-// the wave's tile again on the fp32 matrix cores, straight from global memory
-// with 64-bit addresses: for a wave whose split sums are not finite
-template <bool TA, bool TB, bool PAIR, class T>
-__device__ __forceinline__ void exact_tile(const GemmParams& p, const TileJob& j,
-                                                     f32x16 (&acc)[T::TM][T::TN], int ar0, int br0,
-                                                     int lr, int lh) {
-    constexpr int TM = T::TM, TN = T::TN;
+// one 32x32 block again on the fp32 matrix cores, from global memory with 64-bit
+// addresses: for blocks whose split sums are not finite.  8 k at a time (lanes
+// 0-31 take four of them, lanes 32-63 the others), D such steps in flight.  An
+// infinity in one row of 4096^3 costs 813-843 us in all (1060 with one step in
+// flight; the whole tile again 1340-1865; fp32 cores throughout 915), one in every
+// row 2000-2600 (bound by the loads, which only one block shares)
+template <bool KFAST>
+__device__ __forceinline__ void exact_load(const float* x, int64_t ld, float (&f)[4]) {
+    typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+    if constexpr(KFAST) {
+        const f32x4 y = *reinterpret_cast<const f32x4u*>(x);
 #pragma unroll
-    for(int i = 0; i < TM; ++i)
+        for(int e = 0; e < 4; ++e) f[e] = y[e];
+    } else {
 #pragma unroll
-        for(int jj = 0; jj < TN; ++jj)
-#pragma unroll
-            for(int r = 0; r < 16; ++r) acc[i][jj][r] = 0.0f;
-#pragma unroll 1
-    for(int64_t k0 = j.kbeg; k0 < j.kend; k0 += 8) {
-        const int64_t k = k0 + lh * 4;
-        float fa[TM][4], fb[TN][4];
-#pragma unroll
-        for(int i = 0; i < TM; ++i) {
-            const int64_t r = min(j.row0 + ar0 + i * 32 + lr, p.M - 1);
-#pragma unroll
-            for(int t = 0; t < 4; ++t) {
-                const int64_t kc = min(k + t, j.kend - 1);
-                const float x = j.A[TA ? kc * p.lda + r : r * p.lda + kc];
-                fa[i][t] = k + t < j.kend ? x : 0.0f;
-            }
-        }
-#pragma unroll
-        for(int jj = 0; jj < TN; ++jj) {
-            const int c = br0 + jj * 32 + lr;
-            const int64_t n = min(j.col0 + c + (PAIR && c >= T::BN / 2 ? p.pair_F - T::BN / 2 : 0),
-                                  p.N - 1);
-#pragma unroll
-            for(int t = 0; t < 4; ++t) {
-                const int64_t kc = min(k + t, j.kend - 1);
-                const float x = j.B[TB ? n * p.ldb + kc : kc * p.ldb + n];
-                fb[jj][t] = k + t < j.kend ? x : 0.0f;
-            }
-        }
-#pragma unroll
-        for(int t = 0; t < 4; ++t)
-#pragma unroll
-            for(int i = 0; i < TM; ++i)
-#pragma unroll
-                for(int jj = 0; jj < TN; ++jj)
-                    acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][t], fb[jj][t],
-                                                                      acc[i][jj], 0, 0, 0);
+        for(int e = 0; e < 4; ++e) f[e] = x[e * ld];
     }
+}
+
+template <bool TA, bool TB, bool PAIR, class T, int D>
+__device__ __forceinline__ f32x16 exact_block(const GemmParams& p, const TileJob& j, int ar, int br,
+                                              int lr, int lh) {
+    const int64_t m = min(j.row0 + ar + lr, p.M - 1);
+    const int c = br + lr;
+    const int64_t n = min(j.col0 + c + (PAIR && c >= T::BN / 2 ? p.pair_F - T::BN / 2 : 0), p.N - 1);
+    const int64_t sa = TA ? p.lda : 1, sb = TB ? 1 : p.ldb;
+    const float* const a = j.A + (TA ? m : m * p.lda) + (j.kbeg + 4 * lh) * sa;
+    const float* const b = j.B + (TB ? n * p.ldb : n) + (j.kbeg + 4 * lh) * sb;
+    const int64_t klen = j.kend - j.kbeg;
+    const int64_t whole = klen / 8;  // steps
+    f32x16 acc;
+#pragma unroll
+    for(int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    float fa[D][4], fb[D][4];
+    int64_t s = 0;
+    if(whole >= D) {
+        auto load = [&](int d, int64_t step) {
+            const int64_t k = 8 * min(step, whole - 1);
+            exact_load<!TA>(a + k * sa, p.lda, fa[d]);
+            exact_load<TB>(b + k * sb, p.ldb, fb[d]);
+        };
+#pragma unroll
+        for(int d = 0; d < D; ++d) load(d, d);
+#pragma unroll 1
+        for(; s + D <= whole; s += D) {
+#pragma unroll
+            for(int d = 0; d < D; ++d) {
+#pragma unroll
+                for(int i = 0; i < 4; ++i)
+                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[d][i], fb[d][i], acc, 0, 0, 0);
+                load(d, s + d + D);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+#pragma unroll 1
+    for(int64_t k = 8 * s; k < klen; k += 8) {
+#pragma unroll
+        for(int i = 0; i < 4; ++i) {
+            const bool in = k + 4 * lh + i < klen;
+            fa[0][i] = in ? a[(k + i) * sa] : 0.0f;
+            fb[0][i] = in ? b[(k + i) * sb] : 0.0f;
+        }
+#pragma unroll
+        for(int i = 0; i < 4; ++i)
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[0][i], fb[0][i], acc, 0, 0, 0);
+    }
+    return acc;
 }
 
 // one MFMA, then its share of the phase's other instructions
@@ -548,23 +568,44 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmPara
             }
         }
     }
-    float sum = 0.0f;
+    // the wave's blocks with a sum that is not finite among those it stores (a
+    // tile's rows and columns past M and N may hold anything)
+    unsigned again = 0;
 #pragma unroll
-    for(int i = 0; i < TM; ++i)
+    for(int i = 0; i < TM; ++i) {
+        const int left = (int)min(p.M - job.row0 - ar0 - i * 32 - lh * 4, (int64_t)32);
 #pragma unroll
-        for(int j = 0; j < TN; ++j)
-            if(G == 1 || g == (i * TN + j) % G)
+        for(int j = 0; j < TN; ++j) {
+            if(G > 1 && g != (i * TN + j) % G) continue;
+            float sum = 0.0f;
 #pragma unroll
             for(int r = 0; r < 16; ++r) {
                 if(G == 1 && SETS == 1) acc[i][j][r] *= unscale;
-                sum = fmaf(acc[i][j][r], 0.0f, sum);
+                const bool in = EDGE == kWhole || (r >> 2) * 8 + (r & 3) < left;
+                sum = fmaf(in ? acc[i][j][r] : 0.0f, 0.0f, sum);
             }
-    if(__any(sum != 0.0f))
-        exact_tile<TA, TB, PAIR, T>(p, job, acc, ar0, br0, lr, lh);
-
-    if constexpr(EPI == kEpiPlain)
-        store_tile<EDGE ? kEdgeScalar : kEdgeNone, TM, TN, G>(p, job, acc, ar0, br0, lr, lh, g);
-    else
+            const int c = br0 + j * 32 + lr;
+            const bool in = EDGE == kWhole || (PAIR ? job.col0 + c % (BN / 2) < p.pair_F : job.col0 + c < p.N);
+            if(__any(in && sum != 0.0f)) again |= 1u << (i * TN + j);
+        }
+    }
+    again = __builtin_amdgcn_readfirstlane(again);
+    auto exact = [&](int b) {
+        // (staged epilogues hold the tile's sums meanwhile)
+        constexpr int D = EPI == kEpiPlain || T::WPS <= 2 ? 4 : 2;
+        return exact_block<TA, TB, PAIR, T, D>(p, job, ar0 + b / TN * 32, br0 + b % TN * 32, lr, lh);
+    };
+    if constexpr(EPI == kEpiPlain) {
+        constexpr int EDGES = EDGE == kWhole ? kEdgeNone : kEdgeScalar;
+        store_tile<EDGES, TM, TN, G>(p, job, acc, ar0, br0, lr, lh, g, again);
+        // (last, when the sums' registers are free)
+        for(; again; again &= again - 1) {
+            const int b = __builtin_ctz(again);
+            store_block<EDGES, TM * TN == 1>(p, job, exact(b), ar0 + b / TN * 32, br0 + b % TN * 32,
+                                             lr, lh);
+        }
+    } else {
         staged_epilogue<EPI, T, (int)sizeof(lds_all) / 4>(p, job, acc, reinterpret_cast<float*>(lds_all),
-                                                         ar0, br0, lr, lh, g);
+                                                         ar0, br0, lr, lh, g, again, exact);
+    }
 }

@@ -146,6 +146,47 @@ def test_gemm_swiglu_fwd_equals_product_then_swiglu(dev, M, K, F, prec):
         assert max_rel(h.cpu().numpy(), want) <= 1e-4
 
 
+def _same_or_nan(got, ref):
+    assert torch.equal(torch.isnan(got), torch.isnan(ref))
+    assert torch.equal(torch.nan_to_num(got, nan=0.0), torch.nan_to_num(ref, nan=0.0))
+
+
+# 256 x 256, 128 x 128 and the 64 x 64 tiles; a sum that is not finite has its 32 x 32
+# block computed another way, in the fused epilogue as in the plain product
+@pytest.mark.parametrize("M,F,N", [(4096, 2048, 96), (1000, 2048, 200), (500, 1024, 130), (700, 352, 1100)])
+def test_fused_epilogues_with_infinities(dev, M, F, N):
+    L = _lib.hip_lib()
+    A, X = torch.randn(M, N, device=dev), torch.randn(M, 2 * F, device=dev)
+    W = torch.randn(N, 2 * F, device=dev) * 0.1
+    assert not L.pk_gemm_small_product_f32(M, 2 * F, N)
+    A[3, 5], A[M - 1, N - 1], A[M // 2, 0], W[7, 40] = float("inf"), float("nan"), 3e38, float("-inf")
+    ref, got, h, href, add = (torch.full((M, n), float("nan"), device=dev)
+                              for n in (2 * F, 2 * F, F, F, 2 * F))
+    kern.gemm("N", "N", A, W, ref)
+    kern.swiglu_fwd(ref[:, :F], ref[:, F:], href)
+    _lib.check("pk_gemm_swiglu_fwd_f32", L.pk_gemm_swiglu_fwd_f32(
+        b"N", b"N", M, 2 * F, N, 1.0, A.data_ptr(), N, W.data_ptr(), 2 * F, got.data_ptr(), 2 * F,
+        h.data_ptr(), F, 0, None, None))
+    _same_or_nan(got, ref)
+    _same_or_nan(h, href)
+    _lib.check("pk_gemm_add_f32", L.pk_gemm_add_f32(
+        b"N", b"N", M, 2 * F, N, 1.0, A.data_ptr(), N, W.data_ptr(), 2 * F, 1.0, X.data_ptr(), 2 * F,
+        add.data_ptr(), 2 * F, 0, None, None, 0, None))
+    _same_or_nan(add, X + ref)
+    dh, Wt = torch.empty(M, F, device=dev), W[:, :F].t().contiguous()
+    assert not L.pk_gemm_small_product_f32(M, F, N)
+    kern.gemm("N", "T", A, Wt, dh)
+    for flags in (0, 3):
+        da, want = X.clone(), X.clone()
+        _lib.check("pk_gemm_swiglu_bwd_f32", L.pk_gemm_swiglu_bwd_f32(
+            b"N", b"T", M, F, N, 1.0, A.data_ptr(), N, Wt.data_ptr(), N, X.data_ptr(), 2 * F,
+            X.data_ptr() + 4 * F, 2 * F, da.data_ptr(), da.data_ptr() + 4 * F, 2 * F, flags, 0, None, None))
+        _lib.check("pk_swiglu_bwd_f32", L.pk_swiglu_bwd_f32(
+            M, F, X.data_ptr(), 2 * F, X.data_ptr() + 4 * F, 2 * F, dh.data_ptr(), F, want.data_ptr(),
+            want.data_ptr() + 4 * F, 2 * F, flags, None))
+        _same_or_nan(da, want)
+
+
 def test_gemm_swiglu_fwd_strided_h_and_refusals(dev):
     L = _lib.hip_lib()
     M, K, F = 96, 64, 128

@@ -147,3 +147,46 @@ def test_ragged_operands_end_where_they_end(dev, ta, tb):
     C = torch.full((M, N), float("nan"), device=dev)
     K.gemm(ta, tb, inside(A if ta == "N" else A.t()), inside(B if tb == "N" else B.t()), C)
     assert np.isfinite(C.cpu().numpy()).all() and _within_bound(C, A, B)
+
+
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("T", "N"), ("N", "T"), ("T", "T")])
+@pytest.mark.parametrize("M,N,Kd", [(517, 1031, 1203), (4000, 4100, 100), (1100, 700, 70)])
+def test_what_lies_behind_rows_does_not_choose_the_route(dev, ta, tb, M, N, Kd):
+    """a tile's rows and columns past M and N may read what lies between an
+    operand's rows: NaN there gives the same bits as zeros do, so no block
+    was computed again for it"""
+    g = _gen(8)
+    A = torch.randn(M, Kd, device=dev, generator=g)
+    B = torch.randn(Kd, N, device=dev, generator=g)
+
+    def product(fill):
+        def inside(x):
+            buf = torch.full((x.shape[0] + 64, x.shape[1] + 300), fill, device=dev)
+            buf[:x.shape[0], :x.shape[1]] = x
+            return buf[:x.shape[0], :x.shape[1]]
+        C = torch.full((M, N), 1.0, device=dev)
+        K.gemm(ta, tb, inside(A if ta == "N" else A.t()), inside(B if tb == "N" else B.t()), C, beta=1.0)
+        return C
+
+    assert torch.equal(product(float("nan")), product(0.0))
+
+
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("N", "T"), ("T", "N"), ("T", "T")])
+@pytest.mark.parametrize("M,N,Kd", [(4096, 4096, 77), (2048, 2048, 512), (1024, 1024, 33), (601, 930, 300),
+                                    (4096, 512, 100), (8192, 768, 96)])
+def test_one_row_and_column_not_finite(dev, ta, tb, M, N, Kd):
+    """the other rows and columns keep their accuracy, beta's matrix is added once"""
+    g = _gen(9)
+    A = torch.randn(M, Kd, device=dev, generator=g)
+    B = torch.randn(Kd, N, device=dev, generator=g)
+    A[M // 3, Kd - 1], B[Kd // 2, N - 2] = float("inf"), float("nan")
+    C = torch.full((M, N), 2.0, device=dev)
+    _product(ta, tb, A, B, C, beta=1.0)
+    assert bool(torch.isnan(C[:, N - 2]).all())
+    rest = [i for i in range(N) if i != N - 2]
+    row = C[M // 3][rest].double()
+    assert bool((row == A[M // 3, Kd - 1].double() * B[Kd - 1][rest].double().sign()).all())
+    A[M // 3], B[:, N - 2], C[M // 3], C[:, N - 2] = 0.0, 0.0, 2.0, 2.0
+    a, b = A.double(), B.double()
+    err = (C.double() - 2.0 - a @ b).abs()
+    assert bool((err <= (1.5 * Kd + 10) * 2.0 ** -24 * (a.abs() @ b.abs() + 2.0)).all())
