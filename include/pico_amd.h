@@ -301,8 +301,10 @@ void pico_gpu_fail_next_workspaces(int n);
 /* ---- matmul precision (no reference counterpart: pico is fp32 only) ----
  * PICO_MATMUL_FP32 (the default): pico_matmul, the fused attention's
  * products and their gradients are fp32 products, within the fp32 parity
- * contract (pico_matmul's as six bf16 products of operands split exactly in
- * three, with no larger error than fp32 multiplies).
+ * contract.  pico_matmul's larger ones are six bf16 products of operands split
+ * exactly in three: one product a.b is off by less than 2^-23 |a.b|, and a sum's
+ * relative error (2-norm, random operands) is below that of fp32 multiplies,
+ * but for operands that are half zeros in the largest tiles, up to 14 % above.
  * PICO_MATMUL_BF16: their operands are rounded to bf16 (nearest even) and
  * multiplied on the bf16 matrix cores, accumulating in fp32; tensors, the
  * softmax statistics and every other op stay fp32.  Faster, and outside the

@@ -56,8 +56,8 @@ int pk_device_info(int* cu_count, int* clock_khz, char* arch, int arch_len);
  * ('T','N', beta 1)); a pico_transpose_2d view (src/tensor.c:230-244) maps to 'T'.
  * fp32 in, fp32 sums, 24-bit products: each operand is the exact sum of three
  * bf16 values whose products run on the bf16 matrix cores (the three smallest
- * of nine, below 2^-24 of |a||b|, left out); non-finite tiles are computed on
- * the fp32 cores. */
+ * of nine, below 2^-24 of |a||b|, left out); small products, K of 1 or 2 and
+ * sums that are not finite are computed on the fp32 cores. */
 int pk_gemm_f32(char ta, char tb, int64_t M, int64_t N, int64_t K, float alpha, const float* A,
                 int64_t lda, const float* B, int64_t ldb, float beta, float* C, int64_t ldc,
                 pk_stream_t stream);

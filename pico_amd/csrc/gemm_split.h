@@ -10,11 +10,16 @@
 // nearest, 24 in all), on its way to LDS, and
 //     a.b = hh + hm + mh + mm + hl + lh
 // in six matrix instructions per 16 k; ml, lm and ll, together below 2^-24 of
-// |a||b|, are left out.  Nothing is held in less than fp32's 24 bits, and the
-// sums are fp32.  Against float64 the error is below that of the fp32 matrix
-// instructions (which round after every k): normal operands, relative
-// 2-norm, K 768 / 2048 / 4096: 2.9e-7 / 6.9e-7 / 9.7e-7 against 5.0e-7 /
-// 8.1e-7 / 1.15e-6.
+// |a||b|, are left out (below 0.87 2^-24 of one product at the worst).  Nothing is
+// held in less than fp32's 24 bits, and the sums are fp32.  Against float64,
+// relative 2-norm on random operands, the error is below that of the fp32 matrix
+// instructions (which round after every k) from K 3 on: normal operands, K 4 / 32 /
+// 768 / 2048 / 4096 3.2e-8 / 4.2e-8 / 2.9e-7 / 6.9e-7 / 9.7e-7 against 4.0e-8 /
+// 1.03e-7 / 5.0e-7 / 8.1e-7 / 1.15e-6.  Products of one and two k, whose few
+// roundings they do better (2.5e-8 against 3.5e-8, 3.1e-8 against 3.4e-8), run
+// on the fp32 cores (exact_block).  Half-zero operands (a relu's output) leave the
+// fp32 cores half as many roundings: there 256x256 tiles, which have one sum to a
+// block, are up to 14 % above them (6.5e-7 against 5.7e-7 at K 2048), the others below.
 //  * Range: operands are scaled by 2^16, so that the parts of every normal and
 //    subnormal fp32 number are exact bf16 numbers (l of a 2^-126 would need
 //    2^-149), and the sums by 2^-32 at the end.  What overflows (values above
@@ -370,7 +375,10 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmPara
     short* const lds = lds_all + g * 2 * STAGE;
     // slices per group, an even number unless one group has several sets of sums
     constexpr int STEP = G == 1 && SETS > 1 ? 1 : 2;
-    const int nslices = (int)((job.kend - job.kbeg + STEP * G * SK - 1) / (STEP * G * SK)) * STEP;
+    // (K of 1 or 2 runs on the fp32 cores)
+    const bool cores = p.K <= 2;
+    const int nslices =
+        cores ? 0 : (int)((job.kend - job.kbeg + STEP * G * SK - 1) / (STEP * G * SK)) * STEP;
 
     f32x16 acc[TM][TN], more[SETS > 1 ? SETS - 1 : 1];  // the first set, the others
 #pragma unroll
@@ -586,7 +594,7 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmPara
             }
             const int c = br0 + j * 32 + lr;
             const bool in = EDGE == kWhole || (PAIR ? job.col0 + c % (BN / 2) < p.pair_F : job.col0 + c < p.N);
-            if(__any(in && sum != 0.0f)) again |= 1u << (i * TN + j);
+            if(cores || __any(in && sum != 0.0f)) again |= 1u << (i * TN + j);
         }
     }
     again = __builtin_amdgcn_readfirstlane(again);

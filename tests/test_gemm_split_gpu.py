@@ -190,3 +190,19 @@ def test_one_row_and_column_not_finite(dev, ta, tb, M, N, Kd):
     a, b = A.double(), B.double()
     err = (C.double() - 2.0 - a @ b).abs()
     assert bool((err <= (1.5 * Kd + 10) * 2.0 ** -24 * (a.abs() @ b.abs() + 2.0)).all())
+
+
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("N", "T"), ("T", "N"), ("T", "T")])
+@pytest.mark.parametrize("M,N", [(4096, 4096), (2047, 2049), (1100, 1100), (8192, 768)])
+def test_single_products_are_rounded_once(dev, ta, tb, M, N):
+    """K 1: every output is one fp32 product, correctly rounded; K 2: off by two
+    roundings at most"""
+    g = _gen(10)
+    A = torch.randn(M, 2, device=dev, generator=g)
+    B = torch.randn(2, N, device=dev, generator=g)
+    C = torch.empty(M, N, device=dev)
+    _product(ta, tb, A[:, :1].contiguous(), B[:1].contiguous(), C)
+    assert torch.equal(C, A[:, :1] * B[:1])
+    _product(ta, tb, A, B, C)
+    a, b = A.double(), B.double()
+    assert bool(((C.double() - a @ b).abs() <= 2 * 2.0 ** -24 * (a.abs() @ b.abs())).all())
