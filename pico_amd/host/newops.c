@@ -345,14 +345,18 @@ static void attn_backward(struct PicoTensor* self) {
 /* the fused kernels of head sizes 32, 96 and 128: 16-byte aligned tensors, a
  * sequence within 32-bit byte offsets, and a dS workspace within the cap (the
  * chain's probabilities and scratch would take four times that).  Few long
- * rows of 128 dims run faster as a chain, whose products spread over the chip
- * (forward + backward, us, fused against chain: 192 blocks of 64 rows at T 2048
- * 549 / 438, 128 at T 1024 279 / 221, 256 at T 1024 288 / 275, 264 at T 700
- * 209 / 208, 512 at T 1000 347 / 457; T 128 55 / 59); 32 and 96 dims gain at
- * every size timed, from one head of T 2048 (179 / 308) up */
+ * rows of 96 or 128 dims run faster as a chain, whose products spread over the
+ * chip (forward + backward, us, fused / chain, by blocks of 64 rows).
+ * 128 dims, T 1024: 256 blocks 282 / 265, 320 298 / 294, 384 289 / 335; T 2048: 320
+ * 563 / 559, 384 556 / 634; T 256: 256 96 / 99, 384 121 / 125; T 128 and 65, 16 blocks:
+ * 55 / 62 and 53 / 70, 384: 102 / 98 and 85 / 83.
+ * 96 dims, T 512: 8 blocks 116 / 120; T 1024: 64 214 / 203, 96 217 / 220, 128 216 / 231;
+ * T 2048: 96 418 / 383, 128 408 / 412, 192 423 / 470; T 4096: 64 786 / 722, 128 804 / 831.
+ * 32 dims gain at every size timed (1 head of T 1024 96 / 181) */
 static int wide_applies(struct PicoTensor* const* xs, int64_t B, int64_t H, int64_t T, int64_t hd) {
     if(!pk_flash_wide_supported(T, hd)) return 0;
-    if(hd == 128 && T > 128 && B * H * ((T + 63) / 64) < 384) return 0;
+    const int64_t blocks = B * H * ((T + 63) / 64);
+    if((hd == 128 && T > 128 && blocks < 384) || (hd == 96 && T > 512 && blocks < 128)) return 0;
     for(int i = 0; i < 3; i++)
         if(((uintptr_t)xs[i]->data | (uintptr_t)xs[i]->grad) & 15) return 0;
     const int64_t ld = xs[0]->strides[0];

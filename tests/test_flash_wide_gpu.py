@@ -142,6 +142,29 @@ def test_one_tensor_as_q_k_and_v_and_the_chain_beyond_the_cap(dev, monkeypatch):
         _close(torch.from_numpy(dx).to(dev).reshape(ro.shape), sum(rg))
 
 
+# either side of the lines between the fused kernels and the chain: rows, and
+# blocks of 64 of them
+@pytest.mark.parametrize("H,T,hd", [(1, 512, 96), (1, 513, 96), (12, 600, 96), (13, 600, 96), (1, 128, 128),
+                                    (1, 129, 128), (76, 310, 128), (77, 310, 128)])
+def test_both_sides_of_the_lines(dev, H, T, hd):
+    P = Pico()
+    xs = np.random.default_rng(T + H).standard_normal((3, T, H * hd)).astype(np.float32)
+    with P.arena(1 << 30):
+        q, k, v = (P.param([T, H * hd], x) for x in xs)
+        y = P.attention_causal(q, k, v, 1, H)
+        P.backward(y)
+        out, grads = P.data(y), [P.grad(x) for x in (q, k, v)]
+        for x in (q, k, v):
+            P.free(x)
+    q, k, v = (torch.from_numpy(x).to(dev) for x in xs)
+    ro, _, rg = _reference(1, H, T, hd, q, k, v, torch.ones_like(q))
+    _close(torch.from_numpy(out).to(dev).reshape(ro.shape), ro)
+    for got, want in zip(grads, rg):
+        err = (torch.from_numpy(got).to(dev).reshape(want.shape).double() - want).norm()
+        # (the upstream of ones makes q's and k's exact gradients nearly cancel)
+        assert float(err) <= TOL * float(rg[2].norm())
+
+
 def test_refusals(dev):
     L = _lib.hip_lib()
     x = torch.zeros(64, 256, device=dev)
