@@ -1059,37 +1059,42 @@ enum Precision { kFp32 = 0, kBf16 = 1, kBf16x3 = 2, kFp8 = 3 };
 // launch, a step per partial plane in the reduction's chain (longer where
 // N % 4 leaves it scalar) and the planes' traffic.
 //
-// The constants are fits to about 6500 times: 64 to 2048 tiles of every shape, K 3
-// to 2048, three layouts, whole and ragged, root mean square error 4-11 %.  Over
-// 586 random and transformer shapes with every shape and split timed, the pick
-// ran within 0.7 % (fp32), 2.1 % (bf16) and 0.8 % (split bf16) of the best on average.
-// One time per k and round with a fixed part, which stood here before, ran
-// within 2.6 %, 5.7 % and 2.3 %, and far off at K below 256: [1184, 448] K 32 fp32
-// 8.4 us (now 5.2), [1344, 3712] K 64 19.6 (10.8), [7680, 1344] K 96 35 (22); bf16
-// [4096, 1376] A^T.B K 512 37 (30).
+// A later shape of the lists must be 3 % better than those before it: larger tiles
+// leave more of the chip to what runs beside them (the bf16 feed-forward's
+// [8192, 768] K 4096 A.B^T beside a weight gradient: 256x96 and 128x96 86 us each
+// alone, the layer's step 581 and 613 us).
+//
+// The constants are fits to about 22000 times: 64 to 16384 tiles of every shape, K 3
+// to 2048, three layouts, whole and ragged, and 667 random and transformer products
+// with every shape and split; root mean square error 7 % (bf16 11 %).  Over the
+// products that do not run as small ones the pick is within 0.9 % (fp32), 1.9 %
+// (bf16) and 0.6 % (split bf16) of the best on average.  One time per k and round
+// with a fixed part, which stood here before, was within 2.6 %, 5.7 % and 2.3 %, and
+// far off at K below 256: [1184, 448] K 32 fp32 8.4 us (now 5.2), [1344, 3712] K 64
+// 19.6 (10.8), [7680, 1344] K 96 35 (22); bf16 [4096, 1376] A^T.B K 512 37 (30).
 // 96-column tiles take no split but in fp32.
 struct SplitShape {
     TileKind kind;
     int bm, bn;
     double one, one_k, base, round, per_k, edge, ta;
 };
-constexpr SplitShape kShapesF32[] = {{kTile128, 128, 128, 6.7, 0.0280, 4.8, 4.1, 0.0391, 2.9, 1.04},
-                                     {kTile256, 256, 256, 10.6, 0.1023, 2.3, 12.0, 0.1370, 7.2, 1.00},
-                                     {kTile256x96, 256, 96, 6.3, 0.0477, 6.1, 4.5, 0.0586, 4.1, 1.07},
-                                     {kTile128x64, 128, 64, 4.9, 0.0220, 5.3, 1.2, 0.0229, 1.6, 1.06},
-                                     {kTile64, 64, 64, 6.1, 0.0106, 3.4, 3.3, 0.0126, 2.7, 1.08},
-                                     {kTile64x2, 64, 64, 4.5, 0.0154, 5.4, 0.31, 0.0137, 1.4, 1.05},
-                                     {kTile64x1, 64, 64, 4.0, 0.0262, 4.9, 0.12, 0.0150, 0.8, 1.02}};
-constexpr SplitShape kShapesBf16[] = {{kTile128, 128, 128, 5.5, 0.0161, 5.7, 1.8, 0.0133, 1.0, 1.18},
-                                      {kTile256, 256, 256, 9.5, 0.0299, 1.3, 13.3, 0.0332, 4.2, 1.14},
-                                      {kTile256x96, 256, 96, 7.2, 0.0205, 5.8, 3.3, 0.0159, 0.0, 1.42},
-                                      {kTile96, 128, 96, 4.9, 0.0146, 5.1, 1.5, 0.0096, 0.0, 1.46},
-                                      {kTile64, 64, 64, 3.8, 0.0101, 4.4, 0.20, 0.0061, 1.0, 1.25}};
-constexpr SplitShape kShapesBf16x3[] = {{kTile128, 128, 128, 6.3, 0.0275, 6.0, 2.0, 0.0238, 0.7, 1.13},
-                                        {kTile256, 256, 256, 12.4, 0.0621, 3.3, 13.6, 0.0737, 3.4, 1.06},
-                                        {kTile256x96, 256, 96, 7.2, 0.0322, 4.9, 4.6, 0.0357, 0.0, 1.32},
-                                        {kTile96, 128, 96, 5.2, 0.0239, 5.1, 1.6, 0.0192, 0.0, 1.17},
-                                        {kTile64, 64, 64, 4.1, 0.0167, 4.6, 0.25, 0.0090, 0.9, 1.19}};
+constexpr SplitShape kShapesF32[] = {{kTile256, 256, 256, 8.4, 0.1008, 2.0, 13.0, 0.1342, 5.6, 1.03},
+                                     {kTile256x96, 256, 96, 7.5, 0.0454, 4.8, 5.4, 0.0596, 3.7, 1.09},
+                                     {kTile128, 128, 128, 5.6, 0.0282, 4.2, 4.7, 0.0393, 2.4, 1.07},
+                                     {kTile128x64, 128, 64, 4.5, 0.0224, 5.2, 1.4, 0.0224, 1.3, 1.09},
+                                     {kTile64, 64, 64, 6.0, 0.0109, 3.7, 3.4, 0.0135, 2.5, 1.06},
+                                     {kTile64x2, 64, 64, 5.0, 0.0150, 5.2, 0.64, 0.0135, 1.2, 1.06},
+                                     {kTile64x1, 64, 64, 3.9, 0.0264, 5.0, 0.27, 0.0147, 0.6, 1.02}};
+constexpr SplitShape kShapesBf16[] = {{kTile256, 256, 256, 7.4, 0.0254, 1.9, 13.7, 0.0302, 2.2, 1.31},
+                                      {kTile256x96, 256, 96, 7.5, 0.0195, 5.3, 3.6, 0.0160, 0.0, 1.42},
+                                      {kTile128, 128, 128, 4.7, 0.0145, 5.0, 2.3, 0.0139, 0.7, 1.24},
+                                      {kTile96, 128, 96, 5.2, 0.0140, 5.0, 1.5, 0.0098, 0.0, 1.43},
+                                      {kTile64, 64, 64, 3.7, 0.0108, 4.5, 0.32, 0.0055, 0.9, 1.26}};
+constexpr SplitShape kShapesBf16x3[] = {{kTile256, 256, 256, 10.3, 0.0601, 4.2, 14.8, 0.0738, 0.6, 1.11},
+                                        {kTile256x96, 256, 96, 7.5, 0.0312, 4.4, 4.9, 0.0359, 0.0, 1.31},
+                                        {kTile128, 128, 128, 5.1, 0.0266, 5.7, 2.5, 0.0243, 0.2, 1.12},
+                                        {kTile96, 128, 96, 5.3, 0.0233, 5.0, 1.6, 0.0197, 0.0, 1.16},
+                                        {kTile64, 64, 64, 4.1, 0.0170, 4.7, 0.39, 0.0089, 0.8, 1.13}};
 
 // Whether a whole-tile bf16 or split-bf16 product runs on the four-wave kernel
 // of this file rather than gemm_narrow.hip's: the 96-column tiles (64x96 per
@@ -1113,8 +1118,8 @@ struct SplitPlan {
 // keeps fitting
 constexpr size_t kNoAllocScratchBytes = (size_t)128 << 20;
 
-SplitPlan plan_split(int prec, int64_t M, int64_t N, int64_t K, int64_t batch, bool allow_all,
-                     bool ta, bool allow_split, bool allow_96 = true) {
+SplitPlan find_plan(int prec, int64_t M, int64_t N, int64_t K, int64_t batch, bool allow_all,
+                    bool ta, bool allow_split, bool allow_96) {
     const bool fp32 = prec == kFp32;
     SplitPlan best = {{kTile128, 128, 128}, 1, K};
     double c = -1.0;
@@ -1145,6 +1150,8 @@ SplitPlan plan_split(int prec, int64_t M, int64_t N, int64_t K, int64_t batch, b
         const uint32_t step = fp32 ? 32 * split_groups(t.kind) : 32;
         const bool whole = M % t.bm == 0 && N % t.bn == 0 && K % step == 0;
         const double edge = whole ? 0.0 : t.edge, ta_k = ta ? t.ta : 1.0;
+        SplitPlan own = best;
+        double c_own = -1.0;
         for(const int s : kCounts) {
             if(s > (n96 && !fp32 ? 1 : s_max)) break;
             const uint32_t chunk = s == 1 ? k32 : ((k32 + s - 1) / s + step - 1) / step * step;
@@ -1155,14 +1162,38 @@ SplitPlan plan_split(int prec, int64_t M, int64_t N, int64_t K, int64_t batch, b
                          rounds = 0.5 * ((double)((n + kCUs - 1) / kCUs) + (double)n / kCUs);
             const double ck = std::max(t.one + edge + t.one_k * k,
                                        t.base + rounds * (t.round + edge + t.per_k * k)) +
-                              (splits > 1 ? 0.5 + link * splits + (splits + 1) * plane : 0.0);
-            if(c < 0.0 || ck < c) {
-                c = ck;
-                best = {{t.kind, t.bm, t.bn}, (int)splits, splits == 1 ? K : (int64_t)chunk};
+                              (splits > 1 ? 1.4 + link * splits + (splits + 1) * plane : 0.0);
+            if(c_own < 0.0 || ck < c_own) {
+                c_own = ck;
+                own = {{t.kind, t.bm, t.bn}, (int)splits, splits == 1 ? K : (int64_t)chunk};
             }
+        }
+        if(c < 0.0 || c_own < 0.97 * c) {
+            c = c_own;
+            best = own;
         }
     }
     return best;
+}
+
+// A program's products repeat: each thread keeps the plans of 256 shapes (a
+// split's takes 0.5 to 1 us to find, six of them to size a workspace)
+SplitPlan plan_split(int prec, int64_t M, int64_t N, int64_t K, int64_t batch, bool allow_all,
+                     bool ta, bool allow_split, bool allow_96 = true) {
+    struct Kept {
+        int64_t M, N, K, batch;
+        int how;
+        SplitPlan plan;
+    };
+    static thread_local Kept kept[256] = {};  // (how 0: empty)
+    const int how = 16 * (prec + 1) + 8 * allow_all + 4 * ta + 2 * allow_split + allow_96;
+    const uint64_t h = ((((uint64_t)M * 0x9e3779b97f4a7c15u + (uint64_t)N) * 0x9e3779b97f4a7c15u +
+                         (uint64_t)K) * 0x9e3779b97f4a7c15u + (uint64_t)batch * 128 + (uint64_t)how) *
+                       0x9e3779b97f4a7c15u;
+    Kept& e = kept[h >> 56];
+    if(e.how != how || e.M != M || e.N != N || e.K != K || e.batch != batch)
+        e = {M, N, K, batch, how, find_plan(prec, M, N, K, batch, allow_all, ta, allow_split, allow_96)};
+    return e.plan;
 }
 
 template <bool TA, bool TB, class T, int EDGE, int EPI>
@@ -1504,7 +1535,8 @@ extern "C" size_t pk_gemm_workspace_f32(int64_t M, int64_t N, int64_t K) {
     if(M <= 0 || N <= 0 || K <= 0) return 0;
     int64_t kchunk;
     const int S = choose_splits(M, N, K, true, true, &kchunk);
-    size_t most = S > 1 ? (size_t)S * (size_t)M * (size_t)N * sizeof(float) : 0;
+    if(S == 1) return 0;
+    size_t most = (size_t)S * (size_t)M * (size_t)N * sizeof(float);
     for(const int prec : {kFp32, kBf16, kBf16x3})
         for(const bool ta : {false, true}) most = std::max(most, gemm_workspace(prec, M, N, K, ta));
     return most;

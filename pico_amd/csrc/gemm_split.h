@@ -114,14 +114,19 @@ __device__ __forceinline__ void split_load(const SplitSource& src, int64_t ld, i
                                                      [SplitOperand<KFAST, R, THREADS, W>::KPI]) {
     using O = SplitOperand<KFAST, R, THREADS, W>;
     const int64_t off = k0 * src.kstep;
-    // (2^31 - 1 at most, which no offset of a slice reaches, so that taking k rows
-    // off it stays a 32-bit subtraction)
-    const int num = EDGE ? (int)min(max(src.left - off, (int64_t)0), (int64_t)INT32_MAX) : -16;
-    // the operand from k row t of the slice on
+    const int64_t left = src.left - off;
+    // the operand from the slice's k row t on.  Only slices of 32 k ask for more than
+    // the first: their size stops at 2^31 - 1, which no offset of theirs reaches,
+    // so that taking k rows off it stays a 32-bit subtraction
     auto rest = [&](int t) {
-        const int skip = t * (int)src.kstep;
+        const int skip = W == SK ? 0 : t * (int)src.kstep;
+        int num = (int)0xfffffff0u;
+        if(EDGE && W == SK)
+            num = (int)(left <= 0 ? 0u : left > 0xfffffff0ll ? 0xfffffff0u : (unsigned)left);
+        else if(EDGE)
+            num = max((int)min(max(left, (int64_t)0), (int64_t)INT32_MAX) - skip, 0);
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(src.base + off + skip), (short)0,
-                                                 EDGE ? max(num - skip, 0) : num, 0x00020000);
+                                                 num, 0x00020000);
     };
     const __amdgpu_buffer_rsrc_t rs = rest(0);
 #pragma unroll
@@ -576,26 +581,36 @@ __global__ __launch_bounds__(T::THREADS, T::WPS) void gemm_split_kernel(GemmPara
             }
         }
     }
-    // the wave's blocks with a sum that is not finite among those it stores (a
-    // tile's rows and columns past M and N may hold anything)
+    // the wave's blocks with a sum that is not finite
     unsigned again = 0;
 #pragma unroll
-    for(int i = 0; i < TM; ++i) {
-        const int left = (int)min(p.M - job.row0 - ar0 - i * 32 - lh * 4, (int64_t)32);
+    for(int b = 0; b < TM * TN; ++b) {
+        if(G > 1 && g != b % G) continue;
+        float sum = 0.0f;
 #pragma unroll
-        for(int j = 0; j < TN; ++j) {
-            if(G > 1 && g != (i * TN + j) % G) continue;
+        for(int r = 0; r < 16; ++r) {
+            if(G == 1 && SETS == 1) acc[b / TN][b % TN][r] *= unscale;
+            sum = fmaf(acc[b / TN][b % TN][r], 0.0f, sum);
+        }
+        if(cores || __any(sum != 0.0f)) again |= 1u << b;
+    }
+    // ... among those it stores: a tile's rows and columns past M and N hold anything
+    // (looked at only now: 300 instructions that finite tiles need not run)
+    if(EDGE != kWhole && again && !cores) {
+        unsigned stored = 0;
+#pragma unroll
+        for(int b = 0; b < TM * TN; ++b) {
+            if(G > 1 && g != b % G) continue;
+            const int left = (int)min(p.M - job.row0 - ar0 - b / TN * 32 - lh * 4, (int64_t)32);
+            const int c = br0 + b % TN * 32 + lr;
             float sum = 0.0f;
 #pragma unroll
-            for(int r = 0; r < 16; ++r) {
-                if(G == 1 && SETS == 1) acc[i][j][r] *= unscale;
-                const bool in = EDGE == kWhole || (r >> 2) * 8 + (r & 3) < left;
-                sum = fmaf(in ? acc[i][j][r] : 0.0f, 0.0f, sum);
-            }
-            const int c = br0 + j * 32 + lr;
-            const bool in = EDGE == kWhole || (PAIR ? job.col0 + c % (BN / 2) < p.pair_F : job.col0 + c < p.N);
-            if(cores || __any(in && sum != 0.0f)) again |= 1u << (i * TN + j);
+            for(int r = 0; r < 16; ++r)
+                sum = fmaf((r >> 2) * 8 + (r & 3) < left ? acc[b / TN][b % TN][r] : 0.0f, 0.0f, sum);
+            const bool in = PAIR ? job.col0 + c % (BN / 2) < p.pair_F : job.col0 + c < p.N;
+            if(__any(in && sum != 0.0f)) stored |= 1u << b;
         }
+        again = stored;
     }
     again = __builtin_amdgcn_readfirstlane(again);
     auto exact = [&](int b) {
