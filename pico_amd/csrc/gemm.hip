@@ -9,19 +9,21 @@
 // parts (gemm_split.h); this file holds the choice of tile and K split, the
 // small-product kernels, and the opt-in bf16, split-bf16 and fp8 kernels.
 //
-// Design of those (one 256-thread workgroup = 4 waves per C tile):
+// Design of the kernels of this file (one 256-thread workgroup = 4 waves per C
+// tile); the others' tiles are in gemm_split.hip and gemm_narrow.hip:
 //  * Five tile shapes of 32x32 matrix blocks (16 fp32 accumulators per lane per
-//    block), chosen per call by how evenly they spread over the 256 CUs:
+//    block):
 //      256x256  2x2 waves of 128x128 (4x4 blocks, 256 accumulators held in
-//               AGPRs), one workgroup per CU -- large products;
+//               AGPRs), one workgroup per CU;
 //      256x96   4x1 waves of 64x96, one per CU -- N a multiple of 96 (an
 //               [8192, 768] output, d_model 768, is 256 of them);
 //      128x128  2x2 waves of 64x64, two workgroups per CU;
 //      128x96   4x1 waves of 32x96, two per CU -- N a multiple of 96;
-//      64x64    2x2 waves of 32x32, four per CU -- small products.
-//  * Tiles on the edge of C are handled in the same kernel: with M, N, K and
-//    the strides multiples of 4 each 128-bit load is predicated as a whole;
-//    otherwise loads fall back to 32-bit elements.
+//      64x64    2x2 waves of 32x32, four per CU.
+//  * The bf16 and split-bf16 kernel takes whole tiles only.  The fp8 kernel also
+//    takes tiles on the edge of C: with M, N, K and the strides multiples of 4
+//    each 128-bit load is predicated as a whole; otherwise loads fall back to
+//    32-bit elements.
 //  * K advances 32 at a time through a double-buffered LDS ring, the next slice
 //    staged into the other buffer and the slice after it fetched into registers
 //    under the current slice's matrix instructions, interleaved with them
@@ -976,7 +978,15 @@ bool small_product(int64_t M, int64_t N, int64_t K, bool TA, bool TB, int64_t ld
            extent(TB, N, ldb) < INT32_MAX;
 }
 
-// K split for a product whose output has too few tiles to fill the chip: 2
+// The fp8 product's K split; for the other precisions, whether a shape may split
+// at all, and whether its partials have to fit pk_gemm_noalloc_f32's array
+// (plan_split picks their count).  The units and times below are those of the fp32
+// kernel on the fp32 cores that this rule was measured with, and the fp8 kernel's
+// 128x128 tiles still stand as it does; for the split products it has been kept as
+// a rule, not measured anew: K splits of products that it forbids ([4096, 512] K 8192
+// A.B^T) are not tried.
+//
+// For a product whose output has too few tiles to fill the chip: 2
 // resident workgroups per CU x 256 CUs want >= 512 workgroups.
 //  * K >= 1024 (weight gradients: M, N ~ d_model, K = tokens): slices of at
 //    least 256 (8 LDS stages).  The split count minimises the estimated time
@@ -1460,11 +1470,13 @@ int gemm_impl(char ta, char tb, int64_t M, int64_t N, int64_t K, float alpha, co
     // diagonal logic is exercised at that size)
     TileChoice tc = gp.splits > 1 ? TileChoice{kTile128, 128, 128}
                                   : pick_tile(M, N, batch, causal == 0, gp.pair_F);
+    // (fp8's need; the other precisions' tiles may hold partial columns but keep
+    // to the same contract)
     if(tc.bm == 0)
         return pk::fail("pk_gemm_swiglu_fwd_f32: F=%lld is not a multiple of 32 (no tile holds "
                         "whole gate/up column pairs)", (long long)gp.pair_F);
-    // the others: a shape for M, N and K alone (the SwiGLU-forward product's tiles
-    // may hold partial columns), so every epilogue adds K in the same order
+    // the others: a shape for M, N and K alone, so every epilogue adds K in the
+    // same order
     if(prec != kFp8) tc = plan.tile;
     const int64_t tiles_m = (M + tc.bm - 1) / tc.bm,
                   tiles_n = gp.pair_F ? (gp.pair_F + tc.bn / 2 - 1) / (tc.bn / 2)

@@ -157,7 +157,7 @@ __device__ __forceinline__ void store_tile(const GemmParams& p, const TileJob& j
 }
 
 // Epilogues that read other matrices: the tile goes through LDS (free once
-// the main loop is done) in passes of RP rows, and all 256 threads then walk
+// the main loop is done) in passes of RP rows, and all its threads then walk
 // the staged rows in float4 runs, so every global access is a coalesced
 // 128-bit one and no per-element loads wait inside the accumulator loops
 // (which, in the 256x256 tile, also pushed the accumulators out of

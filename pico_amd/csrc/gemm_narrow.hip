@@ -22,8 +22,8 @@
 //
 // Bf16 against the four-wave kernel it replaces, us: 4096^3 A.B / A.B^T / A^T.B
 // 173 / 145 / 190 -> 166 / 136 / 175, [8192, 4096] K 768 87 -> 79.  Ragged:
-// [2000, 1503] K 1001 54 -> 26 (split bf16 64 -> 35), its A.B^T 73 -> 34 (77 ->
-// 38), [333, 517] K 1201 32 -> 16 (35 -> 18).  gemm.hip keeps that kernel for
+// [2000, 1503] K 1001 54 -> 26 (split bf16 64 -> 37), its A.B^T 73 -> 27 (77 ->
+// 36), [333, 517] K 1201 32 -> 15 (35 -> 18).  gemm.hip keeps that kernel for
 // the whole tiles where it is the faster one (narrow_here).
 #include <type_traits>
 

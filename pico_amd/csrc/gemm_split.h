@@ -13,7 +13,7 @@
 // |a||b|, are left out (below 0.87 2^-24 of one product at the worst).  Nothing is
 // held in less than fp32's 24 bits, and the sums are fp32.  Against float64,
 // relative 2-norm on random operands, the error is below that of the fp32 matrix
-// instructions (which round after every k) from K 3 on: normal operands, K 4 / 32 /
+// instructions (which round after every k) from K 4 on: normal operands, K 4 / 32 /
 // 768 / 2048 / 4096 3.2e-8 / 4.2e-8 / 2.9e-7 / 6.9e-7 / 9.7e-7 against 4.0e-8 /
 // 1.03e-7 / 5.0e-7 / 8.1e-7 / 1.15e-6.  Products of one and two k, whose few
 // roundings they do better (2.5e-8 against 3.5e-8, 3.1e-8 against 3.4e-8), run
@@ -32,8 +32,12 @@
 //    add up in a sum over outputs (a bias gradient, an attention average:
 //    the mean error of [8192, 2304] outputs with K 768 was 2e-6 of the value
 //    in such a sum).  So the parts of op(A) change sign with the sums every
-//    128 k (K group by K group where a workgroup splits K), and the loss
-//    cancels: mean error below 2e-9 of the root mean square.
+//    128 k (K group by K group, or set by set, where a workgroup splits K), and
+//    the loss cancels: mean error below 3e-9 of the root mean square from K 128 on.
+//    Before the first turn (one slice of 16, 64 k in 256x256 tiles) nothing
+//    cancels, up to 1.2e-8, and outputs of one sign keep some of it: probabilities
+//    times values around 1 2e-8 to 4e-8 of the value (the fp32 instructions 2e-9
+//    at K 128, 2e-8 at K 512).
 //  * Bound: 6 instructions of 32 cycles per 32x32 block and 16 k, 2.5 PFLOP/s /
 //    6 = 417 TFLOP/s at the nominal clock; the card settles near 2.06 GHz under
 //    bf16 matrix load (358).  The split costs 6.5 vector instructions per staged
@@ -45,6 +49,10 @@
 //    waves, G groups of them take every G-th slice of K into LDS buffers of
 //    their own and add their sums at the end (256x96: 166 -> 197 TFLOP/s at
 //    [8192, 768] K 2304; 64x64 with G 4: 84 -> 114 at 1024^3).
+//    64x64 tiles of short K have two groups or one, each with several sets of
+//    sums: the same four sums, bit for bit, without a thousand threads' start and
+//    the groups' meeting (256 tiles, us, G 4 / 2 / 1: K 32 9.6 / 7.2 / 5.3, K 256 9.4 /
+//    9.0 / 10.3, K 512 12.8 / 13.1 / 16.1).
 //  * A slice is 16 k.  Its first half multiplies m.m, m.h, h.m while l is read,
 //    the next slice is split and stored and the slice after it fetched; one
 //    barrier; then h.l, l.h, h.h while the next slice's m and h are read into
@@ -53,10 +61,10 @@
 //    at any 4-byte alignment, so ragged sizes take the same path: what lies
 //    behind the end reads as zero, and only a partial last slice is masked.
 //    (The per-element edge path this replaces ran 2000x1503x1001, forward and
-//    backward, at 59 TFLOP/s; now 130.)
+//    backward, at 59 TFLOP/s; now 118-127.)
 //
-// 4096^3 A.B / A.B^T / A^T.B 244-246 TFLOP/s (149 on the fp32 cores), 8192^3
-// 237-243 (151), 2048^3 188-193 (142), 1024^3 114-117 (105-115).
+// TFLOP/s of A.B, A.B^T and A^T.B by card and box: 4096^3 223-250 (149 on the fp32
+// cores), 8192^3 222-243 (151), 2048^3 174-197 (142), 1024^3 100-118 (98-115).
 
 // A tile shape: WM x WN waves, each TM x TN blocks of 32 x 32; WPS waves per SIMD;
 // G groups of them, each with A sets of sums (slice s of K goes to group s % G and
@@ -225,8 +233,11 @@ __device__ __forceinline__ void split3(float x0, float x1, float scale, int& h, 
 }
 
 // LDS: [part][row][16 k], rows of 32 bytes whose two 16-byte halves swap places
-// every 4 rows, so the 8 lanes of a 128-bit access phase (8 rows 32 bytes
-// apart) fall in distinct banks.  Offset in 16-bit elements of (row, k):
+// every 4 rows.  8 rows 32 bytes apart then fall in distinct banks, but rows r and
+// r + 8 share theirs: 3.8e7 conflict cycles over 1.3e7 LDS instructions at 4096^3, 72 a
+// wave and slice or 4 to a fragment read, in every layout.  Under 256x256 tiles'
+// matrix instructions that is hidden; in the small tiles the reads take as long
+// as those.  Offset in 16-bit elements of (row, k):
 __device__ __forceinline__ int split_off(int row, int k) {
     return row * SK + ((((k >> 3) ^ (row >> 2)) & 1) << 3) + (k & 7);
 }
