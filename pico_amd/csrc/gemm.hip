@@ -1534,10 +1534,12 @@ extern "C" int pk_gemm_f32(char ta, char tb, int64_t M, int64_t N, int64_t K, fl
                      0, nullptr, 0, kFp32, stream);
 }
 
-// the split-K partials of op(A) . op(B) for one layout of A
+// the split-K partials of op(A) . op(B) for one layout of A, aligned or not (which
+// decides on 96-column tiles, and those against a split)
 static size_t gemm_workspace(int prec, int64_t M, int64_t N, int64_t K, bool ta) {
     if(M <= 0 || N <= 0 || K <= 0) return 0;
-    const int S = plan_split(prec, M, N, K, 1, true, ta, true).splits;
+    const int S = std::max(plan_split(prec, M, N, K, 1, true, ta, true, true).splits,
+                           plan_split(prec, M, N, K, 1, true, ta, true, false).splits);
     return S > 1 ? (size_t)S * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
